@@ -1,6 +1,7 @@
 // mp_kernels.hip -- gfx950 kernels of the batch-1 MoE decode step.
 //
-//   route_logits    router GEMV (W_r f32 [E][H]), one wavefront per expert row
+//   route_logits    router GEMV (W_r f32 [E][H]), one workgroup per expert row
+//   route_gemm      the same sums for a batch, as tiles on fp32 MFMA
 //   route_select    softmax -> + cache prior -> top-k -> renormalised gate
 //                   weights -> slot lookup, and the Q8_K quantization of x the
 //                   expert kernels consume (one workgroup per token)
@@ -189,6 +190,107 @@ __global__ __launch_bounds__(64 * RL_WAVES) void route_logits_kernel(RouteArgs a
         q8k_store(q, d, a.q8x + ((size_t)tok * (a.H / QK) + blockIdx.x) * Q8K_BYTES, lane);
         if (a.post && tok == 0) q8k_store_sys(q, d, (uint32_t *)(a.post->q8x + (size_t)blockIdx.x * Q8K_BYTES), lane);
     }
+}
+
+// The router of a batch as a matrix product, in the same order to the last
+// bit: RT x RT tiles of 16 tokens by 16 experts per workgroup on fp32 MFMA
+// with K = 1 (v_mfma_f32_16x16x1_4b_f32: one fmaf per element, equal to fmaf
+// for subnormals, infinities and NaN too, and four independent 16x16 blocks).
+// The canonical sum of a logit is a tree over 4 quarters x 64 lanes of chains
+// of H / 1024 * 4 fmaf: wave (q, r) takes lanes 16r .. 16r + 15 of quarter q,
+// block b of an MFMA lane 16r + 4J + b, and the chain's steps (i, c) are
+// successive MFMAs on one accumulator, so no order is left to the hardware.
+// The butterfly's steps o = 1, 2 add the MFMA's blocks, o = 4, 8 the four J
+// (two J at a time: both halves of a 128-byte line requested together),
+// o = 16, 32 and the quarters the waves' sums, in LDS.
+// What bounds it: the operand reads, 16 rows of 64 bytes an instruction
+// (4,096 tokens x 128 experts: ~45 us, the products alone ~17 at the 130
+// TFLOP/s this instruction reaches).  The row-per-workgroup kernel above, which
+// re-reads each row from L2 for every token, took 457 us there, 214 at 1,000 x
+// 256 (here ~20) and 21 at 197 x 128 (~10).
+constexpr int RG_I = 2048 / (RL_WAVES * QK);         // chain steps of four: H = 2048
+constexpr int RG_WAVES = 4 * RL_WAVES;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+template <int RT>
+__global__ __launch_bounds__(64 * RG_WAVES) void route_gemm_kernel(RouteArgs a, int n_tok, int n_tiles) {
+    constexpr int TW = 16 * RT, LD = TW + 4;          // + 4: the four row groups of a tile in distinct banks
+    __shared__ float s_part[RG_WAVES][TW][LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if ((int)blockIdx.x >= n_tiles) {                 // the Q8_K blocks of x, one per wave
+        const int blk = ((int)blockIdx.x - n_tiles) * RG_WAVES + wave;
+        if (blk < n_tok * (a.H / QK)) q8k_wave(a.x + (size_t)QK * blk, a.q8x + (size_t)blk * Q8K_BYTES, lane);
+        return;
+    }
+    // the expert tiles of one token tile on one XCD (workgroups go to the 8
+    // XCDs round-robin), so its L2 reads those tokens once
+    const int ne = a.E / TW, g = (int)blockIdx.x >> 3;
+    const int tt = (g / ne) * 8 + ((int)blockIdx.x & 7), te = g % ne;
+    if (tt * TW >= n_tok) return;
+    const int n = lane & 15, b = lane >> 4;
+    const int q = wave >> 2, r = wave & 3;
+    const float *xp[RT], *wp[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int o = (a.H / RL_WAVES) * q + 4 * (16 * r + b);
+        xp[t] = a.x + (size_t)min(tt * TW + 16 * t + n, n_tok - 1) * a.H + o;
+        wp[t] = a.W + (size_t)(te * TW + 16 * t + n) * a.H + o;
+    }
+    f32x4_t sum[RT][RT];
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {                  // J = 2 jj and the next
+        float4 xv[RT][RG_I][2], wv[RT][RG_I][2];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int i = 0; i < RG_I; ++i)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    xv[t][i][k] = *(const float4 *)(xp[t] + QK * i + 32 * jj + 16 * k);
+                    wv[t][i][k] = *(const float4 *)(wp[t] + QK * i + 32 * jj + 16 * k);
+                }
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int u = 0; u < RT; ++u) {
+                f32x4_t v[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    f32x16_t d = {};
+#pragma unroll
+                    for (int i = 0; i < RG_I; ++i) {
+                        d = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[t][i][k].x, wv[u][i][k].x, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[t][i][k].y, wv[u][i][k].y, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[t][i][k].z, wv[u][i][k].z, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[t][i][k].w, wv[u][i][k].w, d, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[k][c] = (d[c] + d[4 + c]) + (d[8 + c] + d[12 + c]);     // o = 1, 2
+                }
+                const f32x4_t p = v[0] + v[1];        // o = 4, then o = 8
+                sum[t][u] = jj ? sum[t][u] + p : p;
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int u = 0; u < RT; ++u)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s_part[wave][16 * t + 4 * b + c][16 * u + n] = sum[t][u][c];
+    __syncthreads();
+    if (threadIdx.x >= TW * TW) return;
+    const int row = threadIdx.x / TW, col = threadIdx.x % TW;
+    const int tok = tt * TW + row, e = te * TW + col;
+    if (tok >= n_tok) return;
+    float acc = 0.0f;
+#pragma unroll
+    for (int j = 0; j < RL_WAVES; ++j) {              // o = 16, 32; then the quarters in order
+        const float s = (s_part[4 * j][row][col] + s_part[4 * j + 1][row][col]) +
+                        (s_part[4 * j + 2][row][col] + s_part[4 * j + 3][row][col]);
+        acc = j == 0 ? s : acc + s;
+    }
+    if (a.bias) acc = acc + a.bias[(size_t)tok * a.E + e];
+    a.logits[(size_t)tok * a.E + e] = acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -1440,6 +1542,21 @@ static hipError_t launch(F k, dim3 grid, dim3 block, hipStream_t st, hipEvent_t 
     return hipGetLastError();
 }
 
+// When a batch's router runs as a matrix product, and with which tile.  Below
+// ~9,600 logits a workgroup per row and token is faster (us with the selection,
+// rows / product: 64 tokens x 128 experts 12.2 / 13.1, 100 x 128 15.2 / 13.1, 32 x
+// 256 13.6 / 14.9, 64 x 256 18.6 / 15.0).  From 96 tiles of 32 x 32 on, these beat
+// tiles of 16 x 16 (us: 700 x 128, 88 tiles, 22.7 / 22.4; 400 x 256, 104 tiles,
+// 24.4 / 25.3; 4,096 x 128 59 / 87).
+constexpr int ROUTE_GEMM_MIN_LOGITS = 9600, ROUTE_GEMM_MIN_TILES = 96;
+template <int RT>
+static hipError_t launch_route_gemm(const RouteArgs &a, int n_tok, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const int tw = 16 * RT, tt = ((n_tok + tw - 1) / tw + 7) / 8 * 8;      // token tiles, in eights (one per XCD)
+    const int tiles = tt * (a.E / tw);
+    const int q8 = a.q8x ? (n_tok * (a.H / QK) + RG_WAVES - 1) / RG_WAVES : 0;
+    return launch(route_gemm_kernel<RT>, dim3((unsigned)(tiles + q8)), dim3(64 * RG_WAVES), st, e0, e1, a, n_tok, tiles);
+}
+
 hipError_t launch_route(const RouteLaunch &l, hipStream_t st, hipEvent_t *ev) {
     RouteArgs a;
     a.W = l.W; a.x = l.x; a.bias = l.bias; a.prior = l.prior; a.table = l.table; a.dummy = l.dummy;
@@ -1457,9 +1574,15 @@ hipError_t launch_route(const RouteLaunch &l, hipStream_t st, hipEvent_t *ev) {
     if (l.logits_in)
         return launch(route_select_kernel, dim3((unsigned)l.n_tok), dim3(256), st, ev ? ev[2] : nullptr,
                       ev ? ev[3] : nullptr, a);
-    const hipError_t e = launch(route_logits_kernel, dim3((unsigned)l.E * (unsigned)(1 + (l.apost ? l.an : 0)),
-                                                         (unsigned)l.n_tok),
-                                dim3(64 * RL_WAVES), st, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr, a);
+    const hipEvent_t e0 = ev ? ev[0] : nullptr, e1 = ev ? ev[1] : nullptr;
+    hipError_t e;
+    if (l.n_tok > 1 && l.n_tok * l.E >= ROUTE_GEMM_MIN_LOGITS) {       // (post and lookahead are batch-1)
+        const bool big = (l.n_tok + 31) / 32 * (l.E / 32) >= ROUTE_GEMM_MIN_TILES;
+        e = big ? launch_route_gemm<2>(a, l.n_tok, st, e0, e1) : launch_route_gemm<1>(a, l.n_tok, st, e0, e1);
+    } else {
+        e = launch(route_logits_kernel, dim3((unsigned)l.E * (unsigned)(1 + (l.apost ? l.an : 0)), (unsigned)l.n_tok),
+                   dim3(64 * RL_WAVES), st, e0, e1, a);
+    }
     if (e != hipSuccess) return e;
     return launch(route_select_kernel, dim3((unsigned)l.n_tok), dim3(256), st, ev ? ev[2] : nullptr,
                   ev ? ev[3] : nullptr, a);

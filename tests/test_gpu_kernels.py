@@ -98,6 +98,26 @@ def test_route_bit_exact(E, K, n_tok):
             assert np.array_equal(q8[t], O.quant_q8k(x[t]))
 
 
+# both sides of the rule that picks the router kernel of a batch (logits per call), and of the one
+# that picks its tile (32 x 32 tiles per call); ragged last tiles of 1, 6, 11, 15 and 16 tokens
+@pytest.mark.parametrize("E,K,n_tok", [(64, 6, 149), (64, 6, 150), (128, 8, 75), (128, 8, 91), (128, 8, 112), (256, 10, 37),
+                                       (256, 10, 38), (256, 8, 353), (128, 8, 737), (64, 6, 1537)])
+def test_route_batch_bit_exact(E, K, n_tok):
+    rng = np.random.default_rng(E * 10007 + n_tok)
+    W = (rng.standard_normal((E, H)) * 0.02).astype(np.float32)
+    W[E // 2] = W[3]                                # ties: the lower id first
+    x = (rng.standard_normal((n_tok, H)) * rng.uniform(0.01, 8.0, size=(n_tok, 1))).astype(np.float32)
+    x[n_tok // 2] = 0.0                             # every logit equal
+    bias = rng.standard_normal((n_tok, E)).astype(np.float32) if n_tok % 2 else None
+    ids, w, _, probs, q8 = run_route(W, x, K, bias)
+    for t in range(n_tok):
+        rids, rw, _, rprobs = O.route(W, x[t], K, bias=None if bias is None else bias[t])
+        assert np.array_equal(ids[t], rids), t
+        assert np.array_equal(w[t].view(np.uint32), rw.view(np.uint32)), t
+        assert np.array_equal(probs[t].view(np.uint32), rprobs.view(np.uint32)), t
+        assert np.array_equal(q8[t], O.quant_q8k(x[t])), t
+
+
 def test_route_prior_on_logits_bit_exact():
     rng = np.random.default_rng(8)
     E, K = 128, 8
