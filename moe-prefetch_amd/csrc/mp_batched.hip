@@ -7,12 +7,14 @@
 //                        cores consume: the int8 values as fp16 codes, the
 //                        block scale, and the 16-value group sums as fp16 --
 //                        all exact
-//   grouped_q4_kernel    per (64-row tile, expert): the expert's Q4_K rows
-//                        against the activations of every pair dispatched to
-//                        it, on MFMA 16x16x32 f16; up and gate as one 2I-row
-//                        matrix (the expert's [up | gate] layout), and Q4_K
-//                        down with the pair's gate weight, scattered to the
-//                        pair's row
+//   grouped_q4_tile_kernel  per (expert's pairs in chunks, 128-row tiles): the
+//                        expert's Q4_K rows against the activations of the
+//                        chunk's pairs, on MFMA 32x32x16 f16; up and gate as
+//                        one 2I-row matrix (the expert's [up | gate] layout),
+//                        and Q4_K down with the pair's gate weight, scattered
+//                        to the pair's row
+//   grouped_q4_kernel    the same per (64-row tile, expert) on MFMA 16x16x32,
+//                        for shapes of few workgroups
 //   grouped_q6_kernel    the same for a Q6_K down matrix
 //   swiglu_quant_kernel  h = silu(gate) * up, and its Q8_K
 //   combine_kernel       out[t] = sum over k of the weighted rows, k in order
@@ -39,6 +41,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "mp_device.h"
 #include "mp_format.h"
@@ -157,7 +160,10 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *ids, int 
 // Q8_K rows for the matrix cores: one wavefront per (row, 256-value block)
 __device__ inline uint32_t h16(int v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)v); }
 
-// the wave's 4 values per lane -> fp16 codes, block scale and group sums
+// the wave's 4 values per lane -> fp16 codes, block scale and group sums.
+// MFMA: the lane's codes in the order 0, 2, 1, 3 the grouped products read
+// them in (see pack_1024), else 0, 1, 2, 3.
+template <bool MFMA>
 __device__ inline void q8_rows_out(const float xv[4], int lane, size_t off, size_t row, int b, int n,
                                    uint16_t *q16, float *dx, uint16_t *bs16) {
     int q[4];
@@ -165,13 +171,14 @@ __device__ inline void q8_rows_out(const float xv[4], int lane, size_t off, size
     q8k_wave_vals(xv, lane, q, d);
     const int gs = q8k_group_sum(q);
     uint2 o;
-    o.x = h16(q[0]) | (h16(q[1]) << 16);
-    o.y = h16(q[2]) | (h16(q[3]) << 16);
+    o.x = h16(q[0]) | (h16(q[MFMA ? 2 : 1]) << 16);
+    o.y = h16(q[MFMA ? 1 : 2]) | (h16(q[3]) << 16);
     *(uint2 *)(q16 + off) = o;
     if ((lane & 3) == 0) bs16[row * (n / 16) + b * 16 + (lane >> 2)] = (uint16_t)h16(gs);
     if (lane == 0) dx[row * (n / QK) + b] = d;
 }
 
+template <bool MFMA>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const void *src, int bf16, int n_rows, int n,
                                                          uint16_t *q16, float *dx, uint16_t *bs16) {
     const int lane = threadIdx.x & 63;
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const void *src, int bf
         const float4 v = *(const float4 *)((const float *)src + off);
         xv[0] = v.x; xv[1] = v.y; xv[2] = v.z; xv[3] = v.w;
     }
-    q8_rows_out(xv, lane, off, (size_t)row, b, n, q16, dx, bs16);
+    q8_rows_out<MFMA>(xv, lane, off, (size_t)row, b, n, q16, dx, bs16);
 }
 
 // SiLU with the canonical exp (the oracle evaluates the same function)
@@ -214,7 +221,7 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(const float *y2, int 
     const float hv[4] = {silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z), silu_mul(g.w, u.w)};
     const size_t off = (size_t)p * I + (size_t)b * QK + 4 * lane;
     if (h_out) *(float4 *)(h_out + off) = make_float4(hv[0], hv[1], hv[2], hv[3]);
-    q8_rows_out(hv, lane, off, (size_t)p, b, I, q16, dx, bs16);
+    q8_rows_out<true>(hv, lane, off, (size_t)p, b, I, q16, dx, bs16);
 }
 
 // ---------------------------------------------------------------------------
@@ -231,14 +238,16 @@ __device__ inline const uint8_t *grouped_expert(const GroupedArgs &a, int e) {
 }
 
 // 8 small unsigned bytes (two words) -> 8 fp16 holding 1024 + v: byte v under
-// the exponent byte 0x64 (1024 has a unit last place up to 2048)
+// the exponent byte 0x64 (1024 has a unit last place up to 2048).  Each word's
+// bytes in the order 0, 2, 1, 3, in which masks alone separate them (q4_tile_b);
+// the activation codes of the grouped products are stored in the same order.
 __device__ inline half8_t pack_1024(uint32_t w0, uint32_t w1) {
     const uint32_t K = 0x64646464u;
     uint4 r;
-    r.x = __builtin_amdgcn_perm(K, w0, 0x04010400u);
-    r.y = __builtin_amdgcn_perm(K, w0, 0x04030402u);
-    r.z = __builtin_amdgcn_perm(K, w1, 0x04010400u);
-    r.w = __builtin_amdgcn_perm(K, w1, 0x04030402u);
+    r.x = __builtin_amdgcn_perm(K, w0, 0x04020400u);
+    r.y = __builtin_amdgcn_perm(K, w0, 0x04030401u);
+    r.z = __builtin_amdgcn_perm(K, w1, 0x04020400u);
+    r.w = __builtin_amdgcn_perm(K, w1, 0x04030401u);
     return __builtin_bit_cast(half8_t, r);
 }
 
@@ -671,11 +680,11 @@ hipError_t launch_dispatch(const int32_t *ids, int P, int E, int32_t *counts, in
 }
 
 hipError_t launch_quant_rows(const void *src, int bf16, int n_rows, int n, uint16_t *q16, float *dx, uint16_t *bs16,
-                             hipStream_t st) {
+                             bool mfma_order, hipStream_t st) {
     const int64_t blocks = ((int64_t)n_rows * (n / QK) + 3) / 4;
     if (blocks == 0) return hipSuccess;
-    return launch_b(quant_rows_kernel, dim3((unsigned)blocks), dim3(256), st, nullptr, nullptr, src, bf16, n_rows, n,
-                    q16, dx, bs16);
+    return launch_b(mfma_order ? quant_rows_kernel<true> : quant_rows_kernel<false>, dim3((unsigned)blocks), dim3(256),
+                    st, nullptr, nullptr, src, bf16, n_rows, n, q16, dx, bs16);
 }
 
 hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, uint16_t *q16, float *dx, uint16_t *bs16,
@@ -687,23 +696,13 @@ hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, uint
 }
 
 // ---------------------------------------------------------------------------
-// The Q4_K grouped product with the weights read and decoded once per chunk
-// of up to CH passes (CH * 16 * MT pairs): for each super-block s, the lane's
-// weights are loaded once (block s+1 in flight meanwhile) and turned into the
-// eight MFMA B operands once, then every pass of the chunk multiplies its
-// staged activation rows by them.  Each pair still accumulates its
-// super-blocks in order 0, 1, ..., so the arithmetic is the one-pass kernel's.
-// CH = 2 for large batches, (256, 3): up to 168 registers, which the eight
-// operands of two passes need; CH = 1 when experts rarely get more than 32
-// pairs, (256, 4): four waves per SIMD.  MT = 1 (one 16-row M tile a pass)
-// when experts average at most 8 pairs: half the staged rows and products,
-// which would be empty anyway (batch 64 at 128 experts: up/gate 67.0 -> 63.4
-// us a launch, batch 16: 53.1 -> 51.1).  The (256, 5) bound, which the MT = 1
-// kernels fit without spills (73-94 registers), was no faster (batch 64:
-// 10,629 -> 10,633 tok/s).
-template <int NB, bool DOWN, int CH, int MT>
-__global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q4_kernel(GroupedArgs a) {
-    constexpr int GK = 16 * MT;           // pairs per pass: MT M tiles of 16
+// The Q4_K grouped product of few workgroups (see launch_gg): 64 rows of one
+// expert a workgroup, its pairs in passes of 16 on MFMA 16x16x32.  For each
+// super-block s the lane's weights are loaded once (block s + 1 in flight
+// meanwhile); four waves per SIMD.
+template <int NB, bool DOWN>
+__global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
+    constexpr int GK = 16;                // pairs per pass
     int e, tile;
     tile_expert(blockIdx.x, (DOWN ? a.H : 2 * a.I) / 64, a.E, tile, e);
     const int n0 = a.offsets[e], ne = a.offsets[e + 1] - n0;
@@ -731,8 +730,8 @@ __global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q4_kernel(Groupe
     const float *adx = DOWN ? a.hdx : a.xdx;
 
     __shared__ AStageR<GK> st[2];
-    __shared__ int s_rows[CH * GK];
-    __shared__ __attribute__((aligned(16))) float s_dx[NB][CH * GK];   // [block][pair]: a lane's 4 rows in one read
+    __shared__ int s_rows[GK];
+    __shared__ __attribute__((aligned(16))) float s_dx[NB][GK];   // [block][pair]: a lane's 4 rows in one read
     const int gm = (h >> 1) + 2 * (h & 1);
     // the expert's matrix, the activation codes and their group sums as raw
     // buffers; the lane's weight offsets (header, the two qs loads) fixed
@@ -740,34 +739,24 @@ __global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q4_kernel(Groupe
     const i32x4_t ra = raw_buffer(act, 0xffffffffu), rbs = raw_buffer(abs16, 0xffffffffu);
     const int wo0 = row * ROWB, wo1 = wo0 + 16 + 16 * h, wo2 = wo0 + 80 + 16 * h;
 
-    for (int cb = 0; cb < ne; cb += CH * GK) {
-        const int npc = min(CH * GK, ne - cb);
-        const int nps = (npc + GK - 1) / GK;
-        if (tid < CH * GK) {
-            const int pos = n0 + cb + min(tid, npc - 1);
+    for (int cb = 0; cb < ne; cb += GK) {
+        const int np = min(GK, ne - cb);
+        if (tid < GK) {
+            const int pos = n0 + cb + min(tid, np - 1);
             s_rows[tid] = DOWN ? pos : a.perm[pos] / a.K;
         }
         __syncthreads();
-        for (int i = tid; i < CH * GK * NB; i += 256) s_dx[i % NB][i / NB] = adx[(size_t)s_rows[i / NB] * NB + (i % NB)];
-        StageOff<GK> so[CH];
-#pragma unroll
-        for (int p = 0; p < CH; ++p)
-            if (p < nps) stage_offsets(so[p], s_rows + p * GK, min(GK, npc - p * GK), K, wave, lane);
-        stage_a_buf(st[0], so[0], min(GK, npc), ra, rbs, 0, wave);
+        for (int i = tid; i < GK * NB; i += 256) s_dx[i % NB][i / NB] = adx[(size_t)s_rows[i / NB] * NB + (i % NB)];
+        StageOff<GK> so;
+        stage_offsets(so, s_rows, np, K, wave, lane);
+        stage_a_buf(st[0], so, np, ra, rbs, 0, wave);
         uint4 cw[3], nw[3];
         cw[0] = buf_load16(rw, wo0, 0);
         cw[1] = buf_load16(rw, wo1, 0);
         cw[2] = buf_load16(rw, wo2, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        float y[CH][MT][4];
-#pragma unroll
-        for (int p = 0; p < CH; ++p)
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) y[p][t][i] = 0.0f;
-        int j = 0;                       // step j = s * nps + p
+        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
         for (int s = 0; s < NB; ++s) {
             if (s + 1 < NB) {
@@ -777,112 +766,55 @@ __global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q4_kernel(Groupe
             }
             Q4Scales sc;
             q4_scales(cw[0], h, sc);
-            half8_t b[CH > 1 ? 8 : 1];          // kept across the passes (one pass: built where used)
-            if constexpr (CH > 1) {
+            const AStageR<GK> &S = st[s & 1];
+            if (s + 1 < NB) stage_a_buf(st[(s + 1) & 1], so, np, ra, rbs, s + 1, wave);
+            // each 128-value half of the super-block in its own accumulator:
+            // a half's products sum to at most 128 * 63 * 15 * 127 < 2^24, so
+            // it is exact in fp32, and one add gives ggml's (float)sumi (a
+            // whole block's sum can pass 2^24, where a running fp32 sum rounds)
+            float4_t acc = {0, 0, 0, 0}, acc0;
+            // the fragments of K chunk i+1 are read before chunk i's products
+            half8_t fa[2];
+            fa[0] = stage_frag(S, n, q4_a_offset(h, 0));
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int L = i >> 2, nib = (i >> 1) & 1;
-                    b[i] = q4_b(L ? cw[2] : cw[1], i, sc.sc[L][nib]);
+            for (int i = 0; i < 8; ++i) {
+                if (i + 1 < 8) fa[(i + 1) & 1] = stage_frag(S, n, q4_a_offset(h, i + 1 < 8 ? i + 1 : 0));
+                const int L = i >> 2, nib = (i >> 1) & 1;
+                const half8_t bi = q4_b(L ? cw[2] : cw[1], i, sc.sc[L][nib]);
+                if (i == 4) {
+                    acc0 = acc;
+                    acc = float4_t{0, 0, 0, 0};
                 }
+                acc = mfma32(fa[i & 1], bi, acc);
             }
+            acc = acc0 + acc;
+            const float4 dxv = *(const float4 *)&s_dx[s][4 * h];
+            const half4_t am = *(const half4_t *)&S.bs[n][4 * gm];
+            float4_t z = {0, 0, 0, 0};
+            z = __builtin_amdgcn_mfma_f32_16x16x16f16(am, sc.bm, z, 0, 0, 0);
 #pragma unroll
-            for (int p = 0; p < CH; ++p) {
-                if (p < nps) {
-                    // two-pass chunks: a pass whose second M tile holds no pair skips its reads,
-                    // products and sums (512 tokens: up/gate 4.71 -> 4.62 ms per 48 layers;
-                    // in one-pass chunks the branch cost more than it saved)
-                    const bool full = MT == 1 || CH == 1 || npc - p * GK > 16;
-                    const AStageR<GK> &S = st[j & 1];
-                    const int jn = j + 1;
-                    if (jn < NB * nps) {
-                        const int s2 = jn / nps, p2 = jn - s2 * nps;
-                        // the pass's offsets by selects (a runtime index would put so in scratch)
-                        StageOff<GK> sp = so[0];
-                        if constexpr (CH > 1) {
-#pragma unroll
-                            for (int q = 0; q < GK / 8; ++q) sp.a[q] = p2 ? so[1].a[q] : so[0].a[q];
-                            sp.bs = p2 ? so[1].bs : so[0].bs;
-                        }
-                        stage_a_buf(st[jn & 1], sp, min(GK, npc - p2 * GK), ra, rbs, s2, wave);
-                    }
-                    // each 128-value half of the super-block in its own accumulator:
-                    // a half's products sum to at most 128 * 63 * 15 * 127 < 2^24, so
-                    // it is exact in fp32, and one add gives ggml's (float)sumi (a
-                    // whole block's sum can pass 2^24, where a running fp32 sum rounds)
-                    float4_t acc[MT], acc0[MT];
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[t] = float4_t{0, 0, 0, 0};
-                    // the fragments of K chunk i+1 are read before chunk i's products
-                    half8_t fa[2][MT];
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) if (t == 0 || full) fa[0][t] = stage_frag(S, 16 * t + n, q4_a_offset(h, 0));
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        if (i + 1 < 8) {
-#pragma unroll
-                            for (int t = 0; t < MT; ++t) if (t == 0 || full)
-                                fa[(i + 1) & 1][t] = stage_frag(S, 16 * t + n, q4_a_offset(h, i + 1 < 8 ? i + 1 : 0));
-                        }
-                        half8_t bi;
-                        if constexpr (CH > 1) {
-                            bi = b[i];
-                        } else {
-                            const int L = i >> 2, nib = (i >> 1) & 1;
-                            bi = q4_b(L ? cw[2] : cw[1], i, sc.sc[L][nib]);
-                        }
-                        if (i == 4) {
-#pragma unroll
-                            for (int t = 0; t < MT; ++t) {
-                                acc0[t] = acc[t];
-                                acc[t] = float4_t{0, 0, 0, 0};
-                            }
-                        }
-#pragma unroll
-                        for (int t = 0; t < MT; ++t) if (t == 0 || full) acc[t] = mfma32(fa[i & 1][t], bi, acc[t]);
-                    }
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[t] = acc0[t] + acc[t];
-                    float4 dxv[MT];
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) dxv[t] = *(const float4 *)&s_dx[s][p * GK + 16 * t + 4 * h];
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) if (t == 0 || full) {
-                        const half4_t am = *(const half4_t *)&S.bs[16 * t + n][4 * gm];
-                        float4_t z = {0, 0, 0, 0};
-                        z = __builtin_amdgcn_mfma_f32_16x16x16f16(am, sc.bm, z, 0, 0, 0);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            // ggml's order: acc += (d*dx)*sumi; acc -= (dmin*dx)*summ
-                            const float dx = i == 0 ? dxv[t].x : i == 1 ? dxv[t].y : i == 2 ? dxv[t].z : dxv[t].w;
-                            y[p][t][i] = y[p][t][i] + (sc.d * dx) * acc[t][i];
-                            y[p][t][i] = y[p][t][i] - (sc.dmin * dx) * z[i];
-                        }
-                    }
-                    __builtin_amdgcn_s_waitcnt(0);
-                    __syncthreads();
-                    ++j;
-                }
+            for (int i = 0; i < 4; ++i) {
+                // ggml's order: acc += (d*dx)*sumi; acc -= (dmin*dx)*summ
+                const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
+                y[i] = y[i] + (sc.d * dx) * acc[i];
+                y[i] = y[i] - (sc.dmin * dx) * z[i];
             }
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
             cw[0] = nw[0];
             cw[1] = nw[1];
             cw[2] = nw[2];
         }
 #pragma unroll
-        for (int p = 0; p < CH; ++p) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = p * GK + 16 * t + 4 * h + i;
-                    if (r < npc) {
-                        const int pos = n0 + cb + r;
-                        if (DOWN) {
-                            const int pp = a.perm[pos];
-                            a.ypair[(size_t)pp * a.H + row] = a.w[pp] * y[p][t][i];
-                        } else {
-                            a.y2[(size_t)pos * out_n + row] = y[p][t][i];
-                        }
-                    }
+        for (int i = 0; i < 4; ++i) {
+            const int r = 4 * h + i;
+            if (r < np) {
+                const int pos = n0 + cb + r;
+                if (DOWN) {
+                    const int pp = a.perm[pos];
+                    a.ypair[(size_t)pp * a.H + row] = a.w[pp] * y[i];
+                } else {
+                    a.y2[(size_t)pos * out_n + row] = y[i];
                 }
             }
         }
@@ -890,54 +822,408 @@ __global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q4_kernel(Groupe
     }
 }
 
-template <bool DOWN>
-static hipError_t launch_gg(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    const int rows = DOWN ? a.H : 2 * a.I;
-    const int nb = (DOWN ? a.I : a.H) / QK;
-    const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
-    const bool two = a.P > 16 * a.E;                            // many experts above 32 pairs
-    const bool one = a.P <= 8 * a.E;                            // few pairs: one 16-row M tile a pass
-    if (DOWN) {
-        if (a.down_type == TYPE_Q6K) {
-            if (two) {
-                if (nb == 3) return launch_b(grouped_q6_kernel<3, 2, 2>, grid, blk, st, e0, e1, a);
-                if (nb == 2) return launch_b(grouped_q6_kernel<2, 2, 2>, grid, blk, st, e0, e1, a);
-                return launch_b(grouped_q6_kernel<1, 2, 2>, grid, blk, st, e0, e1, a);
-            }
-            if (one) {
-                if (nb == 3) return launch_b(grouped_q6_kernel<3, 1, 1>, grid, blk, st, e0, e1, a);
-                if (nb == 2) return launch_b(grouped_q6_kernel<2, 1, 1>, grid, blk, st, e0, e1, a);
-                return launch_b(grouped_q6_kernel<1, 1, 1>, grid, blk, st, e0, e1, a);
-            }
-            if (nb == 3) return launch_b(grouped_q6_kernel<3, 1, 2>, grid, blk, st, e0, e1, a);
-            if (nb == 2) return launch_b(grouped_q6_kernel<2, 1, 2>, grid, blk, st, e0, e1, a);
-            return launch_b(grouped_q6_kernel<1, 1, 2>, grid, blk, st, e0, e1, a);
-        }
-        if (two) {
-            if (nb == 3) return launch_b(grouped_q4_kernel<3, true, 2, 2>, grid, blk, st, e0, e1, a);
-            if (nb == 2) return launch_b(grouped_q4_kernel<2, true, 2, 2>, grid, blk, st, e0, e1, a);
-            return launch_b(grouped_q4_kernel<1, true, 2, 2>, grid, blk, st, e0, e1, a);
-        }
-        if (one) {
-            if (nb == 3) return launch_b(grouped_q4_kernel<3, true, 1, 1>, grid, blk, st, e0, e1, a);
-            if (nb == 2) return launch_b(grouped_q4_kernel<2, true, 1, 1>, grid, blk, st, e0, e1, a);
-            return launch_b(grouped_q4_kernel<1, true, 1, 1>, grid, blk, st, e0, e1, a);
-        }
-        if (nb == 3) return launch_b(grouped_q4_kernel<3, true, 1, 2>, grid, blk, st, e0, e1, a);
-        if (nb == 2) return launch_b(grouped_q4_kernel<2, true, 1, 2>, grid, blk, st, e0, e1, a);
-        return launch_b(grouped_q4_kernel<1, true, 1, 2>, grid, blk, st, e0, e1, a);
+// ---------------------------------------------------------------------------
+// The Q4_K grouped product on MFMA 32x32x16 f16: a workgroup takes a chunk of up
+// to 32 MT pairs of one expert and rtw tiles of 128 rows (four waves of 32).
+//
+// What bounds it.  The 16-row kernel below reads a row's pieces 16 bytes a lane
+// with neighbouring lanes on different rows, so a load touches 64 separate 16-byte
+// pieces, and each of its waves reads all the activations of the pass from LDS
+// for 16 rows.  Here a wave's raw weights come into LDS lane-contiguous (9 lanes a
+// row's 144 bytes; that stride puts the 16 rows an LDS read touches in distinct
+// banks), no register holds a load in flight, a fragment serves 32 rows, and the
+// activations are staged half a super-block ahead of the products that read
+// them.  A lane decodes one nibble pair by v_and_or and v_pk_fma_f16 (1.1
+// instructions a weight).  An MFMA leaves the vector unit half of its issue slots
+// (measured: 32 cycles alone, 32 with 4 vector instructions, 48 with 8), so the
+// vector work (decode, and 7 instructions per output and super-block in ggml's
+// order) and the products add up rather than overlap: 352 us of up/gate at 4,096
+// tokens x 8 of 128 experts, of which the products alone are ~115.
+// MT = 1: 126 registers, four workgroups a CU, which few pairs per expert need to
+// keep weights in flight; MT = 3: a decode serves up to three tiles, two a CU.
+// us of up/gate (before / here), K = 8, E = 128, I = 768: 64 tokens 58.8 / 56.2,
+// 197 69 / 59, 512 97 / 78, 2,048 256 / 196, 4,096 468 / 352; down 36.0 / 32.8,
+// 44 / 35, 71 / 47, -, 403 / 215.
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef float float32_t __attribute__((ext_vector_type(32)));
+constexpr int TL_ROWS = 128;            // rows of a workgroup
+constexpr int TL_WB = 32 * Q4K_BYTES;   // one wave's raw weights of a super-block
+// A direct load into LDS, 16 bytes a lane, lane-contiguous at lds (it writes no
+// register).  Not by the builtin: the compiler waits for every such load in flight
+// before an LDS read it cannot tell apart.  These are waited for by hand (vmcnt,
+// then a barrier).  m0 holds nothing across statements here: no builtin that takes
+// it is used beside this one.
+__device__ inline void dma16(uint32_t lds, int voff, i32x4_t rsrc, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+__device__ inline uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(lptr_t *)p; }
+constexpr int TL_QUAD = 1024 + 16;      // half a super-block of four rows of activation codes in LDS
+__device__ void buffer_store_f32(float v, i32x4_t rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
+
+__device__ inline void vm_lds_barrier() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The experts' pairs in chunks of up to mt tiles of 32, an expert's tiles spread
+// evenly over its chunks; experts in order.  A wave finds chunk c from the
+// dispatch's offsets (4 experts a lane) and a prefix sum over the lanes.
+struct Chunk { int total, e, p0, np; };
+struct ChunkScan { int off[5], cnt[4], before, total; };
+__device__ inline ChunkScan chunk_scan(const int32_t *offsets, int E, int mt, int lane) {
+    ChunkScan r;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) r.off[j] = offsets[min(4 * lane + j, E)];
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int tiles = (r.off[j + 1] - r.off[j] + 31) / 32;
+        r.cnt[j] = (tiles + mt - 1) / mt;
+        sum += r.cnt[j];
     }
-    if (two) return launch_b(grouped_q4_kernel<8, false, 2, 2>, grid, blk, st, e0, e1, a);
-    if (one) return launch_b(grouped_q4_kernel<8, false, 1, 1>, grid, blk, st, e0, e1, a);
-    return launch_b(grouped_q4_kernel<8, false, 1, 2>, grid, blk, st, e0, e1, a);
+    const int incl = wave_incl_sum(sum, lane);
+    r.before = incl - sum;
+    r.total = __builtin_amdgcn_readlane(incl, 63);
+    return r;
+}
+__device__ inline Chunk chunk_find(const ChunkScan &s, int c, int lane) {
+    int e = -1, p0 = 0, np = 0, b = s.before;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int k = c - b;
+        if (k >= 0 && k < s.cnt[j]) {
+            const int n = s.off[j + 1] - s.off[j], tiles = (n + 31) / 32;
+            const int t0 = k * tiles / s.cnt[j], t1 = (k + 1) * tiles / s.cnt[j];
+            e = 4 * lane + j;
+            p0 = s.off[j] + 32 * t0;
+            np = min(n, 32 * t1) - 32 * t0;
+        }
+        b += s.cnt[j];
+    }
+    const int src = (int)__builtin_ctzll(__ballot(e >= 0));
+    return Chunk{s.total, __builtin_amdgcn_readlane(e, src), __builtin_amdgcn_readlane(p0, src),
+                 __builtin_amdgcn_readlane(np, src)};
+}
+
+// 4 nibbles' worth of B: words of nibbles under masks -> (1024 + q) * sc - 1024 * sc,
+// high nibbles as (1024 + 16 q) * (sc / 16) - 64 * sc: one rounding of an exact integer
+__device__ inline half8_t q4_tile_b(uint32_t w0, uint32_t w1, uint32_t M, uint32_t X, _Float16 s, _Float16 nb) {
+    uint4 r;
+    r.x = (w0 & M) | X;
+    r.y = ((w0 >> 8) & M) | X;
+    r.z = (w1 & M) | X;
+    r.w = ((w1 >> 8) & M) | X;
+    return __builtin_elementwise_fma(__builtin_bit_cast(half8_t, r), splat8(s), splat8(nb));
+}
+
+template <int NB, bool DOWN, int MT>
+__global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(GroupedArgs a, int rtw) {
+    constexpr int GK = 32 * MT;
+    constexpr int K = NB * QK;
+    constexpr int ROWB = NB * Q4K_BYTES;
+    const int out_n = DOWN ? a.H : 2 * a.I;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // workgroup -> (chunk, rtw row tiles): each XCD a contiguous run of them, a chunk's
+    // together
+    const int nt_r = out_n / (TL_ROWS * rtw);
+    const ChunkScan scan = chunk_scan(a.offsets, a.E, MT, lane);
+    const int total = scan.total * nt_r;
+    const int per = (total + 7) / 8, li = (int)blockIdx.x >> 3;
+    const int task = ((int)blockIdx.x & 7) * per + li;
+    if (li >= per || task >= total) return;
+    const Chunk ch = chunk_find(scan, task / nt_r, lane);
+    const int r0 = (task % nt_r) * (TL_ROWS * rtw);
+    const int np = ch.np, nt = (np + 31) / 32;
+    const uint8_t *base = grouped_expert(a, ch.e);
+    if (!base) {
+        for (int rt = 0; rt < rtw; ++rt)
+            for (int i = tid; i < np * TL_ROWS; i += 256) {
+                const int pos = ch.p0 + i / TL_ROWS, c = r0 + rt * TL_ROWS + (i % TL_ROWS);
+                if (DOWN) a.ypair[(size_t)a.perm[pos] * a.H + c] = 0.0f;
+                else a.y2[(size_t)pos * out_n + c] = 0.0f;
+            }
+        return;
+    }
+    const uint8_t *mat = DOWN ? base + 2ull * a.I * (a.H / QK) * Q4K_BYTES : base;
+    const float *adx = DOWN ? a.hdx : a.xdx;
+    const i32x4_t rw = raw_buffer(mat, (uint32_t)((DOWN ? a.H : 2 * a.I) * ROWB));
+    const i32x4_t ra = raw_buffer(DOWN ? a.ha : a.xa, 0xffffffffu), rbs = raw_buffer(DOWN ? a.hbs : a.xbs, 0xffffffffu);
+
+    // Activation codes, half a super-block at a time (the half's products read 8
+    // 16-byte chunks of each 128 values): four rows of 256 bytes per direct load,
+    // chunk c of row r at c ^ 4 (r & 3), four rows to 1040 bytes: the 16 rows one
+    // fragment read touches fall in distinct banks.
+    __shared__ __attribute__((aligned(16))) uint8_t s_a[2][GK / 4][TL_QUAD];
+    __shared__ __attribute__((aligned(16))) _Float16 s_bs[GK][16];
+    __shared__ __attribute__((aligned(16))) uint8_t s_w[4][TL_WB];
+    __shared__ __attribute__((aligned(16))) float s_dx[NB][GK];
+    __shared__ __attribute__((aligned(16))) int s_row[GK];                  // the pair's activation row, in bytes
+    __shared__ __attribute__((aligned(16))) uint32_t s_pp[DOWN ? GK : 4];   // its output row, in bytes
+    __shared__ __attribute__((aligned(16))) float s_gw[DOWN ? GK : 4];
+
+    // the wave's raw weights of super-block s: its 32 rows' 144 bytes, lane-contiguous (5 loads;
+    // the lane's offsets in LDS, as its activation rows are: the products need the registers)
+    __shared__ int s_wo[5][64];
+    for (int i = tid; i < 5 * 64; i += 256) s_wo[i >> 6][i & 63] = (i / 9) * ROWB + 16 * (i % 9);
+    const uint32_t lw = lds_addr(&s_w[wave][0]), la = lds_addr(&s_a[0][2 * wave][0]), lb = lds_addr(&s_bs[32 * wave][0]);
+    auto load_w = [&](int rt, int s) {            // of row tile rt
+        const int so = (r0 + TL_ROWS * rt + 32 * wave) * ROWB + s * Q4K_BYTES;
+        int o[5];
+#pragma unroll
+        for (int j = 0; j < 5; ++j) o[j] = s_wo[j][lane];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma16(lw + 1024 * j, o[j], rw, so);
+        if (lane < 32) dma16(lw + 4096, o[4], rw, so);
+    };
+    __syncthreads();
+    load_w(0, 0);
+    for (int i = tid; i < GK; i += 256) {
+        const int pos = ch.p0 + min(i, np - 1);
+        const int pr = a.perm[pos];
+        const int row = DOWN ? pos : pr / a.K;
+        s_row[i] = row * (2 * K);
+        if (DOWN) {
+            s_pp[i] = i < np ? (uint32_t)pr * (uint32_t)(4 * a.H) : 0xe0000000u;      // past the buffer: not stored
+            s_gw[i] = a.w[pr];
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) s_dx[b][i] = adx[(size_t)row * NB + b];
+    }
+    __syncthreads();
+    const int ac = ((lane & 15) ^ (4 * (lane >> 4)));
+    const int ao = 256 * (ac >> 3) + 16 * (ac & 7);
+    auto load_a = [&](auto ntc, int s, int hf) {          // half hf of super-block s
+        constexpr int NT = decltype(ntc)::value;
+        int o[NT][2];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) o[t][j] = s_row[4 * (8 * t + 2 * wave + j) + (lane >> 4)];
+        const int ob = hf ? s_row[32 * min(wave, NT - 1) + (lane >> 1)] : 0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                dma16(la + (hf * (GK / 4) + 8 * t + j) * TL_QUAD, o[t][j] + ao, ra, s * QK * 2 + 128 * hf);
+        if (hf && wave < NT) dma16(lb, ob / 16 + 16 * (lane & 1), rbs, s * 32);      // the group sums, for after the second half
+    };
+    const i32x4_t ro = DOWN ? raw_buffer(a.ypair, (uint32_t)a.P * (uint32_t)(4 * a.H))
+                            : raw_buffer(a.y2 + (size_t)ch.p0 * out_n, (uint32_t)np * (uint32_t)(4 * out_n));
+    const int n = lane & 31, h = lane >> 5;
+    const uint32_t hm = 0u - (uint32_t)h;
+    // the lane's fragments of its row in a half: chunks 8h + 0..3 and 8h + 4..7
+    const uint8_t *fr = &s_a[0][n >> 2][256 * (n & 3)];
+    const uint8_t *f0 = fr + 16 * ((8 * h) ^ (4 * (n & 3))), *f1 = fr + 16 * ((8 * h + 4) ^ (4 * (n & 3)));
+    auto frag = [&](int hf, int t, int i) {
+        return *(const half8_t *)((i < 4 ? f0 : f1) + 16 * (i & 3) + (hf * (GK / 4) + 8 * t) * TL_QUAD);
+    };
+    // masks and the exponent in registers: one v_and_or each
+    uint32_t mlo, mhi, mx;
+    asm("s_mov_b32 %0, 0x000f000f" : "=s"(mlo));
+    asm("s_mov_b32 %0, 0x00f000f0" : "=s"(mhi));
+    asm("v_mov_b32 %0, 0x64006400" : "=v"(mx));
+    float y[MT][16];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) y[t][i] = 0.0f;
+
+    // the chunk's NT tiles.  Written in the order it is to run in, fixed by the
+    // scheduling barriers: a product, the read of the fragment its register is
+    // needed for next, and beside them the vector work at hand (the decode of the
+    // next operand, or the sums of the tile before).
+    auto body = [&](auto ntc) {
+        constexpr int NT = decltype(ntc)::value;
+        load_a(ntc, 0, 0);
+        vm_lds_barrier();
+        load_a(ntc, 0, 1);
+        // the finished rows of a tile (rows past the chunk's pairs lie past the buffer's
+        // end: not stored), 16 NT stores
+        auto store = [&](int rt) {
+            const int col = 4 * (r0 + TL_ROWS * rt + 32 * wave + n) + (DOWN ? 0 : 16 * h * out_n);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int ru = 32 * t + 8 * (i >> 2) + (i & 3), r = ru + 4 * h;
+                    if (DOWN) buffer_store_f32(s_gw[r] * y[t][i], ro, (int)(s_pp[r] + (uint32_t)col), 0, 0);
+                    else buffer_store_f32(y[t][i], ro, ru * 4 * out_n + col, 0, 0);
+                    y[t][i] = 0.0f;
+                }
+        };
+        int rt = 0, s = 0;
+#pragma unroll 1
+        for (;;) {
+            const bool last = s == NB - 1 && rt == rtw - 1;
+            const int s1 = s == NB - 1 ? 0 : s + 1, rt1 = s == NB - 1 ? rt + 1 : rt;      // the next step
+            // the lane's half of its row's super-block: sub-blocks 4h .. 4h + 3
+            const uint8_t *wp = &s_w[wave][n * Q4K_BYTES];
+            const uint4 hdr = *(const uint4 *)wp;
+            uint4 q[4];
+#pragma unroll
+            for (int L = 0; L < 4; ++L) q[L] = *(const uint4 *)(wp + 16 + 64 * h + 16 * L);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // done with s_w
+            if (!last) load_w(rt1, s1);
+            // the rows of the tile before, behind the loads this step waits for
+            const bool stored = s == 0 && rt > 0;
+            if (stored) store(rt - 1);
+            half8_t f[8], b[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = frag(0, 0, i);
+            const uint32_t sc0 = hdr.y & 0x3f3f3f3fu, mn0 = hdr.z & 0x3f3f3f3fu;
+            const uint32_t sc1 = (hdr.w & 0x0f0f0f0fu) | ((hdr.y >> 2) & 0x30303030u);
+            const uint32_t mn1 = ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u);
+            const uint32_t scb = (sc1 & hm) | (sc0 & ~hm), mnb = (mn1 & hm) | (mn0 & ~hm);
+            // B of product i of half hf: 8 values of sub-block 4h + 2hf (low nibbles, i < 4) or the next (high)
+            _Float16 sf[2], sn[2];
+            auto scales = [&](int hf) {
+#pragma unroll
+                for (int nib = 0; nib < 2; ++nib) {
+                    const float sc = (float)((scb >> (8 * (2 * hf + nib))) & 0xffu);
+                    sf[nib] = (_Float16)(nib ? sc * 0.0625f : sc);
+                    sn[nib] = (_Float16)(sc * (nib ? -64.0f : -1024.0f));
+                }
+            };
+            auto operand = [&](int hf, int i) {
+                const uint4 &w = q[2 * hf + ((i >> 1) & 1)];
+                return q4_tile_b((i & 1) ? w.z : w.x, (i & 1) ? w.w : w.y, i < 4 ? mlo : mhi, mx, sf[i >> 2], sn[i >> 2]);
+            };
+            float16_t a0[NT];
+            scales(0);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (t == 0) b[i] = operand(0, i);
+                    a0[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[i], b[i], i ? a0[t] : float16_t{}, 0, 0, 0);
+                    if (t + 1 < NT) f[i] = frag(0, t + 1, i);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            const float d = h2f_dev((uint16_t)(hdr.x & 0xffffu)), dmin = h2f_dev((uint16_t)(hdr.x >> 16));
+            half8_t bm;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const _Float16 m = (_Float16)(float)((mnb >> (8 * j)) & 0xffu);
+                bm[2 * j] = m;
+                bm[2 * j + 1] = m;
+            }
+            scales(1);
+            // the second half has landed (only the next weights, 5 loads, and the stores stay in
+            // flight) and every wave is done with the first
+            if (last) {
+                vm_lds_barrier();
+            } else {
+                if (stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(5 + 16 * NT) : "memory");
+                else asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                load_a(ntc, s1, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = frag(1, 0, i);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                float16_t a1;
+                const half8_t am = *(const half8_t *)&s_bs[32 * t + n][8 * h];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (t == 0) b[i] = operand(1, i);
+                    a1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[i], b[i], i ? a1 : float16_t{}, 0, 0, 0);
+                    if (t + 1 < NT) f[i] = frag(1, t + 1, i);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const float16_t z = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, float16_t{}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float4 dx = *(const float4 *)&s_dx[s][32 * t + 8 * i + 4 * h];
+                    // ggml's order: acc += (d*dx)*sumi; acc -= (dmin*dx)*summ
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float x = j == 0 ? dx.x : j == 1 ? dx.y : j == 2 ? dx.z : dx.w;
+                        float &v = y[t][4 * i + j];
+                        v = v + (d * x) * (a0[t][4 * i + j] + a1[4 * i + j]);
+                        v = v - (dmin * x) * z[4 * i + j];
+                        asm volatile("" : "+v"(v));         // here, not at the end
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (last) break;
+            vm_lds_barrier();               // the next weights and first half; the second half and the sums are read
+            load_a(ntc, s1, 1);
+            s = s1;
+            rt = rt1;
+        }
+        store(rtw - 1);
+    };
+    if (MT >= 3 && nt == 3) body(std::integral_constant<int, MT < 3 ? 1 : 3>{});
+    else if (MT >= 2 && nt == 2) body(std::integral_constant<int, MT < 2 ? 1 : 2>{});
+    else body(std::integral_constant<int, 1>{});
+}
+
+template <bool DOWN, int MT>
+static hipError_t launch_tile(const GroupedArgs &a, int rtw, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
+    // chunks: at most P / (32 MT) full ones and one more per expert; the rest of the grid returns at once
+    const int64_t tasks = (int64_t)(a.P / (32 * MT) + a.E) * (rows / (TL_ROWS * rtw));
+    const dim3 grid((unsigned)((tasks + 7) / 8 * 8)), blk(256);
+    if constexpr (!DOWN) return launch_b(grouped_q4_tile_kernel<8, false, MT>, grid, blk, st, e0, e1, a, rtw);
+    else if (nb == 3) return launch_b(grouped_q4_tile_kernel<3, true, MT>, grid, blk, st, e0, e1, a, rtw);
+    else if (nb == 2) return launch_b(grouped_q4_tile_kernel<2, true, MT>, grid, blk, st, e0, e1, a, rtw);
+    else return launch_b(grouped_q4_tile_kernel<1, true, MT>, grid, blk, st, e0, e1, a, rtw);
+}
+
+// Which kernel a Q4_K product runs on.  `full` estimates the chunks of one tile
+// that the batch fills.
+//   few  fewer than 512 workgroups of 128 rows: the 64-row kernel has twice as many,
+//        while a pass or two serve an expert (us: 64 experts, I = 256, up/gate of
+//        64 tokens 14.4 there, 17.6 on tiles; 160 tokens 17.8 / 17.5)
+//   wide at least 64 pairs per expert and 600 workgroups of three tiles: those (us,
+//        one tile / three: up/gate of 1,500 x 8 of 128 158 / 153, 3,000 289 / 253;
+//        but 64 experts, I = 256, 2,000 tokens, 500 workgroups, 54 / 59).  With a slot pool also
+//        from 16 pairs on: an expert outside it is read from host memory once per chunk
+// Down rows (short K) take several row tiles a workgroup, which share its start (us: 512
+// tokens 48.7 with one, 46.8 with two; 4,096 255 with one, 215 with four of three tiles).
+template <bool DOWN>
+static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
+    const int rt = rows / TL_ROWS, full = max(a.P / 32, min(a.E, a.P));
+    if (full * rt < 512 && a.P <= 16 * a.E) {
+        const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
+        if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false>, grid, blk, st, e0, e1, a);
+        else if (nb == 3) return launch_b(grouped_q4_kernel<3, true>, grid, blk, st, e0, e1, a);
+        else if (nb == 2) return launch_b(grouped_q4_kernel<2, true>, grid, blk, st, e0, e1, a);
+        else return launch_b(grouped_q4_kernel<1, true>, grid, blk, st, e0, e1, a);
+    }
+    const int rtw3 = DOWN ? 4 : 1;
+    if ((a.P >= 64 * a.E && a.P / 96 * (rt / rtw3) >= 600) || (a.slot_pool && a.P > 16 * a.E))
+        return launch_tile<DOWN, 3>(a, rtw3, st, e0, e1);
+    return launch_tile<DOWN, 1>(a, DOWN && full * rt >= 2048 ? 2 : 1, st, e0, e1);
+}
+
+static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const int nb = a.I / QK;
+    const dim3 grid((unsigned)(a.H / 64 * a.E)), blk(256);      // (row tile, expert) from the linear id
+    if (a.P > 16 * a.E) {                                       // many experts above 32 pairs
+        if (nb == 3) return launch_b(grouped_q6_kernel<3, 2, 2>, grid, blk, st, e0, e1, a);
+        if (nb == 2) return launch_b(grouped_q6_kernel<2, 2, 2>, grid, blk, st, e0, e1, a);
+        return launch_b(grouped_q6_kernel<1, 2, 2>, grid, blk, st, e0, e1, a);
+    }
+    if (a.P <= 8 * a.E) {                                       // few pairs: one 16-row M tile a pass
+        if (nb == 3) return launch_b(grouped_q6_kernel<3, 1, 1>, grid, blk, st, e0, e1, a);
+        if (nb == 2) return launch_b(grouped_q6_kernel<2, 1, 1>, grid, blk, st, e0, e1, a);
+        return launch_b(grouped_q6_kernel<1, 1, 1>, grid, blk, st, e0, e1, a);
+    }
+    if (nb == 3) return launch_b(grouped_q6_kernel<3, 1, 2>, grid, blk, st, e0, e1, a);
+    if (nb == 2) return launch_b(grouped_q6_kernel<2, 1, 2>, grid, blk, st, e0, e1, a);
+    return launch_b(grouped_q6_kernel<1, 1, 2>, grid, blk, st, e0, e1, a);
 }
 
 hipError_t launch_gateup_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    return launch_gg<false>(a, st, e0, e1);
+    return launch_q4<false>(a, st, e0, e1);
 }
 
 hipError_t launch_down_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    return launch_gg<true>(a, st, e0, e1);
+    return a.down_type == TYPE_Q6K ? launch_q6(a, st, e0, e1) : launch_q4<true>(a, st, e0, e1);
 }
 
 hipError_t launch_iota(int n, int32_t *offsets, int32_t *perm, float *ones, hipStream_t st) {

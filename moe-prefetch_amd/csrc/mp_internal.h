@@ -240,11 +240,11 @@ struct GroupedArgs {
     int n_store;
     int E, K, H, I, down_type;
     int P;                      // pairs dispatched (n_tok * K): picks the pass chunking
-    const uint16_t *xa;         // [n_tok][H] Q8_K values of x as fp16
+    const uint16_t *xa;         // [n_tok][H] Q8_K values of x as fp16 (each four as 0, 2, 1, 3)
     const float *xdx;           // [n_tok][H/256]
     const uint16_t *xbs;        // [n_tok][H/16] group sums as fp16
     float *y2;                  // [P][2I] up and gate rows of every pair, dispatch order
-    const uint16_t *ha;         // [P][I] Q8_K of h as fp16
+    const uint16_t *ha;         // [P][I] Q8_K of h as fp16 (the same order)
     const float *hdx;           // [P][I/256]
     const uint16_t *hbs;        // [P][I/16]
     float *ypair;               // [P][H] weighted rows, pair (t*K + k) order
@@ -253,8 +253,9 @@ struct GroupedArgs {
 
 hipError_t launch_dispatch(const int32_t *ids, int P, int E, int32_t *counts, int32_t *offsets, int32_t *perm,
                            hipStream_t st);
+// mfma_order: each four codes in the order 0, 2, 1, 3 the grouped products read
 hipError_t launch_quant_rows(const void *src, int bf16, int n_rows, int n, uint16_t *q16, float *dx, uint16_t *bs16,
-                             hipStream_t st);
+                             bool mfma_order, hipStream_t st);
 hipError_t launch_gateup_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 hipError_t launch_down_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 hipError_t launch_combine(const float *ypair, int n_tok, int K, int H, float *out, int accumulate, hipStream_t st);

@@ -3514,7 +3514,8 @@ int moe_quant_rows(const void *src, int src_type, int n_rows, int n, uint16_t *q
         return fail(MOE_ERR_ARG, "moe_quant_rows: src_type %d unsupported", src_type);
     if (n_rows < 0 || n <= 0 || n % 256) return fail(MOE_ERR_ARG, "moe_quant_rows: n %d must be a multiple of 256", n);
     if (((uintptr_t)src | (uintptr_t)q16) % 16) return fail(MOE_ERR_ARG, "moe_quant_rows: src and q16 must be 16-byte aligned");
-    HIPCHK(mp::launch_quant_rows(src, src_type == MOE_DTYPE_BF16, n_rows, n, q16, d, bsum16, (hipStream_t)stream));
+    HIPCHK(mp::launch_quant_rows(src, src_type == MOE_DTYPE_BF16, n_rows, n, q16, d, bsum16, false,
+                                 (hipStream_t)stream));
     return MOE_OK;
 }
 
@@ -3588,7 +3589,7 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
     auto run = [&]() -> int {
         if (parts & GR_EXPERTS) {
             HIPCHK(mp::launch_quant_rows(d->x, d->x_type == MOE_DTYPE_BF16, d->n_tok, d->H, (uint16_t *)a.xa,
-                                         (float *)a.xdx, (uint16_t *)a.xbs, st));
+                                         (float *)a.xdx, (uint16_t *)a.xbs, true, st));
             HIPCHK(mp::launch_gateup_grouped(a, st, ev[0], ev[1]));
             HIPCHK(mp::launch_swiglu_quant(a.y2, P, d->I, d->h_out, (uint16_t *)a.ha, (float *)a.hdx,
                                            (uint16_t *)a.hbs, st));

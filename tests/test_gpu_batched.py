@@ -377,6 +377,41 @@ def test_grouped_experts_slots_pinned_and_absent():
     assert src[E - 1] == E and src[E - 2] == E
 
 
+# pairs of the first experts: the edges of one, two and three tiles of 32 pairs and of the chunks they
+# are spread over; the other experts share the rest of the batch
+TILE_EDGES = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 161, 193]
+
+
+@pytest.mark.parametrize("pool", [False, True], ids=["store", "pool"])
+@pytest.mark.parametrize("dt,I", [(_lib.TYPE_Q4K, 768), (_lib.TYPE_Q4K, 512), (_lib.TYPE_Q4K, 256)],
+                         ids=["q4k_i768", "q4k_i512", "q4k_i256"])
+def test_grouped_tile_edges(dt, I, pool):
+    """From a store: chunks of one tile.  With a slot pool (some experts in slots, some in the
+    store, the last in neither): chunks of up to three tiles, several row tiles a workgroup."""
+    E, K, T = 20, 8, 150
+    rng = np.random.default_rng(11 * I + pool)
+    store = Store(E, I, dt)
+    flat = np.concatenate([np.full(c, e) for e, c in enumerate(TILE_EDGES)] +
+                          [rng.choice(np.arange(len(TILE_EDGES), E), size=T * K - sum(TILE_EDGES))])
+    ids = rng.permutation(flat).reshape(T, K).astype(np.int32)
+    w = rng.random((T, K)).astype(np.float32)
+    src, kw = np.arange(E), {}
+    if pool:
+        slot_bytes, n_slots = (store.eb + 255) // 256 * 256, 12
+        table = np.full(E, n_slots, np.int32)
+        table[:n_slots] = rng.permutation(n_slots)
+        slots = torch.zeros(n_slots * slot_bytes, dtype=torch.uint8, device=DEV)
+        for e in range(n_slots):
+            slots[table[e] * slot_bytes:table[e] * slot_bytes + store.eb] = store.t[e * store.eb:(e + 1) * store.eb]
+        kw = dict(table=t_(table), slot_pool=slots.data_ptr(), slot_bytes=slot_bytes, n_slots=n_slots, n_store=E - 1)
+        src[E - 1] = E                          # expert E of the padded store: zeros
+    out, h_out, pair, perm, xh = run_grouped(store, T, K, E, ids, w, "f32", **kw)
+    host = np.concatenate([store.host, np.zeros(store.eb, np.uint8)])
+    want, want_h = O.moe_tokens(H, I, dt, host, store.eb, E, src[ids], w, xh, n_threads=16, want_h=True)
+    assert np.array_equal(h_out, want_h.reshape(T * K, I)[perm])
+    assert np.array_equal(out, want)
+
+
 def test_combine_accumulates_in_k_order():
     T, K = 9, 8
     rng = np.random.default_rng(2)
