@@ -2,7 +2,7 @@
 // decode at batch > 1).
 //
 //   dispatch_kernel      per-expert histogram, exclusive scan and the stable
-//                        permutation of (token, k) pairs (one workgroup)
+//                        permutation of (token, k) pairs
 //   quant_rows_kernel    Q8_K of rows (x per token) into the form the matrix
 //                        cores consume: the int8 values as fp16 codes, the
 //                        block scale, and the 16-value group sums as fp16 --
@@ -57,13 +57,17 @@ typedef __attribute__((address_space(3))) void lptr_t;
 // ---------------------------------------------------------------------------
 // dispatch: ids [P] (P = n_tok * K, pair i = t*K + k) -> counts[E], offsets[E+1],
 // perm[offsets[e] + r] = i of the r-th pair routed to e in pair order.
-// Pass 1 counts with LDS atomics (order-free) and one wave turns the counts
-// into offsets with a prefix sum (lane l holds experts 4l .. 4l+3); pass 2
-// places 64-pair chunks: lanes holding the same id find each other with 8
-// ballots (one per id bit), their rank inside the chunk is a popcount, and a
-// per-expert scan over the chunks of the pass (continuing a running count)
-// gives each chunk's base.
-constexpr int DSP_CHUNKS = 64;
+// A workgroup places a segment of 1,024 pairs, a wave a chunk of 64.  Every
+// workgroup counts all of ids with LDS atomics (order-free; the pairs before its
+// segment in the high half of the word), one wave turns the counts into offsets
+// with a prefix sum (lane l holds experts 4l .. 4l+3), and the pairs are ranked:
+// lanes holding the same id find each other with 8 ballots (one per id bit), their
+// rank inside the chunk is a popcount, and a per-expert scan over the segment's
+// chunks gives each chunk's base.  Counting everything in each workgroup (P <
+// 2^16 words from L2) costs less than a second launch or a hand-over, and needs
+// no scratch.  One workgroup placing 4,096 pairs a round took 11, 23, 37 and 70
+// us for 4,096, 8,000, 16,384 and 32,768 pairs.
+constexpr int DSP_WAVES = 16, DSP_SEG = 64 * DSP_WAVES;
 static_assert(MAX_E <= 256, "4 experts a lane in the offsets' prefix sum");
 
 // inclusive prefix sum over the 64 lanes of a wave
@@ -76,84 +80,71 @@ __device__ inline int wave_incl_sum(int v, int lane) {
     return v;
 }
 
-__global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *ids, int P, int E, int32_t *counts,
-                                                        int32_t *offsets, int32_t *perm) {
-    __shared__ int s_off[MAX_E + 1];
-    __shared__ int s_run[MAX_E];
-    __shared__ uint16_t s_c[DSP_CHUNKS][MAX_E];
+__global__ __launch_bounds__(64 * DSP_WAVES) void dispatch_kernel(const int32_t *ids, int P, int E, int32_t *counts,
+                                                                  int32_t *offsets, int32_t *perm) {
+    __shared__ uint32_t s_cnt[MAX_E];       // pairs of the expert: (before the segment << 16) | all
+    __shared__ int s_off[MAX_E];            // where the segment's first pair of the expert goes
+    __shared__ uint16_t s_c[DSP_WAVES][MAX_E];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < E; e += blockDim.x) { s_off[e] = 0; s_run[e] = 0; }
+    const int seg = (int)blockIdx.x * DSP_SEG;
+    for (int e = tid; e < E; e += 64 * DSP_WAVES) s_cnt[e] = 0;
+    for (int i = tid; i < DSP_WAVES * MAX_E; i += 64 * DSP_WAVES) ((uint16_t *)s_c)[i] = 0;
     __syncthreads();
-    for (int i = tid; i < P; i += blockDim.x) {
+#pragma unroll 8
+    for (int i = tid; i < P; i += 64 * DSP_WAVES) {
         const int e = ids[i];
-        if (e >= 0 && e < E) atomicAdd(&s_off[e], 1);
+        if (e >= 0 && e < E) atomicAdd(&s_cnt[e], i < seg ? 0x10001u : 1u);
     }
+    // the segment's own pairs, a chunk a wave
+    const int i = seg + tid;
+    const int e = i < P ? ids[i] : -1;
+    const bool valid = e >= 0 && e < E;
+    uint64_t m = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const bool bit = (e >> b) & 1;
+        const uint64_t bb = __ballot(valid && bit);
+        m &= bit ? bb : ~bb;
+    }
+    const int r = __popcll(m & ((1ull << lane) - 1ull));
+    if (valid && r == 0) s_c[wave][e] = (uint16_t)__popcll(m);
     __syncthreads();
     if (wave == 0) {
-        int c[4], sum = 0;
+        int c[4], before[4], sum = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int e = 4 * lane + j;
-            c[j] = e < E ? s_off[e] : 0;
+            const uint32_t w = 4 * lane + j < E ? s_cnt[4 * lane + j] : 0u;
+            c[j] = (int)(w & 0xffffu);
+            before[j] = (int)(w >> 16);
             sum += c[j];
         }
         const int incl = wave_incl_sum(sum, lane);
         int acc = incl - sum;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int e = 4 * lane + j;
-            if (e < E) {
-                counts[e] = c[j];
-                offsets[e] = acc;
-                s_off[e] = acc;
+            const int x = 4 * lane + j;
+            if (x < E) {
+                s_off[x] = acc + before[j];
+                if (seg == 0) {
+                    counts[x] = c[j];
+                    offsets[x] = acc;
+                }
             }
             acc += c[j];
         }
-        if (lane == 63) offsets[E] = incl;
+        if (lane == 63 && seg == 0) offsets[E] = incl;
+    }
+    for (int x = tid - 64; x >= 0 && x < E; x += 64 * (DSP_WAVES - 1)) {       // beside wave 0's prefix sum
+        int run = 0;
+#pragma unroll
+        for (int c = 0; c < DSP_WAVES; ++c) {
+            const int v = s_c[c][x];
+            s_c[c][x] = (uint16_t)run;
+            run += v;
+        }
     }
     __syncthreads();
-    const int nwaves = blockDim.x >> 6;
-    for (int base = 0; base < P; base += DSP_CHUNKS * 64) {
-        const int nc = min(DSP_CHUNKS, (P - base + 63) / 64);      // chunks holding pairs
-        for (int i = tid; i < nc * E; i += blockDim.x) s_c[i / E][i % E] = 0;
-        __syncthreads();
-        int my_e[DSP_CHUNKS / 16], my_r[DSP_CHUNKS / 16];
-        for (int j = 0, c = wave; c < DSP_CHUNKS; ++j, c += nwaves) {
-            if (c >= nc) break;
-            const int i = base + 64 * c + lane;
-            const int e = i < P ? ids[i] : -1;
-            const bool valid = e >= 0 && e < E;
-            uint64_t m = __ballot(valid);
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const bool bit = (e >> b) & 1;
-                const uint64_t bb = __ballot(valid && bit);
-                m &= bit ? bb : ~bb;
-            }
-            const int r = __popcll(m & ((1ull << lane) - 1ull));
-            if (valid && r == 0) s_c[c][e] = (uint16_t)__popcll(m);
-            my_e[j] = valid ? e : -1;
-            my_r[j] = r;
-        }
-        __syncthreads();
-        for (int e = tid; e < E; e += blockDim.x) {
-            int run = s_run[e];
-#pragma unroll 16
-            for (int c = 0; c < nc; ++c) {
-                const int v = s_c[c][e];
-                s_c[c][e] = (uint16_t)run;
-                run += v;
-            }
-            s_run[e] = run;
-        }
-        __syncthreads();
-        for (int j = 0, c = wave; c < DSP_CHUNKS; ++j, c += nwaves) {
-            if (c >= nc) break;
-            const int e = my_e[j];
-            if (e >= 0) perm[s_off[e] + s_c[c][e] + my_r[j]] = base + 64 * c + lane;
-        }
-        __syncthreads();
-    }
+    if (valid) perm[s_off[e] + s_c[wave][e] + r] = i;
 }
 
 // ---------------------------------------------------------------------------
@@ -676,7 +667,9 @@ static hipError_t launch_b(F k, dim3 grid, dim3 block, hipStream_t st, hipEvent_
 
 hipError_t launch_dispatch(const int32_t *ids, int P, int E, int32_t *counts, int32_t *offsets, int32_t *perm,
                            hipStream_t st) {
-    return launch_b(dispatch_kernel, dim3(1), dim3(1024), st, nullptr, nullptr, ids, P, E, counts, offsets, perm);
+    const unsigned segs = (unsigned)max(1, (P + DSP_SEG - 1) / DSP_SEG);
+    return launch_b(dispatch_kernel, dim3(segs), dim3(64 * DSP_WAVES), st, nullptr, nullptr, ids, P, E, counts, offsets,
+                    perm);
 }
 
 hipError_t launch_quant_rows(const void *src, int bf16, int n_rows, int n, uint16_t *q16, float *dx, uint16_t *bs16,

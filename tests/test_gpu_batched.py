@@ -87,6 +87,20 @@ def test_dispatch_bit_exact(case):
     assert np.array_equal(p[:T * K], op)
 
 
+@pytest.mark.parametrize("P", [1023, 1024, 1025, 2047, 2049, 16385, 65535])
+def test_dispatch_segment_edges(P):
+    """One pair a token: last segments of 1, 1,023 and 1,024 pairs; at the most pairs, one expert
+    that takes all but a few of them."""
+    rng = np.random.default_rng(P)
+    ids = rng.integers(-1, 129, size=(P, 1)).astype(np.int32)
+    if P == 65535:
+        ids = np.where(rng.random((P, 1)) < 0.999, 77, ids).astype(np.int32)
+    c, o, p = gpu_dispatch(ids, 128)
+    rc, ro, rp = ref_dispatch(ids, 128)
+    assert np.array_equal(c, rc) and np.array_equal(o, ro)
+    assert np.array_equal(p[:ro[-1]], rp)
+
+
 def test_dispatch_drops_ids_outside_range():
     rng = np.random.default_rng(3)
     ids = rng.integers(-3, 131, size=(200, 8)).astype(np.int32)
