@@ -15,7 +15,7 @@
 //                        to the pair's row
 //   grouped_q4_kernel    the same per (64-row tile, expert) on MFMA 16x16x32,
 //                        for shapes of few workgroups
-//   grouped_q6_kernel    the same for a Q6_K down matrix
+//   grouped_q6_tile_kernel, grouped_q6_kernel  the same for a Q6_K down matrix
 //   swiglu_quant_kernel  h = silu(gate) * up, and its Q8_K
 //   combine_kernel       out[t] = sum over k of the weighted rows, k in order
 //
@@ -456,18 +456,16 @@ __device__ inline void q6_lane_b(const Q6Lane &w, int i, int h, half8_t &bh, hal
     bl = __builtin_elementwise_fma(q, splat8(sl), splat8((_Float16)(float)(-1056 * (sc & 15))));
 }
 
-// The grouped down product for a Q6_K matrix, the lane's weights streamed from
-// HBM into registers as in grouped_q4_kernel (block s+1 in flight while block
-// s is multiplied, no LDS tile), in chunks of up to CH passes of MT M tiles of
-// 16 pairs: each block's weights are loaded once for the chunk and decoded per
-// pass.  CH = 1, (256, 4): four workgroups a CU; CH = 2 for large batches,
-// (256, 3).  A block's two integer sums stay below 2^24 (256 * 32 * 8 * 127
-// and 256 * 32 * 15 * 127), so each is exact and 16*acc_h + acc_l rounds once,
-// as ggml's (float)sumi.  y = the pair's gate weight times the row value, to
-// the pair's (t*K + k) row.
-template <int NB, int CH, int MT>
-__global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q6_kernel(GroupedArgs a) {
-    constexpr int GK = 16 * MT;
+// The grouped down product for a Q6_K matrix at I = 512 and few pairs (see
+// launch_q6): 64 rows of one expert a workgroup, the lane's weights streamed
+// from HBM into registers (block s + 1 in flight while block s is multiplied),
+// the pairs in passes of 16 on MFMA 16x16x32.  A block's two integer sums stay
+// below 2^24 (256 * 32 * 8 * 127 and 256 * 32 * 15 * 127), so each is exact and
+// 16*acc_h + acc_l rounds once, as ggml's (float)sumi.  y = the pair's gate
+// weight times the row value, to the pair's (t*K + k) row.
+template <int NB>
+__global__ __launch_bounds__(256, 4) void grouped_q6_kernel(GroupedArgs a) {
+    constexpr int GK = 16;
     int e, tile;
     tile_expert(blockIdx.x, a.H / 64, a.E, tile, e);
     const int n0 = a.offsets[e], ne = a.offsets[e + 1] - n0;
@@ -492,104 +490,58 @@ __global__ __launch_bounds__(256, CH == 1 ? 4 : 3) void grouped_q6_kernel(Groupe
     const Q6Off wo = q6_lane_offsets(row * (NB * Q6K_BYTES), h);
 
     __shared__ AStageR<GK> st[2];
-    __shared__ int s_rows[CH * GK];
-    __shared__ __attribute__((aligned(16))) float s_dx[NB][CH * GK];
+    __shared__ int s_rows[GK];
+    __shared__ __attribute__((aligned(16))) float s_dx[NB][GK];
 
-    for (int cb = 0; cb < ne; cb += CH * GK) {
-        const int npc = min(CH * GK, ne - cb);
-        const int nps = (npc + GK - 1) / GK;
-        if (tid < CH * GK) s_rows[tid] = n0 + cb + min(tid, npc - 1);   // h rows are in dispatch order
+    for (int cb = 0; cb < ne; cb += GK) {
+        const int np = min(GK, ne - cb);
+        if (tid < GK) s_rows[tid] = n0 + cb + min(tid, np - 1);   // h rows are in dispatch order
         __syncthreads();
-        for (int i = tid; i < CH * GK * NB; i += 256)
-            s_dx[i % NB][i / NB] = a.hdx[(size_t)s_rows[i / NB] * NB + (i % NB)];
-        StageOff<GK> so[CH];
-#pragma unroll
-        for (int p = 0; p < CH; ++p)
-            if (p < nps) stage_offsets(so[p], s_rows + p * GK, min(GK, npc - p * GK), K, wave, lane);
-        stage_a_buf<GK, false>(st[0], so[0], min(GK, npc), ra, ra, 0, wave);
+        for (int i = tid; i < GK * NB; i += 256) s_dx[i % NB][i / NB] = a.hdx[(size_t)s_rows[i / NB] * NB + (i % NB)];
+        StageOff<GK> so;
+        stage_offsets(so, s_rows, np, K, wave, lane);
+        stage_a_buf<GK, false>(st[0], so, np, ra, ra, 0, wave);
         Q6Lane cw, nw;
         q6_lane_load(cw, rw, wo, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        float y[CH][MT][4];
-#pragma unroll
-        for (int p = 0; p < CH; ++p)
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) y[p][t][i] = 0.0f;
-        int j = 0;                       // step j = s * nps + p
+        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
         for (int s = 0; s < NB; ++s) {
-            if (s + 1 < NB) q6_lane_load(nw, rw, wo, (s + 1) * Q6K_BYTES);
-            const float d = h2f_dev((uint16_t)cw.d);
-#pragma unroll
-            for (int p = 0; p < CH; ++p) {
-                if (p < nps) {
-                    // both M tiles always (skipping an empty second tile, as the Q4_K kernel does,
-                    // made this kernel ~1.7 us a launch slower at 512 tokens)
-                    constexpr bool full = true;
-                    const AStageR<GK> &S = st[j & 1];
-                    const int jn = j + 1;
-                    if (jn < NB * nps) {
-                        const int s2 = jn / nps, p2 = jn - s2 * nps;
-                        StageOff<GK> sp = so[0];
-                        if constexpr (CH > 1) {
-#pragma unroll
-                            for (int q = 0; q < GK / 8; ++q) sp.a[q] = p2 ? so[1].a[q] : so[0].a[q];
-                        }
-                        stage_a_buf<GK, false>(st[jn & 1], sp, min(GK, npc - p2 * GK), ra, ra, s2, wave);
-                    }
-                    float4_t acc[MT], accl[MT];
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[t] = accl[t] = float4_t{0, 0, 0, 0};
-                    half8_t fa[2][MT];
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) if (t == 0 || full) fa[0][t] = stage_frag(S, 16 * t + n, q6_a_offset(h, 0));
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        if (i + 1 < 8) {
-#pragma unroll
-                            for (int t = 0; t < MT; ++t) if (t == 0 || full)
-                                fa[(i + 1) & 1][t] = stage_frag(S, 16 * t + n, q6_a_offset(h, i + 1 < 8 ? i + 1 : 0));
-                        }
-                        half8_t bh, bl;
-                        q6_lane_b(cw, i, h, bh, bl);
-#pragma unroll
-                        for (int t = 0; t < MT; ++t) if (t == 0 || full) {
-                            acc[t] = mfma32(fa[i & 1][t], bh, acc[t]);
-                            accl[t] = mfma32(fa[i & 1][t], bl, accl[t]);
-                        }
-                    }
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) if (t == 0 || full) {
-                        const float4 dxv = *(const float4 *)&s_dx[s][p * GK + 16 * t + 4 * h];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
-                            const float sumi = 16.0f * acc[t][i] + accl[t][i];
-                            y[p][t][i] = y[p][t][i] + (d * dx) * sumi;   // ggml's order: acc += (d*dx)*sumi
-                        }
-                    }
-                    __builtin_amdgcn_s_waitcnt(0);
-                    __syncthreads();
-                    ++j;
-                }
+            if (s + 1 < NB) {
+                q6_lane_load(nw, rw, wo, (s + 1) * Q6K_BYTES);
+                stage_a_buf<GK, false>(st[(s + 1) & 1], so, np, ra, ra, s + 1, wave);
             }
+            const float d = h2f_dev((uint16_t)cw.d);
+            const AStageR<GK> &S = st[s & 1];
+            float4_t acc = {0, 0, 0, 0}, accl = {0, 0, 0, 0};
+            half8_t fa[2];
+            fa[0] = stage_frag(S, n, q6_a_offset(h, 0));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (i + 1 < 8) fa[(i + 1) & 1] = stage_frag(S, n, q6_a_offset(h, i + 1 < 8 ? i + 1 : 0));
+                half8_t bh, bl;
+                q6_lane_b(cw, i, h, bh, bl);
+                acc = mfma32(fa[i & 1], bh, acc);
+                accl = mfma32(fa[i & 1], bl, accl);
+            }
+            const float4 dxv = *(const float4 *)&s_dx[s][4 * h];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
+                const float sumi = 16.0f * acc[i] + accl[i];
+                y[i] = y[i] + (d * dx) * sumi;   // ggml's order: acc += (d*dx)*sumi
+            }
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
             cw = nw;
         }
 #pragma unroll
-        for (int p = 0; p < CH; ++p) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = p * GK + 16 * t + 4 * h + i;
-                    if (r < npc) {
-                        const int q = a.perm[n0 + cb + r];
-                        a.ypair[(size_t)q * a.H + row] = a.w[q] * y[p][t][i];
-                    }
-                }
+        for (int i = 0; i < 4; ++i) {
+            const int r = 4 * h + i;
+            if (r < np) {
+                const int q = a.perm[n0 + cb + r];
+                a.ypair[(size_t)q * a.H + row] = a.w[q] * y[i];
             }
         }
         __syncthreads();
@@ -851,6 +803,7 @@ __device__ inline void dma16(uint32_t lds, int voff, i32x4_t rsrc, int soff) {
                  :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
 }
 __device__ inline uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(lptr_t *)p; }
+constexpr uint32_t TL_NONE = 0xe0000000u;      // an offset past every buffer: reads zeros, is not stored
 constexpr int TL_QUAD = 1024 + 16;      // half a super-block of four rows of activation codes in LDS
 __device__ void buffer_store_f32(float v, i32x4_t rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
 
@@ -941,7 +894,12 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     const uint8_t *mat = DOWN ? base + 2ull * a.I * (a.H / QK) * Q4K_BYTES : base;
     const float *adx = DOWN ? a.hdx : a.xdx;
     const i32x4_t rw = raw_buffer(mat, (uint32_t)((DOWN ? a.H : 2 * a.I) * ROWB));
-    const i32x4_t ra = raw_buffer(DOWN ? a.ha : a.xa, 0xffffffffu), rbs = raw_buffer(DOWN ? a.hbs : a.xbs, 0xffffffffu);
+    // the activation rows; the rows past the chunk's pairs lie past the end and read as
+    // zeros, which costs the products no traffic and little power (a full tile of
+    // repeated rows slowed the whole of a 64-token batch by ~3 %)
+    const uint32_t n_rows = (uint32_t)(DOWN ? a.P : a.P / a.K);
+    const i32x4_t ra = raw_buffer(DOWN ? a.ha : a.xa, n_rows * (2 * K));
+    const i32x4_t rbs = raw_buffer(DOWN ? a.hbs : a.xbs, n_rows * (K / 8));
 
     // Activation codes, half a super-block at a time (the half's products read 8
     // 16-byte chunks of each 128 values): four rows of 256 bytes per direct load,
@@ -951,55 +909,60 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     __shared__ __attribute__((aligned(16))) _Float16 s_bs[GK][16];
     __shared__ __attribute__((aligned(16))) uint8_t s_w[4][TL_WB];
     __shared__ __attribute__((aligned(16))) float s_dx[NB][GK];
-    __shared__ __attribute__((aligned(16))) int s_row[GK];                  // the pair's activation row, in bytes
+    __shared__ __attribute__((aligned(16))) uint32_t s_row[GK];                 // the pair's activation row, in bytes
     __shared__ __attribute__((aligned(16))) uint32_t s_pp[DOWN ? GK : 4];   // its output row, in bytes
     __shared__ __attribute__((aligned(16))) float s_gw[DOWN ? GK : 4];
 
     // the wave's raw weights of super-block s: its 32 rows' 144 bytes, lane-contiguous (5 loads;
     // the lane's offsets in LDS, as its activation rows are: the products need the registers)
     __shared__ int s_wo[5][64];
-    for (int i = tid; i < 5 * 64; i += 256) s_wo[i >> 6][i & 63] = (i / 9) * ROWB + 16 * (i % 9);
     const uint32_t lw = lds_addr(&s_w[wave][0]), la = lds_addr(&s_a[0][2 * wave][0]), lb = lds_addr(&s_bs[32 * wave][0]);
-    auto load_w = [&](int rt, int s) {            // of row tile rt
+    auto load_w = [&](int rt, int s, bool first) {            // of row tile rt
         const int so = (r0 + TL_ROWS * rt + 32 * wave) * ROWB + s * Q4K_BYTES;
         int o[5];
 #pragma unroll
-        for (int j = 0; j < 5; ++j) o[j] = s_wo[j][lane];
+        for (int j = 0; j < 5; ++j) {
+            const int c = lane + 64 * j;
+            o[j] = first ? (c / 9) * ROWB + 16 * (c % 9) : s_wo[j][lane];
+            if (first && wave == 0) s_wo[j][lane] = o[j];
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) dma16(lw + 1024 * j, o[j], rw, so);
         if (lane < 32) dma16(lw + 4096, o[4], rw, so);
     };
-    __syncthreads();
-    load_w(0, 0);
+    load_w(0, 0, true);
     for (int i = tid; i < GK; i += 256) {
         const int pos = ch.p0 + min(i, np - 1);
-        const int pr = a.perm[pos];
-        const int row = DOWN ? pos : pr / a.K;
-        s_row[i] = row * (2 * K);
-        if (DOWN) {
-            s_pp[i] = i < np ? (uint32_t)pr * (uint32_t)(4 * a.H) : 0xe0000000u;      // past the buffer: not stored
-            s_gw[i] = a.w[pr];
-        }
+        const int row = DOWN ? pos : a.perm[pos] / a.K;
+        s_row[i] = i < np ? (uint32_t)row * (2 * K) : TL_NONE;
 #pragma unroll
         for (int b = 0; b < NB; ++b) s_dx[b][i] = adx[(size_t)row * NB + b];
     }
+    // the pairs' output rows and gate weights, fetched beside the first activations
+    auto pairs = [&]() {
+        for (int i = tid; i < GK; i += 256) {
+            const int pr = a.perm[ch.p0 + min(i, np - 1)];
+            s_pp[i] = i < np ? (uint32_t)pr * (uint32_t)(4 * a.H) : TL_NONE;        // not stored
+            s_gw[i] = a.w[pr];
+        }
+    };
     __syncthreads();
     const int ac = ((lane & 15) ^ (4 * (lane >> 4)));
     const int ao = 256 * (ac >> 3) + 16 * (ac & 7);
     auto load_a = [&](auto ntc, int s, int hf) {          // half hf of super-block s
         constexpr int NT = decltype(ntc)::value;
-        int o[NT][2];
+        uint32_t o[NT][2];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int j = 0; j < 2; ++j) o[t][j] = s_row[4 * (8 * t + 2 * wave + j) + (lane >> 4)];
-        const int ob = hf ? s_row[32 * min(wave, NT - 1) + (lane >> 1)] : 0;
+        const uint32_t ob = hf ? s_row[32 * min(wave, NT - 1) + (lane >> 1)] : 0;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                dma16(la + (hf * (GK / 4) + 8 * t + j) * TL_QUAD, o[t][j] + ao, ra, s * QK * 2 + 128 * hf);
-        if (hf && wave < NT) dma16(lb, ob / 16 + 16 * (lane & 1), rbs, s * 32);      // the group sums, for after the second half
+                dma16(la + (hf * (GK / 4) + 8 * t + j) * TL_QUAD, (int)(o[t][j] + ao), ra, s * QK * 2 + 128 * hf);
+        if (hf && wave < NT) dma16(lb, (int)(ob / 16 + 16 * (lane & 1)), rbs, s * 32);      // the group sums, for after the second half
     };
     const i32x4_t ro = DOWN ? raw_buffer(a.ypair, (uint32_t)a.P * (uint32_t)(4 * a.H))
                             : raw_buffer(a.y2 + (size_t)ch.p0 * out_n, (uint32_t)np * (uint32_t)(4 * out_n));
@@ -1029,6 +992,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     auto body = [&](auto ntc) {
         constexpr int NT = decltype(ntc)::value;
         load_a(ntc, 0, 0);
+        if (DOWN) pairs();
         vm_lds_barrier();
         load_a(ntc, 0, 1);
         // the finished rows of a tile (rows past the chunk's pairs lie past the buffer's
@@ -1057,7 +1021,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
 #pragma unroll
             for (int L = 0; L < 4; ++L) q[L] = *(const uint4 *)(wp + 16 + 64 * h + 16 * L);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // done with s_w
-            if (!last) load_w(rt1, s1);
+            if (!last) load_w(rt1, s1, false);
             // the rows of the tile before, behind the loads this step waits for
             const bool stored = s == 0 && rt > 0;
             if (stored) store(rt - 1);
@@ -1153,6 +1117,233 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     else body(std::integral_constant<int, 1>{});
 }
 
+// The same for a Q6_K down matrix (see q6_lane_b for the two exact products): the
+// raw weights of a wave's 32 rows come as the 14 aligned 16-byte pieces that hold
+// each row's 210-byte block, which starts at any even byte m of the first; a lane
+// reads its half of the block from LDS as words and shifts them by m & 2.  Whole
+// blocks' sums stay exact in one accumulator a product.  Bound by the decode (two
+// operands of every weight, ~410 vector instructions a super-block of 32 rows)
+// and, for few pairs, by the weights' latency.  us of down (before / here), E = 128,
+// I = 768: 16 tokens x 8 48 / 39, 64 62 / 51, 512 100 / 69, 2,000 266 / 163.
+constexpr int TL_W6 = 224;              // a row's pieces in LDS
+template <int NB, int MT>
+__global__ __launch_bounds__(256, MT == 1 ? 3 : 2) void grouped_q6_tile_kernel(GroupedArgs a, int rtw) {
+    constexpr int GK = 32 * MT;
+    constexpr int K = NB * QK;
+    constexpr int ROWB = NB * Q6K_BYTES;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nt_r = a.H / (TL_ROWS * rtw);
+    const ChunkScan scan = chunk_scan(a.offsets, a.E, MT, lane);
+    const int total = scan.total * nt_r;
+    const int per = (total + 7) / 8, li = (int)blockIdx.x >> 3;
+    const int task = ((int)blockIdx.x & 7) * per + li;
+    if (li >= per || task >= total) return;
+    const Chunk ch = chunk_find(scan, task / nt_r, lane);
+    const int r0 = (task % nt_r) * (TL_ROWS * rtw);
+    const int np = ch.np, nt = (np + 31) / 32;
+    const uint8_t *base = grouped_expert(a, ch.e);
+    if (!base) {
+        for (int rt = 0; rt < rtw; ++rt)
+            for (int i = tid; i < np * TL_ROWS; i += 256)
+                a.ypair[(size_t)a.perm[ch.p0 + i / TL_ROWS] * a.H + r0 + rt * TL_ROWS + (i % TL_ROWS)] = 0.0f;
+        return;
+    }
+    const i32x4_t rw = raw_buffer(base + 2ull * a.I * (a.H / QK) * Q4K_BYTES, (uint32_t)(a.H * ROWB));
+    const i32x4_t ra = raw_buffer(a.ha, (uint32_t)a.P * (2 * K));
+    const i32x4_t ro = raw_buffer(a.ypair, (uint32_t)a.P * (uint32_t)(4 * a.H));
+
+    __shared__ __attribute__((aligned(16))) uint8_t s_a[2][GK / 4][TL_QUAD];       // as in the Q4_K kernel
+    __shared__ __attribute__((aligned(16))) uint8_t s_w[4][32 * TL_W6];
+    __shared__ __attribute__((aligned(16))) float s_dx[NB][GK];
+    __shared__ __attribute__((aligned(16))) uint32_t s_row[GK];
+    __shared__ __attribute__((aligned(16))) uint32_t s_pp[GK];
+    __shared__ __attribute__((aligned(16))) float s_gw[GK];
+    __shared__ uint32_t s_wo[7][64];                // piece c = 64 j + lane: row c / 14 (bytes), 16 (c % 14) above
+    const uint32_t lw = lds_addr(&s_w[wave][0]), la = lds_addr(&s_a[0][2 * wave][0]);
+    auto load_w = [&](int rt, int s, bool first) {              // 7 loads; 32 rows are a multiple of 16 bytes
+        const int so = (r0 + TL_ROWS * rt + 32 * wave) * ROWB;
+        uint32_t o[7];
+#pragma unroll
+        for (int j = 0; j < 7; ++j) {
+            const int c = lane + 64 * j;
+            o[j] = first ? (uint32_t)((c / 14) * ROWB) | ((uint32_t)(16 * (c % 14)) << 16) : s_wo[j][lane];
+            if (first && wave == 0) s_wo[j][lane] = o[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 7; ++j)
+            dma16(lw + 1024 * j, (int)((((o[j] & 0xffffu) + s * Q6K_BYTES) & ~15u) + (o[j] >> 16)), rw, so);
+    };
+    load_w(0, 0, true);
+    for (int i = tid; i < GK; i += 256) {
+        const int pos = ch.p0 + min(i, np - 1);
+        s_row[i] = i < np ? (uint32_t)pos * (2 * K) : TL_NONE;      // (zeros, as in the Q4_K kernel)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) s_dx[b][i] = a.hdx[(size_t)pos * NB + b];
+    }
+    auto pairs = [&]() {
+        for (int i = tid; i < GK; i += 256) {
+            const int pr = a.perm[ch.p0 + min(i, np - 1)];
+            s_pp[i] = i < np ? (uint32_t)pr * (uint32_t)(4 * a.H) : TL_NONE;        // not stored
+            s_gw[i] = a.w[pr];
+        }
+    };
+    __syncthreads();
+    const int ac = ((lane & 15) ^ (4 * (lane >> 4)));
+    const int ao = 256 * (ac >> 3) + 16 * (ac & 7);
+    auto load_a = [&](auto ntc, int s, int hf) {
+        constexpr int NT = decltype(ntc)::value;
+        uint32_t o[NT][2];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) o[t][j] = s_row[4 * (8 * t + 2 * wave + j) + (lane >> 4)];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                dma16(la + (hf * (GK / 4) + 8 * t + j) * TL_QUAD, (int)(o[t][j] + ao), ra, s * QK * 2 + 128 * hf);
+    };
+    const int n = lane & 31, h = lane >> 5;
+    const uint8_t *fr = &s_a[0][n >> 2][256 * (n & 3)];
+    const uint8_t *f0 = fr + 16 * ((8 * h) ^ (4 * (n & 3))), *f1 = fr + 16 * ((8 * h + 4) ^ (4 * (n & 3)));
+    auto frag = [&](int hf, int t, int i) {
+        return *(const half8_t *)((i < 4 ? f0 : f1) + 16 * (i & 3) + (hf * (GK / 4) + 8 * t) * TL_QUAD);
+    };
+    float y[MT][16];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) y[t][i] = 0.0f;
+
+    auto body = [&](auto ntc) {
+        constexpr int NT = decltype(ntc)::value;
+        load_a(ntc, 0, 0);
+        pairs();
+        vm_lds_barrier();
+        load_a(ntc, 0, 1);
+        auto store = [&](int rt) {                  // 16 NT stores
+            const int col = 4 * (r0 + TL_ROWS * rt + 32 * wave + n);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int r = 32 * t + 8 * (i >> 2) + (i & 3) + 4 * h;
+                    buffer_store_f32(s_gw[r] * y[t][i], ro, (int)(s_pp[r] + (uint32_t)col), 0, 0);
+                    y[t][i] = 0.0f;
+                }
+        };
+        int rt = 0, s = 0;
+#pragma unroll 1
+        for (;;) {
+            const bool last = s == NB - 1 && rt == rtw - 1;
+            const int s1 = s == NB - 1 ? 0 : s + 1, rt1 = s == NB - 1 ? rt + 1 : rt;      // the next step
+            // the lane's half of its row's block: ql 64 bytes, qh 32, 8 scales, and d
+            const int m = (n * ROWB + s * Q6K_BYTES) & 15;
+            const uint8_t *wp = &s_w[wave][n * TL_W6 + (m & ~3)];
+            uint32_t ql[17], qh[9], qs[3];
+            __builtin_memcpy(ql, __builtin_assume_aligned(wp + 64 * h, 4), 68);
+            __builtin_memcpy(qh, __builtin_assume_aligned(wp + 128 + 32 * h, 4), 36);
+            __builtin_memcpy(qs, __builtin_assume_aligned(wp + 192 + 8 * h, 4), 12);
+            const float d = h2f_dev(*(const uint16_t *)(wp + 208 + (m & 2)));
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // done with s_w
+            if (!last) load_w(rt1, s1, false);
+            const bool stored = s == 0 && rt > 0;
+            if (stored) store(rt - 1);
+            half8_t f[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = frag(0, 0, i);
+            const uint32_t sb = (uint32_t)(m & 2);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) ql[j] = __builtin_amdgcn_alignbyte(ql[j + 1], ql[j], sb);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) qh[j] = __builtin_amdgcn_alignbyte(qh[j + 1], qh[j], sb);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) qs[j] = __builtin_amdgcn_alignbyte(qs[j + 1], qs[j], sb);
+            // B of product i of half hf: values 8 (i & 3) .. of group g = 2 hf + (i >> 2), of scale 2 g + ((i >> 1) & 1)
+            _Float16 sh[4], sl[4];
+            auto scales = [&](int hf) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int sc = (int)qs[hf] << (24 - 8 * j) >> 24;
+                    sh[j] = (_Float16)(short)(sc >> 4);
+                    sl[j] = (_Float16)(short)(sc & 15);
+                }
+            };
+            auto operand = [&](int hf, int i, half8_t &bh, half8_t &bl) {
+                const uint32_t M = 0x0F0F0F0Fu, HM = 0x30303030u;
+                const int g = 2 * hf + (i >> 2), k = i & 3;
+                uint32_t v[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const uint32_t lw_ = ql[8 * (g & 1) + 2 * k + j], hw = qh[2 * k + j];
+                    const uint32_t lo = (g >= 2 ? lw_ >> 4 : lw_) & M;
+                    const uint32_t hi = (g == 0 ? hw << 4 : g == 1 ? hw << 2 : g == 2 ? hw : hw >> 2) & HM;
+                    v[j] = lo | hi;
+                }
+                const half8_t q = pack_1024(v[0], v[1]);
+                const _Float16 s0 = sh[2 * (i >> 2) + (k >> 1)], s1_ = sl[2 * (i >> 2) + (k >> 1)];
+                bh = __builtin_elementwise_fma(q, splat8(s0), splat8(s0 * (_Float16)-1056.0f));
+                bl = __builtin_elementwise_fma(q, splat8(s1_), splat8(s1_ * (_Float16)-1056.0f));
+            };
+            float16_t ah[NT], al[NT];
+            half8_t bh[8], bl[8];
+            auto half = [&](auto hfc) {
+                constexpr int hf = decltype(hfc)::value;
+                scales(hf);
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        if (t == 0) operand(hf, i, bh[i], bl[i]);
+                        const bool first = hf == 0 && i == 0;
+                        ah[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[i], bh[i], first ? float16_t{} : ah[t], 0, 0, 0);
+                        al[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[i], bl[i], first ? float16_t{} : al[t], 0, 0, 0);
+                        if (t + 1 < NT) f[i] = frag(hf, t + 1, i);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            };
+            half(std::integral_constant<int, 0>{});
+            // the second half has landed (only the next weights, 7 loads, and the stores stay in
+            // flight) and every wave is done with the first
+            if (last) {
+                vm_lds_barrier();
+            } else {
+                if (stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(7 + 16 * NT) : "memory");
+                else asm volatile("s_waitcnt vmcnt(7) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                load_a(ntc, s1, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = frag(1, 0, i);
+            half(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float4 dx = *(const float4 *)&s_dx[s][32 * t + 8 * i + 4 * h];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float x = j == 0 ? dx.x : j == 1 ? dx.y : j == 2 ? dx.z : dx.w;
+                        float &v = y[t][4 * i + j];
+                        // ggml's order: acc += (d*dx)*sumi; 16 ah is exact, so the fmaf rounds once
+                        v = v + (d * x) * fmaf(16.0f, ah[t][4 * i + j], al[t][4 * i + j]);
+                        asm volatile("" : "+v"(v));
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (last) break;
+            vm_lds_barrier();               // the next weights and first half; the second half is read
+            load_a(ntc, s1, 1);
+            s = s1;
+            rt = rt1;
+        }
+        store(rtw - 1);
+    };
+    if (MT >= 2 && nt == 2) body(std::integral_constant<int, MT < 2 ? 1 : 2>{});
+    else body(std::integral_constant<int, 1>{});
+}
+
 template <bool DOWN, int MT>
 static hipError_t launch_tile(const GroupedArgs &a, int rtw, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
@@ -1168,8 +1359,8 @@ static hipError_t launch_tile(const GroupedArgs &a, int rtw, hipStream_t st, hip
 // Which kernel a Q4_K product runs on.  `full` estimates the chunks of one tile
 // that the batch fills.
 //   few  fewer than 512 workgroups of 128 rows: the 64-row kernel has twice as many,
-//        while a pass or two serve an expert (us: 64 experts, I = 256, up/gate of
-//        64 tokens 14.4 there, 17.6 on tiles; 160 tokens 17.8 / 17.5)
+//        while a pass of 16 pairs serves an expert (us: 64 experts, I = 256, up/gate of
+//        64 tokens 14.4 there, 17.6 on tiles; 128 tokens 19.9 / 17.7)
 //   wide at least 64 pairs per expert and 600 workgroups of three tiles: those (us,
 //        one tile / three: up/gate of 1,500 x 8 of 128 158 / 153, 3,000 289 / 253;
 //        but 64 experts, I = 256, 2,000 tokens, 500 workgroups, 54 / 59).  With a slot pool also
@@ -1180,7 +1371,7 @@ template <bool DOWN>
 static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
     const int rt = rows / TL_ROWS, full = max(a.P / 32, min(a.E, a.P));
-    if (full * rt < 512 && a.P <= 16 * a.E) {
+    if (full * rt < 512 && a.P <= 8 * a.E) {
         const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
         if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false>, grid, blk, st, e0, e1, a);
         else if (nb == 3) return launch_b(grouped_q4_kernel<3, true>, grid, blk, st, e0, e1, a);
@@ -1193,22 +1384,29 @@ static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0,
     return launch_tile<DOWN, 1>(a, DOWN && full * rt >= 2048 ? 2 : 1, st, e0, e1);
 }
 
-static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+template <int MT>
+static hipError_t launch_tile6(const GroupedArgs &a, int rtw, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int nb = a.I / QK;
-    const dim3 grid((unsigned)(a.H / 64 * a.E)), blk(256);      // (row tile, expert) from the linear id
-    if (a.P > 16 * a.E) {                                       // many experts above 32 pairs
-        if (nb == 3) return launch_b(grouped_q6_kernel<3, 2, 2>, grid, blk, st, e0, e1, a);
-        if (nb == 2) return launch_b(grouped_q6_kernel<2, 2, 2>, grid, blk, st, e0, e1, a);
-        return launch_b(grouped_q6_kernel<1, 2, 2>, grid, blk, st, e0, e1, a);
-    }
-    if (a.P <= 8 * a.E) {                                       // few pairs: one 16-row M tile a pass
-        if (nb == 3) return launch_b(grouped_q6_kernel<3, 1, 1>, grid, blk, st, e0, e1, a);
-        if (nb == 2) return launch_b(grouped_q6_kernel<2, 1, 1>, grid, blk, st, e0, e1, a);
-        return launch_b(grouped_q6_kernel<1, 1, 1>, grid, blk, st, e0, e1, a);
-    }
-    if (nb == 3) return launch_b(grouped_q6_kernel<3, 1, 2>, grid, blk, st, e0, e1, a);
-    if (nb == 2) return launch_b(grouped_q6_kernel<2, 1, 2>, grid, blk, st, e0, e1, a);
-    return launch_b(grouped_q6_kernel<1, 1, 2>, grid, blk, st, e0, e1, a);
+    const int64_t tasks = (int64_t)(a.P / (32 * MT) + a.E) * (a.H / (TL_ROWS * rtw));
+    const dim3 grid((unsigned)((tasks + 7) / 8 * 8)), blk(256);
+    if (nb == 3) return launch_b(grouped_q6_tile_kernel<3, MT>, grid, blk, st, e0, e1, a, rtw);
+    if (nb == 2) return launch_b(grouped_q6_tile_kernel<2, MT>, grid, blk, st, e0, e1, a, rtw);
+    return launch_b(grouped_q6_tile_kernel<1, MT>, grid, blk, st, e0, e1, a, rtw);
+}
+
+// Which kernel a Q6_K down product runs on.
+//   I = 512, half a pair to 4 pairs per expert: the 64-row kernel (us, there / on tiles:
+//        256 experts, 16 tokens 33.3 / 36.7, 128 tokens 75.0 / 77.8; below and above that range
+//        8 tokens 28.7 / 25.0, 512 tokens 89.9 / 81.5; I = 768, 128 experts, 64 tokens 62.4 / 50.5)
+//   two tiles a chunk from 48 pairs per expert on (us, one / two: 32 pairs 68.8 / 69.1, 62
+//        pairs 104 / 100, 188 pairs 273 / 238); with a slot pool from 16 on, as for Q4_K
+// Two row tiles a workgroup, but one below two pairs per expert (us, one / two: 128
+// experts, 24 tokens 43 / 48, 1,000 tokens 111 / 104).
+static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    if (a.I == 512 && 2 * a.P > a.E && a.P <= 4 * a.E)
+        return launch_b(grouped_q6_kernel<2>, dim3((unsigned)(a.H / 64 * a.E)), dim3(256), st, e0, e1, a);
+    if (a.P >= 48 * a.E || (a.slot_pool && a.P > 16 * a.E)) return launch_tile6<2>(a, 2, st, e0, e1);
+    return launch_tile6<1>(a, a.P < 2 * a.E ? 1 : 2, st, e0, e1);
 }
 
 hipError_t launch_gateup_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {

@@ -397,8 +397,9 @@ TILE_EDGES = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 161, 193]
 
 
 @pytest.mark.parametrize("pool", [False, True], ids=["store", "pool"])
-@pytest.mark.parametrize("dt,I", [(_lib.TYPE_Q4K, 768), (_lib.TYPE_Q4K, 512), (_lib.TYPE_Q4K, 256)],
-                         ids=["q4k_i768", "q4k_i512", "q4k_i256"])
+@pytest.mark.parametrize("dt,I", [(_lib.TYPE_Q4K, 768), (_lib.TYPE_Q4K, 512), (_lib.TYPE_Q4K, 256), (_lib.TYPE_Q6K, 768),
+                                  (_lib.TYPE_Q6K, 512), (_lib.TYPE_Q6K, 256)],
+                         ids=["q4k_i768", "q4k_i512", "q4k_i256", "q6k_i768", "q6k_i512", "q6k_i256"])
 def test_grouped_tile_edges(dt, I, pool):
     """From a store: chunks of one tile.  With a slot pool (some experts in slots, some in the
     store, the last in neither): chunks of up to three tiles, several row tiles a workgroup."""
