@@ -197,9 +197,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const void *src, int bf
 __device__ inline float silu_mul(float g, float u) { return g / (1.0f + canon_expf(-g)) * u; }
 
 // h = silu(gate) * up from the up/gate rows y2 [P][2I] (up first), then its
-// Q8_K: one wavefront per (pair, 256-value block); h itself to h_out if given
-__global__ __launch_bounds__(256) void swiglu_quant_kernel(const float *y2, int P, int I, float *h_out, uint16_t *q16,
-                                                           float *dx, uint16_t *bs16) {
+// Q8_K: one wavefront per (pair, 256-value block); h itself of the first n_h pairs
+// to h_out if given
+__global__ __launch_bounds__(256) void swiglu_quant_kernel(const float *y2, int P, int I, float *h_out, int n_h,
+                                                           uint16_t *q16, float *dx, uint16_t *bs16) {
     const int lane = threadIdx.x & 63;
     const int nb = I / QK;
     const int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(const float *y2, int 
     const float4 g = *(const float4 *)(yr + I);
     const float hv[4] = {silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z), silu_mul(g.w, u.w)};
     const size_t off = (size_t)p * I + (size_t)b * QK + 4 * lane;
-    if (h_out) *(float4 *)(h_out + off) = make_float4(hv[0], hv[1], hv[2], hv[3]);
+    if (h_out && p < n_h) *(float4 *)(h_out + off) = make_float4(hv[0], hv[1], hv[2], hv[3]);
     q8_rows_out<true>(hv, lane, off, (size_t)p, b, I, q16, dx, bs16);
 }
 
@@ -562,9 +563,10 @@ __global__ void iota_kernel(int n, int32_t *offsets, int32_t *perm, float *ones)
     }
 }
 
-// out[t] (+)= sum_k ypair[t*K + k], k ascending; one float4 per thread
-__global__ __launch_bounds__(256) void combine_kernel(const float *ypair, int n_tok, int K, int H, float *out,
-                                                      int accumulate) {
+// out[t] (+)= sum_k ypair[t*K + k], k ascending, then the shared expert's row
+// yshared[t] if given; one float4 per thread
+__global__ __launch_bounds__(256) void combine_kernel(const float *ypair, const float *yshared, int n_tok, int K, int H,
+                                                      float *out, int accumulate) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t h4 = (size_t)H / 4;
     if (i >= (size_t)n_tok * h4) return;
@@ -580,13 +582,18 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *ypair, int n_
         const float4 p = *o;
         s.x = p.x + s.x; s.y = p.y + s.y; s.z = p.z + s.z; s.w = p.w + s.w;
     }
+    if (yshared) {
+        const float4 v = ((const float4 *)yshared)[i];
+        s.x = s.x + v.x; s.y = s.y + v.y; s.z = s.z + v.z; s.w = s.w + v.w;
+    }
     *o = s;
 }
 
 // the same with the host's rows: pair i's row from hrows when hflag[i] (mapped
 // host memory, read over PCIe), else from ypair; k ascending either way
 __global__ __launch_bounds__(256) void combine_host_kernel(const float *ypair, const float *hrows, const uint8_t *hflag,
-                                                           int n_tok, int K, int H, float *out, int accumulate) {
+                                                           const float *yshared, int n_tok, int K, int H, float *out,
+                                                           int accumulate) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t h4 = (size_t)H / 4;
     if (i >= (size_t)n_tok * h4) return;
@@ -604,6 +611,10 @@ __global__ __launch_bounds__(256) void combine_host_kernel(const float *ypair, c
     if (accumulate) {
         const float4 p = *o;
         s.x = p.x + s.x; s.y = p.y + s.y; s.z = p.z + s.z; s.w = p.w + s.w;
+    }
+    if (yshared) {
+        const float4 v = ((const float4 *)yshared)[i];
+        s.x = s.x + v.x; s.y = s.y + v.y; s.z = s.z + v.z; s.w = s.w + v.w;
     }
     *o = s;
 }
@@ -632,12 +643,12 @@ hipError_t launch_quant_rows(const void *src, int bf16, int n_rows, int n, uint1
                     st, nullptr, nullptr, src, bf16, n_rows, n, q16, dx, bs16);
 }
 
-hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, uint16_t *q16, float *dx, uint16_t *bs16,
-                               hipStream_t st) {
+hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, int n_h, uint16_t *q16, float *dx,
+                               uint16_t *bs16, hipStream_t st) {
     const int64_t blocks = ((int64_t)P * (I / QK) + 3) / 4;
     if (blocks == 0) return hipSuccess;
-    return launch_b(swiglu_quant_kernel, dim3((unsigned)blocks), dim3(256), st, nullptr, nullptr, y2, P, I, h_out, q16,
-                    dx, bs16);
+    return launch_b(swiglu_quant_kernel, dim3((unsigned)blocks), dim3(256), st, nullptr, nullptr, y2, P, I, h_out, n_h,
+                    q16, dx, bs16);
 }
 
 // ---------------------------------------------------------------------------
@@ -851,6 +862,18 @@ __device__ inline Chunk chunk_find(const ChunkScan &s, int c, int lane) {
                  __builtin_amdgcn_readlane(np, src)};
 }
 
+// The task'th chunk: with a shared expert its chunks first (e = -1; rows
+// P .. P + n_tok - 1 of the activations and up/gate rows), then the routed ones.
+__device__ inline int shared_chunks(const GroupedArgs &a, int mt) {
+    return a.shared ? ((a.P / a.K + 31) / 32 + mt - 1) / mt : 0;
+}
+__device__ inline Chunk chunk_of(const GroupedArgs &a, const ChunkScan &scan, int c, int ns, int lane) {
+    if (c >= ns) return chunk_find(scan, c - ns, lane);
+    const int n = a.P / a.K, tiles = (n + 31) / 32;
+    const int t0 = c * tiles / ns, t1 = (c + 1) * tiles / ns;
+    return Chunk{scan.total, -1, a.P + 32 * t0, min(n, 32 * t1) - 32 * t0};
+}
+
 // 4 nibbles' worth of B: words of nibbles under masks -> (1024 + q) * sc - 1024 * sc,
 // high nibbles as (1024 + 16 q) * (sc / 16) - 64 * sc: one rounding of an exact integer
 __device__ inline half8_t q4_tile_b(uint32_t w0, uint32_t w1, uint32_t M, uint32_t X, _Float16 s, _Float16 nb) {
@@ -874,14 +897,15 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     // together
     const int nt_r = out_n / (TL_ROWS * rtw);
     const ChunkScan scan = chunk_scan(a.offsets, a.E, MT, lane);
-    const int total = scan.total * nt_r;
+    const int ns = shared_chunks(a, MT), total = (ns + scan.total) * nt_r;
     const int per = (total + 7) / 8, li = (int)blockIdx.x >> 3;
     const int task = ((int)blockIdx.x & 7) * per + li;
     if (li >= per || task >= total) return;
-    const Chunk ch = chunk_find(scan, task / nt_r, lane);
+    const Chunk ch = chunk_of(a, scan, task / nt_r, ns, lane);
+    const bool sh = ch.e < 0;
     const int r0 = (task % nt_r) * (TL_ROWS * rtw);
     const int np = ch.np, nt = (np + 31) / 32;
-    const uint8_t *base = grouped_expert(a, ch.e);
+    const uint8_t *base = sh ? a.shared : grouped_expert(a, ch.e);
     if (!base) {
         for (int rt = 0; rt < rtw; ++rt)
             for (int i = tid; i < np * TL_ROWS; i += 256) {
@@ -897,7 +921,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     // the activation rows; the rows past the chunk's pairs lie past the end and read as
     // zeros, which costs the products no traffic and little power (a full tile of
     // repeated rows slowed the whole of a 64-token batch by ~3 %)
-    const uint32_t n_rows = (uint32_t)(DOWN ? a.P : a.P / a.K);
+    const uint32_t n_tok = (uint32_t)(a.P / a.K), n_rows = DOWN ? a.P + (sh ? n_tok : 0u) : n_tok;
     const i32x4_t ra = raw_buffer(DOWN ? a.ha : a.xa, n_rows * (2 * K));
     const i32x4_t rbs = raw_buffer(DOWN ? a.hbs : a.xbs, n_rows * (K / 8));
 
@@ -933,7 +957,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     load_w(0, 0, true);
     for (int i = tid; i < GK; i += 256) {
         const int pos = ch.p0 + min(i, np - 1);
-        const int row = DOWN ? pos : a.perm[pos] / a.K;
+        const int row = DOWN ? pos : sh ? pos - a.P : a.perm[pos] / a.K;
         s_row[i] = i < np ? (uint32_t)row * (2 * K) : TL_NONE;
 #pragma unroll
         for (int b = 0; b < NB; ++b) s_dx[b][i] = adx[(size_t)row * NB + b];
@@ -941,9 +965,10 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
     // the pairs' output rows and gate weights, fetched beside the first activations
     auto pairs = [&]() {
         for (int i = tid; i < GK; i += 256) {
-            const int pr = a.perm[ch.p0 + min(i, np - 1)];
+            const int pos = ch.p0 + min(i, np - 1);
+            const int pr = sh ? pos - a.P : a.perm[pos];
             s_pp[i] = i < np ? (uint32_t)pr * (uint32_t)(4 * a.H) : TL_NONE;        // not stored
-            s_gw[i] = a.w[pr];
+            s_gw[i] = sh ? 1.0f : a.w[pr];
         }
     };
     __syncthreads();
@@ -964,7 +989,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
                 dma16(la + (hf * (GK / 4) + 8 * t + j) * TL_QUAD, (int)(o[t][j] + ao), ra, s * QK * 2 + 128 * hf);
         if (hf && wave < NT) dma16(lb, (int)(ob / 16 + 16 * (lane & 1)), rbs, s * 32);      // the group sums, for after the second half
     };
-    const i32x4_t ro = DOWN ? raw_buffer(a.ypair, (uint32_t)a.P * (uint32_t)(4 * a.H))
+    const i32x4_t ro = DOWN ? raw_buffer(sh ? a.yshared : a.ypair, (sh ? n_tok : (uint32_t)a.P) * (uint32_t)(4 * a.H))
                             : raw_buffer(a.y2 + (size_t)ch.p0 * out_n, (uint32_t)np * (uint32_t)(4 * out_n));
     const int n = lane & 31, h = lane >> 5;
     const uint32_t hm = 0u - (uint32_t)h;
@@ -1135,14 +1160,15 @@ __global__ __launch_bounds__(256, MT == 1 ? 3 : 2) void grouped_q6_tile_kernel(G
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nt_r = a.H / (TL_ROWS * rtw);
     const ChunkScan scan = chunk_scan(a.offsets, a.E, MT, lane);
-    const int total = scan.total * nt_r;
+    const int ns = shared_chunks(a, MT), total = (ns + scan.total) * nt_r;
     const int per = (total + 7) / 8, li = (int)blockIdx.x >> 3;
     const int task = ((int)blockIdx.x & 7) * per + li;
     if (li >= per || task >= total) return;
-    const Chunk ch = chunk_find(scan, task / nt_r, lane);
+    const Chunk ch = chunk_of(a, scan, task / nt_r, ns, lane);
+    const bool sh = ch.e < 0;
     const int r0 = (task % nt_r) * (TL_ROWS * rtw);
     const int np = ch.np, nt = (np + 31) / 32;
-    const uint8_t *base = grouped_expert(a, ch.e);
+    const uint8_t *base = sh ? a.shared : grouped_expert(a, ch.e);
     if (!base) {
         for (int rt = 0; rt < rtw; ++rt)
             for (int i = tid; i < np * TL_ROWS; i += 256)
@@ -1150,8 +1176,9 @@ __global__ __launch_bounds__(256, MT == 1 ? 3 : 2) void grouped_q6_tile_kernel(G
         return;
     }
     const i32x4_t rw = raw_buffer(base + 2ull * a.I * (a.H / QK) * Q4K_BYTES, (uint32_t)(a.H * ROWB));
-    const i32x4_t ra = raw_buffer(a.ha, (uint32_t)a.P * (2 * K));
-    const i32x4_t ro = raw_buffer(a.ypair, (uint32_t)a.P * (uint32_t)(4 * a.H));
+    const uint32_t n_out = (uint32_t)(sh ? a.P / a.K : a.P);
+    const i32x4_t ra = raw_buffer(a.ha, (uint32_t)(a.P + (sh ? a.P / a.K : 0)) * (2 * K));
+    const i32x4_t ro = raw_buffer(sh ? a.yshared : a.ypair, n_out * (uint32_t)(4 * a.H));
 
     __shared__ __attribute__((aligned(16))) uint8_t s_a[2][GK / 4][TL_QUAD];       // as in the Q4_K kernel
     __shared__ __attribute__((aligned(16))) uint8_t s_w[4][32 * TL_W6];
@@ -1183,9 +1210,10 @@ __global__ __launch_bounds__(256, MT == 1 ? 3 : 2) void grouped_q6_tile_kernel(G
     }
     auto pairs = [&]() {
         for (int i = tid; i < GK; i += 256) {
-            const int pr = a.perm[ch.p0 + min(i, np - 1)];
+            const int pos = ch.p0 + min(i, np - 1);
+            const int pr = sh ? pos - a.P : a.perm[pos];
             s_pp[i] = i < np ? (uint32_t)pr * (uint32_t)(4 * a.H) : TL_NONE;        // not stored
-            s_gw[i] = a.w[pr];
+            s_gw[i] = sh ? 1.0f : a.w[pr];
         }
     };
     __syncthreads();
@@ -1344,11 +1372,14 @@ __global__ __launch_bounds__(256, MT == 1 ? 3 : 2) void grouped_q6_tile_kernel(G
     else body(std::integral_constant<int, 1>{});
 }
 
+template <int MT>
+static int shared_chunks_max(const GroupedArgs &a) { return a.shared ? (a.P / a.K + 31) / 32 / MT + 1 : 0; }
+
 template <bool DOWN, int MT>
 static hipError_t launch_tile(const GroupedArgs &a, int rtw, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
     // chunks: at most P / (32 MT) full ones and one more per expert; the rest of the grid returns at once
-    const int64_t tasks = (int64_t)(a.P / (32 * MT) + a.E) * (rows / (TL_ROWS * rtw));
+    const int64_t tasks = (int64_t)(a.P / (32 * MT) + a.E + shared_chunks_max<MT>(a)) * (rows / (TL_ROWS * rtw));
     const dim3 grid((unsigned)((tasks + 7) / 8 * 8)), blk(256);
     if constexpr (!DOWN) return launch_b(grouped_q4_tile_kernel<8, false, MT>, grid, blk, st, e0, e1, a, rtw);
     else if (nb == 3) return launch_b(grouped_q4_tile_kernel<3, true, MT>, grid, blk, st, e0, e1, a, rtw);
@@ -1359,7 +1390,7 @@ static hipError_t launch_tile(const GroupedArgs &a, int rtw, hipStream_t st, hip
 // Which kernel a Q4_K product runs on.  `full` estimates the chunks of one tile
 // that the batch fills.
 //   few  fewer than 512 workgroups of 128 rows: the 64-row kernel has twice as many,
-//        while a pass of 16 pairs serves an expert (us: 64 experts, I = 256, up/gate of
+//        while a pass of 16 pairs serves an expert, or the one expert of 16 tokens (us: 64 experts, I = 256, up/gate of
 //        64 tokens 14.4 there, 17.6 on tiles; 128 tokens 19.9 / 17.7)
 //   wide at least 64 pairs per expert and 600 workgroups of three tiles: those (us,
 //        one tile / three: up/gate of 1,500 x 8 of 128 158 / 153, 3,000 289 / 253;
@@ -1371,7 +1402,7 @@ template <bool DOWN>
 static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
     const int rt = rows / TL_ROWS, full = max(a.P / 32, min(a.E, a.P));
-    if (full * rt < 512 && a.P <= 8 * a.E) {
+    if (full * rt < 512 && a.P <= 8 * a.E + 8 && !a.shared) {
         const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
         if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false>, grid, blk, st, e0, e1, a);
         else if (nb == 3) return launch_b(grouped_q4_kernel<3, true>, grid, blk, st, e0, e1, a);
@@ -1387,7 +1418,7 @@ static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0,
 template <int MT>
 static hipError_t launch_tile6(const GroupedArgs &a, int rtw, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int nb = a.I / QK;
-    const int64_t tasks = (int64_t)(a.P / (32 * MT) + a.E) * (a.H / (TL_ROWS * rtw));
+    const int64_t tasks = (int64_t)(a.P / (32 * MT) + a.E + shared_chunks_max<MT>(a)) * (a.H / (TL_ROWS * rtw));
     const dim3 grid((unsigned)((tasks + 7) / 8 * 8)), blk(256);
     if (nb == 3) return launch_b(grouped_q6_tile_kernel<3, MT>, grid, blk, st, e0, e1, a, rtw);
     if (nb == 2) return launch_b(grouped_q6_tile_kernel<2, MT>, grid, blk, st, e0, e1, a, rtw);
@@ -1403,7 +1434,7 @@ static hipError_t launch_tile6(const GroupedArgs &a, int rtw, hipStream_t st, hi
 // Two row tiles a workgroup, but one below two pairs per expert (us, one / two: 128
 // experts, 24 tokens 43 / 48, 1,000 tokens 111 / 104).
 static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    if (a.I == 512 && 2 * a.P > a.E && a.P <= 4 * a.E)
+    if (a.I == 512 && 2 * a.P > a.E && a.P <= 4 * a.E && !a.shared)
         return launch_b(grouped_q6_kernel<2>, dim3((unsigned)(a.H / 64 * a.E)), dim3(256), st, e0, e1, a);
     if (a.P >= 48 * a.E || (a.slot_pool && a.P > 16 * a.E)) return launch_tile6<2>(a, 2, st, e0, e1);
     return launch_tile6<1>(a, a.P < 2 * a.E ? 1 : 2, st, e0, e1);
@@ -1422,18 +1453,19 @@ hipError_t launch_iota(int n, int32_t *offsets, int32_t *perm, float *ones, hipS
                     ones);
 }
 
-hipError_t launch_combine(const float *ypair, int n_tok, int K, int H, float *out, int accumulate, hipStream_t st) {
+hipError_t launch_combine(const float *ypair, const float *yshared, int n_tok, int K, int H, float *out, int accumulate,
+                          hipStream_t st) {
     const size_t n4 = (size_t)n_tok * H / 4;
     if (n4 == 0) return hipSuccess;
-    return launch_b(combine_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), st, nullptr, nullptr, ypair, n_tok,
-                    K, H, out, accumulate);
+    return launch_b(combine_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), st, nullptr, nullptr, ypair, yshared,
+                    n_tok, K, H, out, accumulate);
 }
 
-hipError_t launch_combine_host(const float *ypair, const float *hrows, const uint8_t *hflag, int n_tok, int K, int H,
-                               float *out, int accumulate, hipStream_t st) {
+hipError_t launch_combine_host(const float *ypair, const float *hrows, const uint8_t *hflag, const float *yshared,
+                               int n_tok, int K, int H, float *out, int accumulate, hipStream_t st) {
     const size_t n4 = (size_t)n_tok * (H / 4);
     return launch_b(combine_host_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), st, nullptr, nullptr, ypair,
-                    hrows, hflag, n_tok, K, H, out, accumulate);
+                    hrows, hflag, yshared, n_tok, K, H, out, accumulate);
 }
 
 // ---------------------------------------------------------------------------

@@ -249,6 +249,8 @@ struct GroupedArgs {
     const uint16_t *hbs;        // [P][I/16]
     float *ypair;               // [P][H] weighted rows, pair (t*K + k) order
     const uint8_t *host_mask;   // [E] or null: experts the host computes (their rows read as zeros)
+    const uint8_t *shared;      // an always-on expert beside the routed ones in the same launches, or null: its
+    float *yshared;             // rows follow the P pairs' in y2, ha, hdx and hbs, its outputs are yshared [n_tok][H]
 };
 
 hipError_t launch_dispatch(const int32_t *ids, int P, int E, int32_t *counts, int32_t *offsets, int32_t *perm,
@@ -258,19 +260,21 @@ hipError_t launch_quant_rows(const void *src, int bf16, int n_rows, int n, uint1
                              bool mfma_order, hipStream_t st);
 hipError_t launch_gateup_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 hipError_t launch_down_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
-hipError_t launch_combine(const float *ypair, int n_tok, int K, int H, float *out, int accumulate, hipStream_t st);
+// yshared [n_tok][H] or null: added after the sum over k
+hipError_t launch_combine(const float *ypair, const float *yshared, int n_tok, int K, int H, float *out, int accumulate,
+                          hipStream_t st);
 // the same sum with the rows of pairs flagged in hflag [n_tok*K] taken from hrows [n_tok*K][H]
 // (the host's, in mapped memory) instead of ypair
-hipError_t launch_combine_host(const float *ypair, const float *hrows, const uint8_t *hflag, int n_tok, int K, int H,
-                               float *out, int accumulate, hipStream_t st);
+hipError_t launch_combine_host(const float *ypair, const float *hrows, const uint8_t *hflag, const float *yshared,
+                               int n_tok, int K, int H, float *out, int accumulate, hipStream_t st);
 hipError_t launch_iota(int n, int32_t *offsets, int32_t *perm, float *ones, hipStream_t st);
 // the allocation-free grouped entry point's workspace: this device's address
 // of a static device array of STATIC_SCRATCH_BYTES
 constexpr size_t STATIC_SCRATCH_BYTES = 16ull << 20;
 hipError_t static_scratch(void **ptr);
-// h = silu(gate) * up from y2 and its Q8_K (h itself to h_out when not null)
-hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, uint16_t *q16, float *dx, uint16_t *bs16,
-                               hipStream_t st);
+// h = silu(gate) * up from y2 and its Q8_K (h itself of the first n_h rows to h_out when not null)
+hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, int n_h, uint16_t *q16, float *dx,
+                               uint16_t *bs16, hipStream_t st);
 
 // ev (optional): [logits start, logits end, select start, select end]
 hipError_t launch_route(const RouteLaunch &l, hipStream_t st, hipEvent_t *ev = nullptr);

@@ -1313,11 +1313,13 @@ int check_weight_ptrs(const char *who, const void *a, const void *b) {
 
 // workspace of the batched expert path, offsets in bytes
 struct GroupedWs {
-    size_t xa, xdx, xbs, h, ha, hdx, hbs, ypair, sh_offs, sh_perm, sh_ones, total;
+    size_t xa, xdx, xbs, h, ha, hdx, hbs, ypair, yshared, sh_offs, sh_perm, sh_ones, total;
 };
 
-GroupedWs grouped_ws(int n_tok, int K, int H, int I) {
-    const size_t T = (size_t)n_tok, P = (size_t)n_tok * K;
+// shared: with room for a shared expert's rows beside the pairs' (moe_decode_batch's own
+// workspace); without, a shared expert reuses the pairs' after them
+GroupedWs grouped_ws(int n_tok, int K, int H, int I, bool shared = false) {
+    const size_t T = (size_t)n_tok, P0 = (size_t)n_tok * K, P = P0 + (shared ? T : 0);
     GroupedWs w{};
     size_t o = 0;
     w.xa = o;    o += align_up(T * H * 2, 256);
@@ -1327,7 +1329,8 @@ GroupedWs grouped_ws(int n_tok, int K, int H, int I) {
     w.ha = o;    o += align_up(P * I * 2, 256);
     w.hdx = o;   o += align_up(P * (I / 256) * 4, 256);
     w.hbs = o;   o += align_up(P * (I / 16) * 2, 256);
-    w.ypair = o; o += align_up(P * H * 4, 256);
+    w.ypair = o; o += align_up(P0 * H * 4, 256);
+    w.yshared = o; o += shared ? align_up(T * H * 4, 256) : 0;
     w.sh_offs = o; o += 256;                              // shared expert: trivial dispatch
     w.sh_perm = o; o += align_up(T * 4, 256);
     w.sh_ones = o; o += align_up(T * 4, 256);
@@ -3528,7 +3531,7 @@ int moe_combine(const float *pair_rows, int n_tok, int K, int H, float *out, int
     if (!pair_rows || !out) return fail(MOE_ERR_ARG, "moe_combine: null argument");
     if (n_tok < 0 || K < 1 || H <= 0 || H % 4) return fail(MOE_ERR_ARG, "moe_combine: bad shape");
     if (((uintptr_t)pair_rows | (uintptr_t)out) % 16) return fail(MOE_ERR_ARG, "moe_combine: 16-byte alignment");
-    HIPCHK(mp::launch_combine(pair_rows, n_tok, K, H, out, accumulate, (hipStream_t)stream));
+    HIPCHK(mp::launch_combine(pair_rows, nullptr, n_tok, K, H, out, accumulate, (hipStream_t)stream));
     return MOE_OK;
 }
 
@@ -3566,10 +3569,14 @@ static int grouped_check(const moe_grouped_desc *d) {
 // once the host's rows are written, the combine taking flagged pairs' rows
 // from hrows (hflag [P]) and the shared expert.
 constexpr int GR_EXPERTS = 1, GR_COMBINE = 2;
+// beside: ws has room for the shared expert's rows, so it runs in the routed experts'
+// launches and the combine adds its row (batch 16, 256 experts, I = 512: ~27 us a layer in
+// launches of its own, which leave the GPU nearly idle).
 static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, int parts = GR_EXPERTS | GR_COMBINE,
                        const uint8_t *host_mask = nullptr, const float *hrows = nullptr,
-                       const uint8_t *hflag = nullptr) {
-    const GroupedWs w = grouped_ws(d->n_tok, d->K, d->H, d->I);
+                       const uint8_t *hflag = nullptr, bool beside = false) {
+    const GroupedWs w = grouped_ws(d->n_tok, d->K, d->H, d->I, beside);
+    beside = beside && d->shared;
     mp::GroupedArgs a{};
     a.offsets = d->offsets; a.perm = d->perm; a.w = d->w;
     a.table = d->table; a.slot_pool = d->slot_pool; a.slot_bytes = d->slot_bytes; a.n_slots = d->n_slots;
@@ -3582,6 +3589,10 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
     a.host_mask = host_mask;
     const int P = d->n_tok * d->K;
     a.P = P;
+    if (beside) {
+        a.shared = d->shared;
+        a.yshared = (float *)(ws + w.yshared);
+    }
     hipEvent_t ev[4] = {};
     const bool timed = d->kernel_ms != nullptr;
     if (timed)
@@ -3591,16 +3602,17 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
             HIPCHK(mp::launch_quant_rows(d->x, d->x_type == MOE_DTYPE_BF16, d->n_tok, d->H, (uint16_t *)a.xa,
                                          (float *)a.xdx, (uint16_t *)a.xbs, true, st));
             HIPCHK(mp::launch_gateup_grouped(a, st, ev[0], ev[1]));
-            HIPCHK(mp::launch_swiglu_quant(a.y2, P, d->I, d->h_out, (uint16_t *)a.ha, (float *)a.hdx,
-                                           (uint16_t *)a.hbs, st));
+            HIPCHK(mp::launch_swiglu_quant(a.y2, P + (beside ? d->n_tok : 0), d->I, d->h_out, P, (uint16_t *)a.ha,
+                                           (float *)a.hdx, (uint16_t *)a.hbs, st));
             HIPCHK(mp::launch_down_grouped(a, st, ev[2], ev[3]));
         }
         if (!(parts & GR_COMBINE)) return MOE_OK;
         if (hflag)
-            HIPCHK(mp::launch_combine_host(a.ypair, hrows, hflag, d->n_tok, d->K, d->H, d->out, d->accumulate, st));
+            HIPCHK(mp::launch_combine_host(a.ypair, hrows, hflag, a.yshared, d->n_tok, d->K, d->H, d->out,
+                                           d->accumulate, st));
         else
-            HIPCHK(mp::launch_combine(a.ypair, d->n_tok, d->K, d->H, d->out, d->accumulate, st));
-        if (d->shared) {
+            HIPCHK(mp::launch_combine(a.ypair, a.yshared, d->n_tok, d->K, d->H, d->out, d->accumulate, st));
+        if (d->shared && !beside) {
             // the shared expert as a one-expert dispatch of every token, added after the routed sum
             mp::GroupedArgs sa = a;
             sa.host_mask = nullptr;
@@ -3611,10 +3623,10 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
             sa.store = d->shared; sa.n_store = 1; sa.E = 1; sa.K = 1; sa.P = d->n_tok;
             HIPCHK(mp::launch_iota(d->n_tok, (int32_t *)sa.offsets, (int32_t *)sa.perm, (float *)sa.w, st));
             HIPCHK(mp::launch_gateup_grouped(sa, st, nullptr, nullptr));
-            HIPCHK(mp::launch_swiglu_quant(sa.y2, d->n_tok, d->I, nullptr, (uint16_t *)sa.ha, (float *)sa.hdx,
+            HIPCHK(mp::launch_swiglu_quant(sa.y2, d->n_tok, d->I, nullptr, 0, (uint16_t *)sa.ha, (float *)sa.hdx,
                                            (uint16_t *)sa.hbs, st));
             HIPCHK(mp::launch_down_grouped(sa, st, nullptr, nullptr));
-            HIPCHK(mp::launch_combine(sa.ypair, d->n_tok, 1, d->H, d->out, 1, st));
+            HIPCHK(mp::launch_combine(sa.ypair, nullptr, d->n_tok, 1, d->H, d->out, 1, st));
         }
         return MOE_OK;
     };
@@ -3668,7 +3680,7 @@ static int batch_buffers(moe_cache *c, int n_tok) {
     c->b_route_ws = c->b_ws = nullptr;
     c->b_cap = 0;
     const size_t NL = c->L.size(), TK = (size_t)n_tok * c->K;
-    const size_t rws = route_ws_bytes(c->E, n_tok), gws = grouped_ws(n_tok, c->K, c->H, c->I).total;
+    const size_t rws = route_ws_bytes(c->E, n_tok), gws = grouped_ws(n_tok, c->K, c->H, c->I, true).total;
     bool ok = hipMalloc(&c->b_ids, NL * TK * 4) == hipSuccess && hipMalloc(&c->b_slots, TK * 4) == hipSuccess &&
               hipMalloc(&c->b_w, TK * 4) == hipSuccess && hipMalloc(&c->b_counts, (size_t)c->E * 4) == hipSuccess &&
               hipMalloc(&c->b_offs, ((size_t)c->E + 1) * 4) == hipSuccess && hipMalloc(&c->b_perm, TK * 4) == hipSuccess &&
@@ -3764,7 +3776,7 @@ static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped
         yp[(size_t)j] = c->bs_y.data() + (size_t)j * c->H;
     }
     std::atomic_thread_fence(std::memory_order_release);
-    int r = grouped_run(gd, (uint8_t *)c->b_ws, st, GR_EXPERTS, c->bs_mask_d + (size_t)par * c->E);
+    int r = grouped_run(gd, (uint8_t *)c->b_ws, st, GR_EXPERTS, c->bs_mask_d + (size_t)par * c->E, nullptr, nullptr, true);
     if (r != MOE_OK) return r;
     if (n) {
         c->sc_computing.store(l, std::memory_order_relaxed);
@@ -3782,7 +3794,7 @@ static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped
     c->sc_cpu_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t1).count();
     std::atomic_thread_fence(std::memory_order_release);
     return grouped_run(gd, (uint8_t *)c->b_ws, st, GR_COMBINE, nullptr, c->bs_rows_d + (size_t)par * TK * c->H,
-                       c->bs_flag_d + (size_t)par * TK);
+                       c->bs_flag_d + (size_t)par * TK, true);
 }
 
 int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out, int n_tok, int32_t *ids_host,
@@ -3790,6 +3802,7 @@ int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out
     if (!c || !x || !out) return fail(MOE_ERR_ARG, "bad arguments");
     if (c->host_only) return fail(MOE_ERR_STATE, "host-only cache (device < 0) cannot decode");
     if (n_tok < 1 || n_tok > 4096) return fail(MOE_ERR_ARG, "n_tok %d out of range 1..4096", n_tok);
+    if ((int64_t)n_tok * c->K > 65535) return fail(MOE_ERR_ARG, "n_tok %d x K %d out of range", n_tok, c->K);
     if (((uintptr_t)x | (uintptr_t)out) % 16) return fail(MOE_ERR_ARG, "x and out must be 16-byte aligned");
     HIPCHK(hipSetDevice(c->cfg.device));
     int r = batch_buffers(c, n_tok);
@@ -3843,10 +3856,12 @@ int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out
         gd.out = out + (size_t)l * n_tok * c->H; gd.accumulate = 0;
         gd.workspace = c->b_ws; gd.shared = ls.shared;
         gd.kernel_ms = c->timing ? gms : nullptr;
+        if ((r = grouped_check(&gd)) != MOE_OK) return r;
         if (!sc) {
-            if ((r = moe_grouped_experts(&gd, stream)) != MOE_OK) return r;
+            if ((r = grouped_run(&gd, (uint8_t *)c->b_ws, st, GR_EXPERTS | GR_COMBINE, nullptr, nullptr, nullptr, true)) !=
+                MOE_OK)
+                return r;
         } else {
-            if ((r = grouped_check(&gd)) != MOE_OK) return r;
             if (!ls.store_host) return fail(MOE_ERR_STATE, "layer %d: CPU-assisted serving needs the host store", l);
             if ((r = batch_sidecar_layer(c, l, n_tok, &gd, st)) != MOE_OK) return r;
         }

@@ -193,6 +193,28 @@ def test_decode_256_experts_shared_expert(tmp_path):
         rig.close()
 
 
+# the shared expert's rows beside the routed pairs: one to five tiles of 32 tokens, ragged, in chunks of
+# one tile and (E = 64, over 16 pairs per expert) of up to three; Q4_K and Q6_K down
+@pytest.mark.parametrize("E,I,B", [(256, 512, 1), (256, 512, 33), (128, 768, 97), (64, 256, 65), (64, 256, 150)])
+def test_decode_batch_shared_expert_tiles(E, I, B):
+    rig = Rig([E - 8, E // 2], [Q4, Q6], T=B, I=I, E=E, shared=True, zipf_s=1.0, admit="window", batch_tables=True)
+    oc = rig.oracle_cache()
+    try:
+        out = torch.empty((rig.nl, B, 2048), dtype=torch.float32, device=rig.dev)
+        xb = rig.x[:B].transpose(0, 1).contiguous()
+        bb = None if rig.bias is None else rig.bias[:B].transpose(0, 1).contiguous()
+        ids = rig.cache.decode_batch(xb, out, bias=bb, stream=torch.cuda.current_stream().cuda_stream)
+        got = out.cpu().numpy()
+        for l in range(rig.nl):
+            tbl, _ = oc.table(l)
+            for t in range(B):
+                rids, rw, _, _ = O.route(rig.Wh[l], rig.xh[t, l], 8, bias=None if rig.bh is None else rig.bh[t, l], table=tbl)
+                assert np.array_equal(ids[l, t], rids), (l, t)
+                assert np.array_equal(got[l, t], rig.oracle_layer(t, l, rids, rw)), (l, t)
+    finally:
+        rig.close()
+
+
 @pytest.mark.parametrize("shape", ["e256_shared_i512", "e128_i768", "e128_unsteered_prior", "e256_shared_i512_cpu",
                                    "e128_i768_cpu_2of3", "e128_i768_cpu_1of2_b5", "e128_i768_cpu_0of1",
                                    "e128_i768_cpu_1of1_b80_timed"])
