@@ -482,12 +482,15 @@ int moe_cache_set_timing(moe_cache *c, int on);
  * 3 router GEMV, selection, gate/up and down as four launches; 1 resident and
  * absent experts as separate launches on two streams, forked and joined per
  * layer; 2 the same launches one after the other on one stream.
+ * Without CPU-assisted serving the fused layers of a token, whose inputs are
+ * all given, share launches (one for up to 56 layers), except where, launched
+ * directly, out overlaps x or bias: then they run one by one, in order.
  * graph: 1 (default) replay each token's launches as one captured HIP graph,
- * except that a token of at most 8 layers without CPU-assisted serving or
- * streaming launches its layers directly: a graph launch costs ~30 us of
- * latency against ~11 us for a kernel launch (ROCm 7, MI355X), and direct
- * launches need no copies of x, out or the sequence number; 2 always the
- * graph; 0 always direct launches.  Timing mode launches directly.  Every
+ * except that a token whose layers share launches, or of at most 8 layers
+ * without CPU-assisted serving or streaming, launches directly: a graph launch
+ * costs ~30 us of latency against ~11 us for a kernel launch (ROCm 7, MI355X),
+ * and direct launches need no copies of x, out or the sequence number; 2 always
+ * the graph; 0 always direct launches.  Timing mode launches directly.  Every
  * path gives the same bits.  MOE_ERR_ARG for split outside 0..3 or graph
  * outside 0..2. */
 int moe_cache_set_decode_path(moe_cache *c, int split, int graph);

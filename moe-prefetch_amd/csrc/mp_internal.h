@@ -212,11 +212,31 @@ struct FusedArgs {
     // workgroup writes the layer's words after every combine workgroup has
     // written its output rows (through to memory), and with pub_done the late
     // word: when every word carries the token's number its outputs are complete.
+    // After a wait of this token ran out nothing more is published.
     uint64_t *pub;
     uint64_t *pub_ctr;        // (seq << 32) | the layer's combine workgroups finished
     int pub_layer, pub_L;
     int pub_done;
 };
+// Up to FUSED_MULTI layers of one token in one launch (kernel arguments: at most 4 KiB), GPU only
+// (no post, x.ypart null).  c: the first layer's arguments; layer i's buffers lie i strides
+// further ([L][H] x and out, [L][E] bias, prior and table, [L][K] ids, w and slots, [L][K] staging
+// experts, `words` exchange words, one pub_ctr), and l[i] holds what differs.  kt: the most
+// experts of a layer, the shared one counted.
+struct FusedLayer {
+    const float *W;
+    const uint8_t *slot_pool, *store, *shared;
+    uint64_t slot_bytes, expert_bytes;
+    int n_slots, down_type;
+};
+constexpr int FUSED_MULTI = 56;
+struct FusedMulti {
+    int n, kt;
+    uint64_t words;
+    FusedArgs c;
+    FusedLayer l[FUSED_MULTI];
+};
+static_assert(sizeof(FusedMulti) <= 4096, "kernel arguments");
 // exchange words per layer of the fused decode
 inline size_t fused_words(int K, int I, int H) {
     return (size_t)FUSED_LOG_COPIES * 256 + (size_t)FUSED_COPIES * FUSED_REC + (size_t)(K + 1) * I +
@@ -282,6 +302,7 @@ hipError_t launch_experts(const ExpertArgs &a, hipStream_t st);
 hipError_t launch_join(const JoinArgs &a, hipStream_t st);
 // the fused layer (see FusedArgs); its down rows are of down_type
 hipError_t launch_fused(const FusedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
+hipError_t launch_fused_multi(const FusedMulti &m, hipStream_t st);
 // src: 0 every routed expert, 1 only those resident in HBM slots, 2 only
 // those read from the pinned host store.  A src = 2 down launch accumulates
 // into out when the caller sets accumulate.

@@ -1458,6 +1458,10 @@ __device__ void fused_publish(const FusedArgs &a, uint32_t seq, const uint64_t *
                                                    __HIP_MEMORY_SCOPE_AGENT));
     if ((uint32_t)nv != (uint32_t)n_comb) return;
     const int K = a.x.K;
+    // a workgroup of this token gave up: nothing is published, so the host, which wants every
+    // layer's words, copies back and synchronises and sees it (a layer beside this one may
+    // already have published the late word)
+    if (__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == seq) return;
     for (int k = 0; k < K; ++k)
         __hip_atomic_store(a.pub + (size_t)a.pub_layer * K + k, s_rec[k], __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1504,6 +1508,74 @@ __global__ __launch_bounds__(256) void fused_kernel(FusedArgs a) {
         fused_down<DT>(a, g, seq, smem);
     } else {
         fused_combine(a, g - nD, seq, smem);
+    }
+}
+
+// Several layers of one token, whose inputs are all given, in one launch.  A
+// layer alone is a chain of hand-overs (router, selection, gate/up, down,
+// combine) that leaves the memory idle most of its ~15 us; here the workgroups
+// of group k are the router rows of layer k + 1, the selection and gate/up rows
+// of layer k and the down rows and combine of layer k - 1 (the router rows of
+// layer 0 before them all), so a workgroup's inputs are mostly there when it
+// starts and the next layer's bytes move meanwhile.  Every wait is still for
+// workgroups of a lower index.
+__device__ inline FusedArgs fused_layer(const FusedMulti &m, int l) {
+    FusedArgs a = m.c;
+    const FusedLayer &p = m.l[l];
+    const size_t sH = (size_t)l * a.r.H, sE = (size_t)l * a.r.E, sK = (size_t)l * a.r.K, sx = (size_t)l * m.words;
+    a.r.W = p.W;
+    a.r.x += sH;
+    if (a.r.bias) a.r.bias += sE;
+    if (a.r.prior) a.r.prior += sE;
+    a.r.table += sE;
+    a.r.dummy = p.n_slots;
+    a.r.ids += sK; a.r.w += sK; a.r.slots += sK;
+    a.x.ids += sK; a.x.w += sK; a.x.slots += sK;
+    a.x.slot_pool = p.slot_pool; a.x.slot_bytes = p.slot_bytes; a.x.n_slots = p.n_slots;
+    a.x.host_store = p.store; a.x.expert_bytes = p.expert_bytes;
+    a.x.down_type = p.down_type;
+    a.x.shared = p.shared; a.x.n_shared = p.shared ? 1 : 0;
+    a.x.out += sH;
+    if (a.x.stage) a.x.stage += sK * a.x.stage_stride;
+    a.xlog += sx; a.rec += sx; a.hx += sx; a.yx += sx;
+    if (a.pub) {
+        a.pub_ctr += l;
+        a.pub_layer += l;
+        a.pub_done = a.pub_layer + 1 == a.pub_L;
+    }
+    return a;
+}
+__global__ __launch_bounds__(256) void fused_multi_kernel(FusedMulti m) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[FUSED_LDS];
+    const int E = m.c.r.E, H = m.c.x.H;
+    const int nG = m.kt * (m.c.x.I / FUSED_GU_TILE), nD = m.kt * (H / FUSED_DN_TILE), nC = H / 256;
+    const int size = E + 1 + nG + nD + nC;
+    int l = 0, g = (int)blockIdx.x, role = 0;           // router, selection, gate/up, down, combine
+    if (g >= E) {
+        const int k = (g - E) / size;
+        g -= E + k * size;
+        l = k;
+        if (g < E) l = k + 1;
+        else if (g == E) role = 1;
+        else if ((g -= E + 1) < nG) role = 2;
+        else {
+            g -= nG;
+            l = k - 1;
+            role = g < nD ? 3 : 4;
+            if (role == 4) g -= nD;
+        }
+    }
+    if (l < 0 || l >= m.n) return;
+    const FusedArgs a = fused_layer(m, l);
+    const uint32_t seq = a.r.seq ? *a.r.seq : a.r.seq_val;
+    const int kt = a.x.K + a.x.n_shared;
+    if (role == 0) fused_router(a, g, seq, smem);
+    else if (role == 1) fused_select(a, seq, smem);
+    else if (role == 2) { if (g < kt * (a.x.I / FUSED_GU_TILE)) fused_gateup(a, g, seq, smem); }
+    else if (role == 4) fused_combine(a, g, seq, smem);
+    else if (g < kt * (H / FUSED_DN_TILE)) {
+        if (a.x.down_type == TYPE_Q6K) fused_down<TYPE_Q6K>(a, g, seq, smem);
+        else fused_down<TYPE_Q4K>(a, g, seq, smem);
     }
 }
 
@@ -1742,6 +1814,12 @@ hipError_t launch_fused(const FusedArgs &a, hipStream_t st, hipEvent_t e0, hipEv
                                   kt * (a.x.H / FUSED_DN_TILE) + (a.x.ypart ? 0 : a.x.H / 256));
     if (a.x.down_type == TYPE_Q6K) return launch(fused_kernel<TYPE_Q6K>, dim3(n), dim3(256), st, e0, e1, a);
     return launch(fused_kernel<TYPE_Q4K>, dim3(n), dim3(256), st, e0, e1, a);
+}
+
+hipError_t launch_fused_multi(const FusedMulti &m, hipStream_t st) {
+    const FusedArgs &a = m.c;
+    const unsigned size = (unsigned)(a.r.E + 1 + m.kt * (a.x.I / FUSED_GU_TILE) + m.kt * (a.x.H / FUSED_DN_TILE) + a.x.H / 256);
+    return launch(fused_multi_kernel, dim3((unsigned)a.r.E + (unsigned)(m.n + 1) * size), dim3(256), st, nullptr, nullptr, m);
 }
 
 hipError_t launch_experts(const ExpertArgs &a, hipStream_t st) {

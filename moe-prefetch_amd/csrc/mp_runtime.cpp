@@ -2874,12 +2874,22 @@ int moe_cache_sync(moe_cache *c) {
     return MOE_OK;
 }
 
+// the collected layers of a token in one launch
+static int send_layers(mp::FusedMulti *m, hipStream_t st) {
+    if (m->n == 1) HIPCHK(mp::launch_fused(m->c, st, nullptr, nullptr));
+    else if (m->n > 1) HIPCHK(mp::launch_fused_multi(*m, st));
+    m->n = m->kt = 0;
+    return MOE_OK;
+}
+
 // fused: split is 0 and streaming is off; the router, selection, experts and
 // combine run as one launch.  seq_val: 0, the token's sequence number is in
-// d_seq (moe_decode_token); else the call's own number, passed by value
+// d_seq (moe_decode_token); else the call's own number, passed by value.
+// multi (fused, no sidecar): the layer joins those of the next launch, which
+// goes out when it is full (the caller sends the last one)
 static int decode_layer_impl(moe_cache *c, int layer, const float *x, const float *bias, float *out,
                              int32_t *ids_dev, float *w_dev, hipStream_t st, hipEvent_t *ev, bool stage,
-                             bool sidecar, bool fused, uint32_t seq_val) {
+                             bool sidecar, bool fused, uint32_t seq_val, mp::FusedMulti *multi = nullptr) {
     if (!c || !x || !out || layer < 0 || layer >= (int)c->L.size()) return fail(MOE_ERR_ARG, "bad arguments");
     if (c->host_only) return fail(MOE_ERR_STATE, "host-only cache (device < 0) cannot decode");
     const Layer &ls = c->L[layer];
@@ -2981,6 +2991,14 @@ static int decode_layer_impl(moe_cache *c, int layer, const float *x, const floa
             f.pub_layer = layer;
             f.pub_L = (int)c->L.size();
             f.pub_done = layer + 1 == (int)c->L.size();
+        }
+        if (multi) {
+            if (multi->n == 0) multi->c = f;
+            multi->words = c->fx_words;
+            multi->l[multi->n++] = {ls.router, ls.pool, ls.store_dev, ls.shared, ls.slot_bytes, ls.expert_bytes, ls.S,
+                                    ls.down_type};
+            multi->kt = std::max(multi->kt, c->K + f.x.n_shared);
+            return multi->n < mp::FUSED_MULTI ? MOE_OK : send_layers(multi, st);
         }
         HIPCHK(mp::launch_fused(f, st, E_(0), E_(1)));
     } else {
@@ -3271,7 +3289,7 @@ int moe_decode_layer(moe_cache *c, int layer, const float *x, const float *bias,
     return MOE_OK;
 }
 
-// tokens of at most this many layers launch directly in graph mode (see below)
+// tokens of at most this many layers, launched one by one, launch directly in graph mode (see below)
 constexpr int DIRECT_MAX_LAYERS = 8;
 
 // every word the fused launches publish (h_pub) carries this token's number:
@@ -3330,21 +3348,31 @@ int moe_decode_token(moe_cache *c, const float *x, const float *bias, float *out
     // reads h_seq when the stream reaches it; the previous token synchronised
     // the stream before returning, so no copy of an older number is pending.
     const uint32_t seq = next_seq(c);
+    const bool fused = c->split == 0 && !stm;
+    // The layers' inputs are all given, so the fused layers share launches (at
+    // most FUSED_MULTI a launch; us a token, one by one / together: 4 layers 84 / 47,
+    // 12 layers 212 / 106, 48 layers 789 / 388; a graph of the 48 as four branches
+    // 516, as launches of 7 layers 409).  Not with CPU-assisted serving (the
+    // host serves them in order) nor in timing mode, and launched directly only
+    // where no output lies in a layer's input (one by one, a later layer reads
+    // it; the graph copies the inputs first).
+    const size_t xb = (size_t)NL * c->H, bb = (size_t)NL * c->E;
+    const bool apart = (out + xb <= x || x + xb <= out) && (!bias || out + xb <= bias || bias + bb <= out);
+    const bool together = fused && !sc && !c->timing;
     // A captured graph's launch costs ~30 us of latency here (ROCm 7 on
-    // MI355X) against ~11 us for a kernel launch, and launching ~15 us layers
-    // one by one measured faster at every layer count (1 layer: 26 against
-    // 35 us a step; 48 layers within 1 %).  The graph frees the host sooner,
+    // MI355X) against ~11 us for a kernel launch.  The graph frees the host sooner,
     // which CPU-assisted serving and streaming need (the host serves a layer
     // while the GPU runs the next), and it costs less host time for many
-    // layers.  So a token of at most DIRECT_MAX_LAYERS layers without them
-    // launches its layers directly, with the sequence number by value and the
-    // caller's x and out: no copies.  (graph 2 keeps the graph for any token.)
-    const bool use_graph = c->graph && !c->timing && (c->graph == 2 || NL > DIRECT_MAX_LAYERS || sc || stm);
+    // launches.  So a token whose layers share a launch, or of at most
+    // DIRECT_MAX_LAYERS layers without serving or streaming, launches directly,
+    // with the sequence number by value and the caller's x and out: no copies.
+    // (graph 2 keeps the graph for any token.)
+    const bool use_graph = c->graph && !c->timing &&
+                           (c->graph == 2 || (NL > DIRECT_MAX_LAYERS && !(together && apart)) || sc || stm);
     if (use_graph) {
         *c->h_seq = seq;
         HIPCHK(hipMemcpyAsync(c->d_seq, c->h_seq, 4, hipMemcpyHostToDevice, st));
     }
-    const bool fused = c->split == 0 && !stm;
     // An earlier token that failed may have left SC_ABORT in the answers; a
     // join of this token must wait for this token's answer, not end on that.
     // Nothing of this token runs yet, so plain stores suffice.
@@ -3391,12 +3419,15 @@ int moe_decode_token(moe_cache *c, const float *x, const float *bias, float *out
     c->pub_on = publish;
     // per-kernel HIP-event timing needs eager launches: hipEventElapsedTime
     // does not accept events recorded as nodes of a graph
+    mp::FusedMulti many{};
+    mp::FusedMulti *multi = together && (use_graph || apart) ? &many : nullptr;
     if (!use_graph) {
         for (int l = 0; l < NL; ++l) {
-            const int r = decode_layer_impl(c, l, x + (size_t)l * c->H, bias ? bias + (size_t)l * c->E : nullptr,
+            int r = decode_layer_impl(c, l, x + (size_t)l * c->H, bias ? bias + (size_t)l * c->E : nullptr,
                                             out + (size_t)l * c->H, nullptr, nullptr, st,
                                             c->timing ? c->tev.data() + (size_t)l * 12 : nullptr, stage, sc, fused,
-                                            seq);
+                                            seq, multi);
+            if (r == MOE_OK && multi && l + 1 == NL) r = send_layers(multi, st);
             if (r != MOE_OK) {
                 c->pub_on = false;
                 abort_joins();
@@ -3417,7 +3448,8 @@ int moe_decode_token(moe_cache *c, const float *x, const float *bias, float *out
             for (int l = 0; l < NL && r == MOE_OK; ++l)
                 r = decode_layer_impl(c, l, c->x_buf + (size_t)l * c->H, key ? c->bias_buf + (size_t)l * c->E : nullptr,
                                       c->out_buf + (size_t)l * c->H, nullptr, nullptr, c->cap_stream, nullptr, stage,
-                                      sc, fused, 0);
+                                      sc, fused, 0, multi);
+            if (r == MOE_OK && multi) r = send_layers(multi, c->cap_stream);
 
             hipGraph_t g = nullptr;
             const hipError_t ec = hipStreamEndCapture(c->cap_stream, &g);

@@ -13,8 +13,8 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_rig import L, Rig, stream
-from moe_prefetch import ExpertCache, _lib
+from gpu_rig import L, Pinned, Rig, stream, synth_experts_dev
+from moe_prefetch import ExpertCache, MoeCache, _lib
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -191,6 +191,103 @@ def test_decode_256_experts_shared_expert(tmp_path):
         print("worst rel-L2", worst)
     finally:
         rig.close()
+
+
+def _token_cache(NL, E, I, n_slots, shared_layers=(), K=8):
+    """A cache of NL layers over one pinned store (Q6_K down in odd layers, a shared expert in the
+    layers named), the first n_slots experts of each layer in slots; and layer-sized buffers."""
+    dev = torch.device("cuda:0")
+    types = [Q6 if l % 2 else Q4 for l in range(NL)]
+    held = {}
+    for dt in set(types):
+        eb = L().moe_expert_bytes(2048, I, dt)
+        held[dt] = Pinned(E * eb)
+        synth_experts_dev(7, 0, 0, E, I, dt, held[dt].dev, eb)
+    torch.cuda.synchronize()
+    c = MoeCache(NL, n_experts=E, n_expert_used=K, intermediate=I, n_slots=n_slots, max_inserts=n_slots, down_types=types,
+                 batch_tables=True, device=0)
+    g = torch.Generator(device=dev)
+    g.manual_seed(NL)
+    keep = []
+    for l in range(NL):
+        eb = L().moe_expert_bytes(2048, I, types[l])
+        W = torch.randn((E, 2048), device=dev, generator=g) * 0.02
+        c.set_host_store(l, held[types[l]].ptr)
+        c.set_router(l, W)
+        if l in shared_layers:
+            sh = torch.empty(eb, dtype=torch.uint8, device=dev)
+            synth_experts_dev(9, l, 0, 1, I, types[l], sh.data_ptr(), eb)
+            c.set_shared(l, sh)
+            keep.append(sh)
+        keep.append(W)
+        c.observe(l, np.arange(n_slots, dtype=np.int32), n_tok=n_slots)
+    c.step()
+    c.sync()
+    c.step()
+    c.freeze()
+    x = torch.randn((NL, 2048), device=dev, generator=g)
+    torch.cuda.synchronize()
+    return c, held, keep, x
+
+
+# a token's layers share launches: two layers, a full launch, one layer more (a launch of its own), two more;
+# some layers with a shared expert, absent experts read from the store; a graph of the same launches
+@pytest.mark.parametrize("NL,graph", [(2, 1), (7, 1), (9, 1), (56, 1), (57, 1), (58, 1), (9, 2), (58, 2), (9, 0)])
+def test_token_layers_together(NL, graph):
+    E, I, K = 64, 256, 8
+    c, held, keep, x = _token_cache(NL, E, I, 60, shared_layers=(0, 3, NL - 1))
+    st = torch.cuda.current_stream().cuda_stream
+    try:
+        want = torch.empty((NL, 2048), device=x.device)
+        wid = torch.empty((NL, K), dtype=torch.int32, device=x.device)
+        for l in range(NL):
+            c.decode_layer(l, x[l], want[l], ids=wid[l], stream=st)
+        torch.cuda.synchronize()
+        wid = wid.cpu().numpy()
+        for l in range(NL):
+            c.observe(l, wid[l])
+        c.step()
+        c.set_decode_path(0, graph)
+        for rep in range(3):
+            out = torch.full((NL, 2048), float("nan"), device=x.device)
+            ids = c.decode_token(x, out, stream=st)
+            assert np.array_equal(ids, wid), rep
+            assert torch.equal(out, want), rep
+    finally:
+        c.close()
+        for h in held.values():
+            h.free()
+
+
+def test_token_outputs_in_inputs_run_in_order():
+    """Launched directly, a token whose outputs are its layers' inputs is a chain: each layer reads
+    what the one below wrote, and the in-place token reads its own input."""
+    NL, E, I = 5, 64, 256
+    c, held, keep, x = _token_cache(NL, E, I, 64)
+    st = torch.cuda.current_stream().cuda_stream
+    try:
+        for chained in (True, False):
+            buf = torch.zeros((NL + 1, 2048), device=x.device)
+            if chained:
+                buf[0] = x[0]
+                src, dst = buf[:NL], buf[1:]
+            else:
+                buf[:NL] = x
+                src = dst = buf[:NL]
+            want, h = [], x[0]
+            for l in range(NL):
+                o = torch.empty(2048, device=x.device)
+                c.decode_layer(l, h if chained else x[l], o, stream=st)
+                want.append(o)
+                h = o
+            c.step()
+            c.decode_token(src, dst, stream=st)
+            torch.cuda.synchronize()
+            assert torch.equal(dst, torch.stack(want)), chained
+    finally:
+        c.close()
+        for hd in held.values():
+            hd.free()
 
 
 # the shared expert's rows beside the routed pairs: one to five tiles of 32 tokens, ragged, in chunks of
