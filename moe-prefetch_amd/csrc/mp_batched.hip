@@ -149,26 +149,6 @@ __global__ __launch_bounds__(64 * DSP_WAVES) void dispatch_kernel(const int32_t 
 
 // ---------------------------------------------------------------------------
 // Q8_K rows for the matrix cores: one wavefront per (row, 256-value block)
-__device__ inline uint32_t h16(int v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)v); }
-
-// the wave's 4 values per lane -> fp16 codes, block scale and group sums.
-// MFMA: the lane's codes in the order 0, 2, 1, 3 the grouped products read
-// them in (see pack_1024), else 0, 1, 2, 3.
-template <bool MFMA>
-__device__ inline void q8_rows_out(const float xv[4], int lane, size_t off, size_t row, int b, int n,
-                                   uint16_t *q16, float *dx, uint16_t *bs16) {
-    int q[4];
-    float d;
-    q8k_wave_vals(xv, lane, q, d);
-    const int gs = q8k_group_sum(q);
-    uint2 o;
-    o.x = h16(q[0]) | (h16(q[MFMA ? 2 : 1]) << 16);
-    o.y = h16(q[MFMA ? 1 : 2]) | (h16(q[3]) << 16);
-    *(uint2 *)(q16 + off) = o;
-    if ((lane & 3) == 0) bs16[row * (n / 16) + b * 16 + (lane >> 2)] = (uint16_t)h16(gs);
-    if (lane == 0) dx[row * (n / QK) + b] = d;
-}
-
 template <bool MFMA>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const void *src, int bf16, int n_rows, int n,
                                                          uint16_t *q16, float *dx, uint16_t *bs16) {

@@ -224,6 +224,26 @@ __device__ inline int q8k_group_sum(const int q[4]) {
     return gs;
 }
 
+__device__ inline uint32_t h16(int v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)v); }
+
+// the wave's 4 values per lane -> fp16 codes, block scale and group sums.
+// MFMA: the lane's codes in the order 0, 2, 1, 3 the grouped products read
+// them in (pack_1024), else 0, 1, 2, 3.
+template <bool MFMA>
+__device__ inline void q8_rows_out(const float xv[4], int lane, size_t off, size_t row, int b, int n,
+                                   uint16_t *q16, float *dx, uint16_t *bs16) {
+    int q[4];
+    float d;
+    q8k_wave_vals(xv, lane, q, d);
+    const int gs = q8k_group_sum(q);
+    uint2 o;
+    o.x = h16(q[0]) | (h16(q[MFMA ? 2 : 1]) << 16);
+    o.y = h16(q[MFMA ? 1 : 2]) | (h16(q[3]) << 16);
+    *(uint2 *)(q16 + off) = o;
+    if ((lane & 3) == 0) bs16[row * (n / 16) + b * 16 + (lane >> 2)] = (uint16_t)h16(gs);
+    if (lane == 0) dx[row * (n / QK) + b] = d;
+}
+
 // byte i (0..11) of the Q4_K scale field held in three words
 __device__ inline int sc_byte(const uint4 &hdr, int i) {
     const uint32_t w = i < 4 ? hdr.y : (i < 8 ? hdr.z : hdr.w);

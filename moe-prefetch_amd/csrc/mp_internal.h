@@ -81,7 +81,10 @@ struct RouteLaunch {
     float *w;              // out [n_tok][K]
     int32_t *slots;        // out [n_tok][K]
     float *probs;          // out [n_tok][E] or null
-    uint8_t *q8x;          // out [n_tok][H/256][292]
+    uint8_t *q8x;          // out [n_tok][H/256][292] or null
+    uint16_t *xa;          // out or null (router GEMV path): x's Q8_K as launch_quant_rows writes it in mfma_order,
+    float *xdx;            // beside the logits instead of in a launch of its own
+    uint16_t *xbs;
     SidecarPost *post;     // batch-1 decode with CPU-assisted serving: post ids + Q8_K(x), or null
     const uint32_t *seq;   // device: the token's sequence number, or null: seq_val (one layer decoded on
     uint32_t seq_val;      // its own carries the call's number by value; 0 reads as 1)

@@ -111,6 +111,9 @@ struct RouteArgs {
     int32_t *slots;        // [n_tok][K]
     float *probs;          // [n_tok][E] or null
     uint8_t *q8x;          // [n_tok][H/256 * 292]
+    uint16_t *xa;          // or null: x's Q8_K as the grouped products read it (launch_quant_rows, mfma_order)
+    float *xdx;
+    uint16_t *xbs;
     SidecarPost *post;     // batch 1 with CPU-assisted serving, or null
     const uint32_t *seq;   // or null: seq_val
     uint32_t seq_val;
@@ -181,9 +184,13 @@ __global__ __launch_bounds__(64 * RL_WAVES) void route_logits_kernel(RouteArgs a
     // CPU-assisted serving (batch 1) also into the host's post, written
     // through before this kernel ends, so that the select kernel's post only
     // adds the ids
-    if (t == 0 && a.q8x && wave == 0 && (int)blockIdx.x < a.H / QK) {
+    if (t == 0 && (a.q8x || a.xa) && wave == 0 && (int)blockIdx.x < a.H / QK) {
         const float4 v = *(const float4 *)(x + QK * blockIdx.x + 4 * lane);
         const float xv[4] = {v.x, v.y, v.z, v.w};
+        if (a.xa)
+            q8_rows_out<true>(xv, lane, (size_t)tok * a.H + QK * blockIdx.x + 4 * lane, (size_t)tok, (int)blockIdx.x, a.H,
+                              a.xa, a.xdx, a.xbs);
+        if (!a.q8x) return;
         int q[4];
         float d;
         q8k_wave_vals(xv, lane, q, d);
@@ -219,7 +226,14 @@ __global__ __launch_bounds__(64 * RG_WAVES) void route_gemm_kernel(RouteArgs a, 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if ((int)blockIdx.x >= n_tiles) {                 // the Q8_K blocks of x, one per wave
         const int blk = ((int)blockIdx.x - n_tiles) * RG_WAVES + wave;
-        if (blk < n_tok * (a.H / QK)) q8k_wave(a.x + (size_t)QK * blk, a.q8x + (size_t)blk * Q8K_BYTES, lane);
+        if (blk >= n_tok * (a.H / QK)) return;
+        if (a.q8x) q8k_wave(a.x + (size_t)QK * blk, a.q8x + (size_t)blk * Q8K_BYTES, lane);
+        if (a.xa) {
+            const size_t off = (size_t)QK * blk + 4 * lane;
+            const float4 v = *(const float4 *)(a.x + off);
+            const float xv[4] = {v.x, v.y, v.z, v.w};
+            q8_rows_out<true>(xv, lane, off, (size_t)(blk / (a.H / QK)), blk % (a.H / QK), a.H, a.xa, a.xdx, a.xbs);
+        }
         return;
     }
     // the expert tiles of one token tile on one XCD (workgroups go to the 8
@@ -1625,7 +1639,7 @@ template <int RT>
 static hipError_t launch_route_gemm(const RouteArgs &a, int n_tok, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int tw = 16 * RT, tt = ((n_tok + tw - 1) / tw + 7) / 8 * 8;      // token tiles, in eights (one per XCD)
     const int tiles = tt * (a.E / tw);
-    const int q8 = a.q8x ? (n_tok * (a.H / QK) + RG_WAVES - 1) / RG_WAVES : 0;
+    const int q8 = a.q8x || a.xa ? (n_tok * (a.H / QK) + RG_WAVES - 1) / RG_WAVES : 0;
     return launch(route_gemm_kernel<RT>, dim3((unsigned)(tiles + q8)), dim3(64 * RG_WAVES), st, e0, e1, a, n_tok, tiles);
 }
 
@@ -1643,6 +1657,7 @@ hipError_t launch_route(const RouteLaunch &l, hipStream_t st, hipEvent_t *ev) {
         a.adummy[t] = l.adummy[t]; a.atarget[t] = l.atarget[t];
     }
     a.alayer = l.alayer; a.alog = l.alog; a.apost = l.apost; a.fresh = l.fresh;
+    a.xa = l.xa; a.xdx = l.xdx; a.xbs = l.xbs;
     if (l.logits_in)
         return launch(route_select_kernel, dim3((unsigned)l.n_tok), dim3(256), st, ev ? ev[2] : nullptr,
                       ev ? ev[3] : nullptr, a);

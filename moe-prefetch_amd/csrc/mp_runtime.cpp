@@ -1261,7 +1261,7 @@ size_t exp_ws_bytes(int I, int K) {
 int run_route(const moe_route_desc *d, hipStream_t st, hipEvent_t *ev = nullptr, mp::SidecarPost *post = nullptr,
               const uint32_t *seq = nullptr, const mp::RouteLaunch *ahead = nullptr, uint32_t seq_val = 0) {
     mp::RouteLaunch l{};
-    if (ahead) l = *ahead;          // lookahead and table-freshness fields; the rest is set below
+    if (ahead) l = *ahead;          // lookahead, table-freshness and xa fields; the rest is set below
     l.W = d->W; l.x = d->x; l.bias = d->bias; l.prior = d->prior; l.table = d->table; l.dummy = d->dummy;
     l.prior_on_logits = d->prior_on_logits;
     l.E = d->E; l.H = d->H; l.K = d->K; l.n_tok = d->n_tok;
@@ -3600,11 +3600,12 @@ static int grouped_check(const moe_grouped_desc *d) {
 // the host's experts masked out (host_mask, device view of [E] flags), then,
 // once the host's rows are written, the combine taking flagged pairs' rows
 // from hrows (hflag [P]) and the shared expert.
-constexpr int GR_EXPERTS = 1, GR_COMBINE = 2;
+// GR_X: x's Q8_K rows first (without it they are in ws already).
+constexpr int GR_EXPERTS = 1, GR_COMBINE = 2, GR_X = 4;
 // beside: ws has room for the shared expert's rows, so it runs in the routed experts'
 // launches and the combine adds its row (batch 16, 256 experts, I = 512: ~27 us a layer in
 // launches of its own, which leave the GPU nearly idle).
-static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, int parts = GR_EXPERTS | GR_COMBINE,
+static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, int parts = GR_X | GR_EXPERTS | GR_COMBINE,
                        const uint8_t *host_mask = nullptr, const float *hrows = nullptr,
                        const uint8_t *hflag = nullptr, bool beside = false) {
     const GroupedWs w = grouped_ws(d->n_tok, d->K, d->H, d->I, beside);
@@ -3630,9 +3631,10 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
     if (timed)
         for (auto &e : ev) HIPCHK(hipEventCreate(&e));
     auto run = [&]() -> int {
-        if (parts & GR_EXPERTS) {
+        if (parts & GR_X)
             HIPCHK(mp::launch_quant_rows(d->x, d->x_type == MOE_DTYPE_BF16, d->n_tok, d->H, (uint16_t *)a.xa,
                                          (float *)a.xdx, (uint16_t *)a.xbs, true, st));
+        if (parts & GR_EXPERTS) {
             HIPCHK(mp::launch_gateup_grouped(a, st, ev[0], ev[1]));
             HIPCHK(mp::launch_swiglu_quant(a.y2, P + (beside ? d->n_tok : 0), d->I, d->h_out, P, (uint16_t *)a.ha,
                                            (float *)a.hdx, (uint16_t *)a.hbs, st));
@@ -3808,7 +3810,8 @@ static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped
         yp[(size_t)j] = c->bs_y.data() + (size_t)j * c->H;
     }
     std::atomic_thread_fence(std::memory_order_release);
-    int r = grouped_run(gd, (uint8_t *)c->b_ws, st, GR_EXPERTS, c->bs_mask_d + (size_t)par * c->E, nullptr, nullptr, true);
+    int r = grouped_run(gd, (uint8_t *)c->b_ws, st, GR_X | GR_EXPERTS, c->bs_mask_d + (size_t)par * c->E, nullptr,
+                        nullptr, true);
     if (r != MOE_OK) return r;
     if (n) {
         c->sc_computing.store(l, std::memory_order_relaxed);
@@ -3869,7 +3872,17 @@ int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out
         rd.E = c->E; rd.H = c->H; rd.K = c->K; rd.n_tok = n_tok;
         rd.ids = c->b_ids + (size_t)l * TK; rd.w = c->b_w; rd.slots = c->b_slots; rd.q8x = c->b_q8x;
         rd.workspace = c->b_route_ws;
-        if ((r = run_route(&rd, st)) != MOE_OK) return r;
+        // the router's launch also writes x's Q8_K: for the host's share, or as the grouped products read it
+        mp::RouteLaunch xq{};
+        if (!sc) {
+            rd.q8x = nullptr;
+            uint8_t *ws = (uint8_t *)c->b_ws;
+            const GroupedWs w = grouped_ws(n_tok, c->K, c->H, c->I, true);
+            xq.xa = (uint16_t *)(ws + w.xa);
+            xq.xdx = (float *)(ws + w.xdx);
+            xq.xbs = (uint16_t *)(ws + w.xbs);
+        }
+        if ((r = run_route(&rd, st, nullptr, nullptr, nullptr, &xq)) != MOE_OK) return r;
         if (sc) {                       // the routing back to the host for its share
             HIPCHK(hipMemcpyAsync(c->bh_ids + (size_t)l * TK, rd.ids, (size_t)TK * 4, hipMemcpyDeviceToHost, st));
             HIPCHK(hipMemcpyAsync(c->bs_w, c->b_w, (size_t)TK * 4, hipMemcpyDeviceToHost, st));
