@@ -322,6 +322,9 @@ __device__ inline i32x4_t raw_buffer(const void *p, uint32_t bytes) {
     r.y = __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu));
     r.z = __builtin_amdgcn_readfirstlane((int)bytes);
     r.w = BUF_WORD3;
+    // a vector memory instruction may read a scalar register five wait states after the vector
+    // unit (readfirstlane) wrote it; the compiler does not count them before inline assembly
+    asm("s_nop 4" : "+s"(r));
     return r;
 }
 template <int R>
@@ -632,7 +635,7 @@ hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, int 
 }
 
 // ---------------------------------------------------------------------------
-// The Q4_K grouped product of few workgroups (see launch_gg): 64 rows of one
+// The Q4_K grouped product of few workgroups (see launch_q4): 64 rows of one
 // expert a workgroup, its pairs in passes of 16 on MFMA 16x16x32.  For each
 // super-block s the lane's weights are loaded once (block s + 1 in flight
 // meanwhile); four waves per SIMD.
@@ -762,7 +765,7 @@ __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
 // The Q4_K grouped product on MFMA 32x32x16 f16: a workgroup takes a chunk of up
 // to 32 MT pairs of one expert and rtw tiles of 128 rows (four waves of 32).
 //
-// What bounds it.  The 16-row kernel below reads a row's pieces 16 bytes a lane
+// What bounds it.  The 64-row kernel above reads a row's pieces 16 bytes a lane
 // with neighbouring lanes on different rows, so a load touches 64 separate 16-byte
 // pieces, and each of its waves reads all the activations of the pass from LDS
 // for 16 rows.  Here a wave's raw weights come into LDS lane-contiguous (9 lanes a
@@ -805,7 +808,7 @@ __device__ inline void vm_lds_barrier() {
 // The experts' pairs in chunks of up to mt tiles of 32, an expert's tiles spread
 // evenly over its chunks; experts in order.  A wave finds chunk c from the
 // dispatch's offsets (4 experts a lane) and a prefix sum over the lanes.
-struct Chunk { int total, e, p0, np; };
+struct Chunk { int e, p0, np; };
 struct ChunkScan { int off[5], cnt[4], before, total; };
 __device__ inline ChunkScan chunk_scan(const int32_t *offsets, int E, int mt, int lane) {
     ChunkScan r;
@@ -838,8 +841,7 @@ __device__ inline Chunk chunk_find(const ChunkScan &s, int c, int lane) {
         b += s.cnt[j];
     }
     const int src = (int)__builtin_ctzll(__ballot(e >= 0));
-    return Chunk{s.total, __builtin_amdgcn_readlane(e, src), __builtin_amdgcn_readlane(p0, src),
-                 __builtin_amdgcn_readlane(np, src)};
+    return Chunk{__builtin_amdgcn_readlane(e, src), __builtin_amdgcn_readlane(p0, src), __builtin_amdgcn_readlane(np, src)};
 }
 
 // The task'th chunk: with a shared expert its chunks first (e = -1; rows
@@ -851,7 +853,7 @@ __device__ inline Chunk chunk_of(const GroupedArgs &a, const ChunkScan &scan, in
     if (c >= ns) return chunk_find(scan, c - ns, lane);
     const int n = a.P / a.K, tiles = (n + 31) / 32;
     const int t0 = c * tiles / ns, t1 = (c + 1) * tiles / ns;
-    return Chunk{scan.total, -1, a.P + 32 * t0, min(n, 32 * t1) - 32 * t0};
+    return Chunk{-1, a.P + 32 * t0, min(n, 32 * t1) - 32 * t0};
 }
 
 // 4 nibbles' worth of B: words of nibbles under masks -> (1024 + q) * sc - 1024 * sc,
