@@ -629,6 +629,16 @@ size_t moe_grouped_workspace_bytes(int n_tok, int K, int H, int I);
  * moe_dispatch left out is never written. */
 int moe_grouped_experts(const moe_grouped_desc *d, void *stream);
 
+/* No counterpart in the reference.  Which kernel the up/gate (down 0) or down
+ * product of such a call runs on: plan[0] rows of a workgroup (64 or 128),
+ * plan[1] tiles of 32 pairs a chunk holds (128 rows; with 64 rows, M tiles of
+ * 16 pairs a pass), plan[2] row tiles a workgroup takes.  host_weights: some
+ * weights lie, or may lie, in host memory; beside_shared: a shared expert runs
+ * in the same launches (moe_decode_batch).  The results are the same bits
+ * either way.  Host code only: needs no GPU. */
+int moe_grouped_plan(int down, int down_type, int n_tok, int K, int E, int I, int host_weights, int beside_shared,
+                     int32_t plan[3]);
+
 /* No counterpart in the reference.  moe_grouped_experts for callers that
  * cannot allocate device memory (code under HIP graph capture, serving loops
  * and harnesses that forbid hipMalloc): the same kernels and results, with

@@ -1369,32 +1369,54 @@ static hipError_t launch_tile(const GroupedArgs &a, int rtw, hipStream_t st, hip
     else return launch_b(grouped_q4_tile_kernel<1, true, MT>, grid, blk, st, e0, e1, a, rtw);
 }
 
-// Which kernel a Q4_K product runs on.  `full` estimates the chunks of one tile
-// that the batch fills.
+// Row tiles a workgroup takes of a down matrix in host memory: four where a row is one
+// super-block, or for few pairs, but one for so few that the workgroups of an absent expert or
+// two wait on PCIe's latency (ms of down, one / four: 128 experts, I = 768, 16 tokens 1.53 / 1.52, 200 2.47 /
+// 2.74; 256, I = 512, 4 tokens 0.393 / 0.349; 64, I = 256, 4 tokens 0.187 / 0.151, 200 0.381 / 0.368; two layers of
+// 128 experts, 16 of them absent, batch of 2, the whole call 0.324 / 0.347).
+static int host_row_tiles(const GroupedArgs &a) { return a.I == QK || (a.P > 16 && a.P <= 2 * a.E) ? 4 : 1; }
+
+// How a Q4_K product runs.  `full` estimates the chunks of one tile that the batch
+// fills.
 //   few  fewer than 512 workgroups of 128 rows: the 64-row kernel has twice as many,
 //        while a pass of 16 pairs serves an expert, or the one expert of 16 tokens (us: 64 experts, I = 256, up/gate of
 //        64 tokens 14.4 there, 17.6 on tiles; 128 tokens 19.9 / 17.7)
-//   wide at least 64 pairs per expert and 600 workgroups of three tiles: those (us,
-//        one tile / three: up/gate of 1,500 x 8 of 128 158 / 153, 3,000 289 / 253;
-//        but 64 experts, I = 256, 2,000 tokens, 500 workgroups, 54 / 59).  With a slot pool also
-//        from 16 pairs on: an expert outside it is read from host memory once per chunk
+//   wide chunks of three tiles, where they fill the chip and are mostly full themselves:
+//        up/gate from 40 pairs per expert and 510 workgroups on (us, one tile / three: 128 experts, I =
+//        768, 32 pairs 77.7 / 82.5, 40 90.9 / 85.8, 64 115.3 / 107.5, 250 354 / 319; 256, I = 512, 40 117.5 /
+//        113.1; 64, I = 768, 64 pairs, 504 workgroups, 62.9 / 65.2), down with four row tiles from
+//        600 workgroups on, or where a chunk holds an expert and these fill the 512 places of one
+//        round (128 experts, I = 768, 40 pairs 55.5 / 52.4, 64 68.5 / 66.6, 96 91.3 / 107.5, 128 116.9 /
+//        113.7; 64 experts, 64 pairs 40.0 / 43.6)
+//   host with weights in host memory, chunks of three tiles at any number of pairs: an expert
+//        is read once per chunk over PCIe, and two workgroups a CU instead of four fetch
+//        fewer of the lines that two super-blocks share twice (all weights pinned, 128
+//        experts, I = 768, ms of up/gate + down, one tile / three: 64 tokens 5.86 + 3.28 / 5.20 + 2.42, 200
+//        5.94 + 3.36 / 5.25 + 2.47, 700 6.00 + 2.98 / 5.34 + 2.57; the 64-row kernels of 32-pair
+//        passes that were here before read them in 5.35 + 2.64)
 // Down rows (short K) take several row tiles a workgroup, which share its start (us: 512
 // tokens 48.7 with one, 46.8 with two; 4,096 255 with one, 215 with four of three tiles).
+static GroupedPlan plan_q4(const GroupedArgs &a, bool down) {
+    const int rt = (down ? a.H : 2 * a.I) / TL_ROWS, full = max(a.P / 32, min(a.E, a.P));
+    const bool wide = down ? a.P >= 64 * a.E && a.P / 96 * (rt / 4) >= 600 : a.P >= 40 * a.E && a.P / 96 * rt >= 510;
+    if (wide) return {TL_ROWS, 3, down ? 4 : 1};
+    if (a.host) return {TL_ROWS, 3, down ? host_row_tiles(a) : 1};
+    if (down && a.P >= 36 * a.E && a.P <= 64 * a.E && a.E * (rt / 4) >= 512) return {TL_ROWS, 3, 4};
+    if (full * rt < 512 && a.P <= 8 * a.E + 8 && !a.shared) return {64, 1, 1};
+    return {TL_ROWS, 1, down && full * rt >= 2048 ? 2 : 1};
+}
+
 template <bool DOWN>
 static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
-    const int rt = rows / TL_ROWS, full = max(a.P / 32, min(a.E, a.P));
-    if (full * rt < 512 && a.P <= 8 * a.E + 8 && !a.shared) {
-        const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
-        if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false>, grid, blk, st, e0, e1, a);
-        else if (nb == 3) return launch_b(grouped_q4_kernel<3, true>, grid, blk, st, e0, e1, a);
-        else if (nb == 2) return launch_b(grouped_q4_kernel<2, true>, grid, blk, st, e0, e1, a);
-        else return launch_b(grouped_q4_kernel<1, true>, grid, blk, st, e0, e1, a);
-    }
-    const int rtw3 = DOWN ? 4 : 1;
-    if ((a.P >= 64 * a.E && a.P / 96 * (rt / rtw3) >= 600) || (a.slot_pool && a.P > 16 * a.E))
-        return launch_tile<DOWN, 3>(a, rtw3, st, e0, e1);
-    return launch_tile<DOWN, 1>(a, DOWN && full * rt >= 2048 ? 2 : 1, st, e0, e1);
+    const GroupedPlan p = plan_q4(a, DOWN);
+    if (p.rows == TL_ROWS)
+        return p.tiles == 3 ? launch_tile<DOWN, 3>(a, p.row_tiles, st, e0, e1) : launch_tile<DOWN, 1>(a, p.row_tiles, st, e0, e1);
+    const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
+    if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false>, grid, blk, st, e0, e1, a);
+    else if (nb == 3) return launch_b(grouped_q4_kernel<3, true>, grid, blk, st, e0, e1, a);
+    else if (nb == 2) return launch_b(grouped_q4_kernel<2, true>, grid, blk, st, e0, e1, a);
+    else return launch_b(grouped_q4_kernel<1, true>, grid, blk, st, e0, e1, a);
 }
 
 template <int MT>
@@ -1407,20 +1429,33 @@ static hipError_t launch_tile6(const GroupedArgs &a, int rtw, hipStream_t st, hi
     return launch_b(grouped_q6_tile_kernel<1, MT>, grid, blk, st, e0, e1, a, rtw);
 }
 
-// Which kernel a Q6_K down product runs on.
+// How a Q6_K down product runs.
+//   host with weights in host memory, chunks of two tiles, as for Q4_K (all pinned, 128
+//        experts, I = 768, ms, one tile / two: 64 tokens 4.07 / 3.57, 200 4.23 / 3.67, 700 3.94 / 3.81;
+//        the 64-row kernel of 32-pair passes before 3.75, 3.79, 3.71)
 //   I = 512, half a pair to 4 pairs per expert: the 64-row kernel (us, there / on tiles:
 //        256 experts, 16 tokens 33.3 / 36.7, 128 tokens 75.0 / 77.8; below and above that range
 //        8 tokens 28.7 / 25.0, 512 tokens 89.9 / 81.5; I = 768, 128 experts, 64 tokens 62.4 / 50.5)
-//   two tiles a chunk from 48 pairs per expert on (us, one / two: 32 pairs 68.8 / 69.1, 62
-//        pairs 104 / 100, 188 pairs 273 / 238); with a slot pool from 16 on, as for Q4_K
+//   two tiles a chunk from 40 pairs per expert on (us, one / two: 128 experts, I = 768, 32 pairs
+//        66.7 / 68.0, 48 85.8 / 75.4, 128 177 / 158; 64, I = 512, 40 pairs 37.7 / 31.2)
 // Two row tiles a workgroup, but one below two pairs per expert (us, one / two: 128
 // experts, 24 tokens 43 / 48, 1,000 tokens 111 / 104).
-static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    if (a.I == 512 && 2 * a.P > a.E && a.P <= 4 * a.E && !a.shared)
-        return launch_b(grouped_q6_kernel<2>, dim3((unsigned)(a.H / 64 * a.E)), dim3(256), st, e0, e1, a);
-    if (a.P >= 48 * a.E || (a.slot_pool && a.P > 16 * a.E)) return launch_tile6<2>(a, 2, st, e0, e1);
-    return launch_tile6<1>(a, a.P < 2 * a.E ? 1 : 2, st, e0, e1);
+static GroupedPlan plan_q6(const GroupedArgs &a) {
+    if (a.host) return {TL_ROWS, 2, host_row_tiles(a)};
+    if (a.P >= 40 * a.E) return {TL_ROWS, 2, 2};
+    if (a.I == 512 && 2 * a.P > a.E && a.P <= 4 * a.E && !a.shared) return {64, 1, 1};
+    return {TL_ROWS, 1, a.P < 2 * a.E ? 1 : 2};
 }
+
+static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const GroupedPlan p = plan_q6(a);
+    if (p.rows == TL_ROWS)
+        return p.tiles == 2 ? launch_tile6<2>(a, p.row_tiles, st, e0, e1) : launch_tile6<1>(a, p.row_tiles, st, e0, e1);
+    return launch_b(grouped_q6_kernel<2>, dim3((unsigned)(a.H / 64 * a.E)), dim3(256), st, e0, e1, a);
+}
+
+GroupedPlan plan_gateup_grouped(const GroupedArgs &a) { return plan_q4(a, false); }
+GroupedPlan plan_down_grouped(const GroupedArgs &a) { return a.down_type == TYPE_Q6K ? plan_q6(a) : plan_q4(a, true); }
 
 hipError_t launch_gateup_grouped(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     return launch_q4<false>(a, st, e0, e1);

@@ -274,7 +274,17 @@ struct GroupedArgs {
     const uint8_t *host_mask;   // [E] or null: experts the host computes (their rows read as zeros)
     const uint8_t *shared;      // an always-on expert beside the routed ones in the same launches, or null: its
     float *yshared;             // rows follow the P pairs' in y2, ha, hdx and hbs, its outputs are yshared [n_tok][H]
+    int host;                   // 1: some of the weights lie in host memory, or may (the launches that read it over
+                                // PCIe want large chunks, see GroupedPlan)
 };
+// How a grouped product runs, chosen on the host from its shape (the rules and their
+// figures are at the definitions).  rows: of a workgroup, 64 or 128; tiles: of 32 pairs a
+// chunk (128 rows; 64 rows take passes of 16 pairs); row_tiles: of 128 rows a workgroup
+struct GroupedPlan {
+    int rows, tiles, row_tiles;
+};
+GroupedPlan plan_gateup_grouped(const GroupedArgs &a);
+GroupedPlan plan_down_grouped(const GroupedArgs &a);
 
 hipError_t launch_dispatch(const int32_t *ids, int P, int E, int32_t *counts, int32_t *offsets, int32_t *perm,
                            hipStream_t st);

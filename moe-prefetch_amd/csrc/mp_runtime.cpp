@@ -1296,8 +1296,10 @@ int run_experts(const moe_experts_desc *d, hipStream_t st) {
 }
 
 // A kernel read of unmapped memory faults the GPU: refuse anything the runtime
-// does not know as device memory or device-mapped pinned memory.
-int check_weight_ptrs(const char *who, const void *a, const void *b) {
+// does not know as device memory or device-mapped pinned memory.  host (optional):
+// whether one of them is not device memory
+int check_weight_ptrs(const char *who, const void *a, const void *b, bool *host = nullptr) {
+    if (host) *host = false;
     for (const void *p : {a, b}) {
         if (!p) continue;
         hipPointerAttribute_t at{};
@@ -1307,6 +1309,7 @@ int check_weight_ptrs(const char *who, const void *a, const void *b) {
             return fail(MOE_ERR_ARG, "%s: %p is not device memory or mapped pinned memory", who, p);
         if (at.type == hipMemoryTypeHost && at.devicePointer != p)
             return fail(MOE_ERR_ARG, "%s: pass the device address of pinned memory (moe_host_device_ptr)", who);
+        if (host) *host |= at.type != hipMemoryTypeDevice;
     }
     return MOE_OK;
 }
@@ -3567,8 +3570,14 @@ int moe_combine(const float *pair_rows, int n_tok, int K, int H, float *out, int
     return MOE_OK;
 }
 
-// shape and pointer checks shared by both grouped entry points
-static int grouped_check(const moe_grouped_desc *d) {
+// the weights of a grouped call that lie in host memory, or may
+struct GroupedHost {
+    bool routed = false, shared = false;
+};
+
+// shape and pointer checks shared by the grouped entry points; host: what the pointers say
+// (a routed expert outside a slot pool in HBM counts when its store is host memory)
+static int grouped_check(const moe_grouped_desc *d, GroupedHost &host) {
     if (!d || !d->offsets || !d->perm || !d->w || !d->x || !d->out)
         return fail(MOE_ERR_ARG, "moe_grouped_experts: null argument");
     if (d->H != 2048) return fail(MOE_ERR_ARG, "hidden size %d unsupported (the kernels are built for 2048)", d->H);
@@ -3588,9 +3597,9 @@ static int grouped_check(const moe_grouped_desc *d) {
     if (((uintptr_t)d->slot_pool | (uintptr_t)d->store | (uintptr_t)d->x | (uintptr_t)d->out |
          (uintptr_t)d->workspace | (uintptr_t)d->pair_out | (uintptr_t)d->h_out) % 16)
         return fail(MOE_ERR_ARG, "weights, activations and outputs must be 16-byte aligned");
-    int r = check_weight_ptrs("moe_grouped_experts", d->slot_pool, d->store);
+    int r = check_weight_ptrs("moe_grouped_experts", d->slot_pool, d->store, &host.routed);
     if (r != MOE_OK) return r;
-    if (d->shared && (r = check_weight_ptrs("moe_grouped_experts", d->shared, nullptr)) != MOE_OK) return r;
+    if (d->shared && (r = check_weight_ptrs("moe_grouped_experts", d->shared, nullptr, &host.shared)) != MOE_OK) return r;
     if ((uintptr_t)d->shared % 16) return fail(MOE_ERR_ARG, "shared expert must be 16-byte aligned");
     return MOE_OK;
 }
@@ -3605,9 +3614,9 @@ constexpr int GR_EXPERTS = 1, GR_COMBINE = 2, GR_X = 4;
 // beside: ws has room for the shared expert's rows, so it runs in the routed experts'
 // launches and the combine adds its row (batch 16, 256 experts, I = 512: ~27 us a layer in
 // launches of its own, which leave the GPU nearly idle).
-static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, int parts = GR_X | GR_EXPERTS | GR_COMBINE,
-                       const uint8_t *host_mask = nullptr, const float *hrows = nullptr,
-                       const uint8_t *hflag = nullptr, bool beside = false) {
+static int grouped_run(const moe_grouped_desc *d, const GroupedHost &host, uint8_t *ws, hipStream_t st,
+                       int parts = GR_X | GR_EXPERTS | GR_COMBINE, const uint8_t *host_mask = nullptr, const float *hrows = nullptr, const uint8_t *hflag = nullptr,
+                       bool beside = false) {
     const GroupedWs w = grouped_ws(d->n_tok, d->K, d->H, d->I, beside);
     beside = beside && d->shared;
     mp::GroupedArgs a{};
@@ -3626,6 +3635,7 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
         a.shared = d->shared;
         a.yshared = (float *)(ws + w.yshared);
     }
+    a.host = host.routed || (beside && host.shared);
     hipEvent_t ev[4] = {};
     const bool timed = d->kernel_ms != nullptr;
     if (timed)
@@ -3655,6 +3665,7 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
             sa.w = (const float *)(ws + w.sh_ones);
             sa.table = nullptr; sa.slot_pool = nullptr; sa.n_slots = 0;
             sa.store = d->shared; sa.n_store = 1; sa.E = 1; sa.K = 1; sa.P = d->n_tok;
+            sa.host = host.shared;
             HIPCHK(mp::launch_iota(d->n_tok, (int32_t *)sa.offsets, (int32_t *)sa.perm, (float *)sa.w, st));
             HIPCHK(mp::launch_gateup_grouped(sa, st, nullptr, nullptr));
             HIPCHK(mp::launch_swiglu_quant(sa.y2, d->n_tok, d->I, nullptr, 0, (uint16_t *)sa.ha, (float *)sa.hdx,
@@ -3679,14 +3690,16 @@ static int grouped_run(const moe_grouped_desc *d, uint8_t *ws, hipStream_t st, i
 }
 
 int moe_grouped_experts(const moe_grouped_desc *d, void *stream) {
-    int r = grouped_check(d);
+    GroupedHost host;
+    int r = grouped_check(d, host);
     if (r != MOE_OK) return r;
     if (!d->workspace) return fail(MOE_ERR_ARG, "moe_grouped_experts: null workspace");
-    return grouped_run(d, (uint8_t *)d->workspace, (hipStream_t)stream);
+    return grouped_run(d, host, (uint8_t *)d->workspace, (hipStream_t)stream);
 }
 
 int moe_grouped_experts_static(const moe_grouped_desc *d, void *stream) {
-    int r = grouped_check(d);
+    GroupedHost host;
+    int r = grouped_check(d, host);
     if (r != MOE_OK) return r;
     if (d->workspace) return fail(MOE_ERR_ARG, "moe_grouped_experts_static: workspace must be NULL (it uses its own)");
     if (d->kernel_ms) return fail(MOE_ERR_ARG, "moe_grouped_experts_static: kernel_ms must be NULL (timing creates events)");
@@ -3698,7 +3711,22 @@ int moe_grouped_experts_static(const moe_grouped_desc *d, void *stream) {
     void *ws = nullptr;
     const hipError_t e = mp::static_scratch(&ws);
     if (e != hipSuccess) return fail(MOE_ERR_HIP, "static scratch: %s", hipGetErrorString(e));
-    return grouped_run(d, (uint8_t *)ws, (hipStream_t)stream);
+    return grouped_run(d, host, (uint8_t *)ws, (hipStream_t)stream);
+}
+
+int moe_grouped_plan(int down, int down_type, int n_tok, int K, int E, int I, int host_weights, int beside_shared,
+                     int32_t plan[3]) {
+    if (!plan || n_tok < 1 || K < 1 || (int64_t)n_tok * K > 65535 || E < 1 || E > mp::MAX_E || I < 256 || I > 768 ||
+        I % 256 || (down_type != MOE_TYPE_Q4K && down_type != MOE_TYPE_Q6K))
+        return fail(MOE_ERR_ARG, "moe_grouped_plan: bad arguments");
+    static const uint8_t some = 0;
+    mp::GroupedArgs a{};
+    a.P = n_tok * K; a.K = K; a.E = E; a.H = 2048; a.I = I; a.down_type = down_type;
+    a.host = host_weights != 0;
+    a.shared = beside_shared ? &some : nullptr;
+    const mp::GroupedPlan p = down ? mp::plan_down_grouped(a) : mp::plan_gateup_grouped(a);
+    plan[0] = p.rows; plan[1] = p.tiles; plan[2] = p.row_tiles;
+    return MOE_OK;
 }
 
 // ---- batched decode through the cache ------------------------------------------
@@ -3758,7 +3786,8 @@ static int batch_sidecar_buffers(moe_cache *c, int n_tok) {
 // grouped products it then enqueues, computes their pairs from the pinned
 // store while the GPU runs the rest, and writes each pair's weighted row
 // (w * y, the kernels' one multiplication) for the combine.
-static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped_desc *gd, hipStream_t st) {
+static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped_desc *gd, GroupedHost host,
+                               hipStream_t st) {
     const Layer &ls = c->L[l];
     const int TK = n_tok * c->K, par = l & 1;
     const auto t0 = std::chrono::steady_clock::now();
@@ -3776,9 +3805,11 @@ static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped
         if (!(slot >= 0 && slot < ls.S)) absent[id] = 1;
     }
     const int num = c->sb_den ? c->sb_num : c->sc_num, den = c->sb_den ? c->sb_den : c->sc_den;
+    host.routed = false;
     for (int e = 0, r = 0; e < c->E; ++e) {
         mask[e] = absent[e] && r % den < num;
         r += absent[e];
+        host.routed |= absent[e] && !mask[e];       // the GPU reads it from the store
     }
     // the host's pairs grouped by expert (ascending id, pairs in order): each
     // expert's rows are read from memory once for all of its tokens
@@ -3810,8 +3841,8 @@ static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped
         yp[(size_t)j] = c->bs_y.data() + (size_t)j * c->H;
     }
     std::atomic_thread_fence(std::memory_order_release);
-    int r = grouped_run(gd, (uint8_t *)c->b_ws, st, GR_X | GR_EXPERTS, c->bs_mask_d + (size_t)par * c->E, nullptr,
-                        nullptr, true);
+    int r = grouped_run(gd, host, (uint8_t *)c->b_ws, st, GR_X | GR_EXPERTS, c->bs_mask_d + (size_t)par * c->E,
+                        nullptr, nullptr, true);
     if (r != MOE_OK) return r;
     if (n) {
         c->sc_computing.store(l, std::memory_order_relaxed);
@@ -3828,7 +3859,7 @@ static int batch_sidecar_layer(moe_cache *c, int l, int n_tok, const moe_grouped
     c->n_cpu_served += n;
     c->sc_cpu_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t1).count();
     std::atomic_thread_fence(std::memory_order_release);
-    return grouped_run(gd, (uint8_t *)c->b_ws, st, GR_COMBINE, nullptr, c->bs_rows_d + (size_t)par * TK * c->H,
+    return grouped_run(gd, host, (uint8_t *)c->b_ws, st, GR_COMBINE, nullptr, c->bs_rows_d + (size_t)par * TK * c->H,
                        c->bs_flag_d + (size_t)par * TK, true);
 }
 
@@ -3901,14 +3932,22 @@ int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out
         gd.out = out + (size_t)l * n_tok * c->H; gd.accumulate = 0;
         gd.workspace = c->b_ws; gd.shared = ls.shared;
         gd.kernel_ms = c->timing ? gms : nullptr;
-        if ((r = grouped_check(&gd)) != MOE_OK) return r;
+        GroupedHost host;
+        if ((r = grouped_check(&gd, host)) != MOE_OK) return r;
         if (!sc) {
-            if ((r = grouped_run(&gd, (uint8_t *)c->b_ws, st, GR_EXPERTS | GR_COMBINE, nullptr, nullptr, nullptr, true)) !=
-                MOE_OK)
+            // the store is pinned memory: read only where the table leaves an expert out
+            bool absent = false;
+            for (int e = 0; e < ls.E && !absent; ++e) {
+                const int slot = c->h_tbl[(size_t)l * c->E + e];
+                absent = !(slot >= 0 && slot < ls.S);
+            }
+            host.routed = host.routed && absent;
+            if ((r = grouped_run(&gd, host, (uint8_t *)c->b_ws, st, GR_EXPERTS | GR_COMBINE, nullptr, nullptr, nullptr,
+                                 true)) != MOE_OK)
                 return r;
         } else {
             if (!ls.store_host) return fail(MOE_ERR_STATE, "layer %d: CPU-assisted serving needs the host store", l);
-            if ((r = batch_sidecar_layer(c, l, n_tok, &gd, st)) != MOE_OK) return r;
+            if ((r = batch_sidecar_layer(c, l, n_tok, &gd, host, st)) != MOE_OK) return r;
         }
         if (c->timing) {
             c->kt.grouped_gateup_ms += gms[0];

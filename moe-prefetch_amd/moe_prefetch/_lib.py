@@ -226,6 +226,7 @@ SIGNATURES = {
     "moe_quant_rows": (ctypes.c_int, [P, ctypes.c_int, ctypes.c_int, ctypes.c_int, P, P, P, P]),
     "moe_grouped_workspace_bytes": (SZ, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "moe_grouped_experts": (ctypes.c_int, [ctypes.POINTER(GroupedDesc), P]),
+    "moe_grouped_plan": (ctypes.c_int, [ctypes.c_int] * 8 + [P]),
     "moe_grouped_experts_static": (ctypes.c_int, [ctypes.POINTER(GroupedDesc), P]),
     "moe_combine": (ctypes.c_int, [P, ctypes.c_int, ctypes.c_int, ctypes.c_int, P, ctypes.c_int, P]),
     "moe_pool_create": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, SZ, ctypes.c_int, ctypes.POINTER(P)]),

@@ -396,21 +396,41 @@ def test_grouped_experts_slots_pinned_and_absent():
 TILE_EDGES = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 161, 193]
 
 
-@pytest.mark.parametrize("pool", [False, True], ids=["store", "pool"])
+@pytest.mark.parametrize("pool", [False, True, "pinned"], ids=["store", "pool", "pinned"])
 @pytest.mark.parametrize("dt,I", [(_lib.TYPE_Q4K, 768), (_lib.TYPE_Q4K, 512), (_lib.TYPE_Q4K, 256), (_lib.TYPE_Q6K, 768),
                                   (_lib.TYPE_Q6K, 512), (_lib.TYPE_Q6K, 256)],
                          ids=["q4k_i768", "q4k_i512", "q4k_i256", "q6k_i768", "q6k_i512", "q6k_i256"])
 def test_grouped_tile_edges(dt, I, pool):
-    """From a store: chunks of one tile.  With a slot pool (some experts in slots, some in the
-    store, the last in neither): chunks of up to three tiles, several row tiles a workgroup."""
+    """From a store in HBM, alone or behind a slot pool (some experts in slots, some in the store,
+    the last in neither): chunks of one tile (Q6_K: two).  Behind a slot pool from a pinned store:
+    chunks of up to three tiles (two)."""
     E, K, T = 20, 8, 150
-    rng = np.random.default_rng(11 * I + pool)
-    store = Store(E, I, dt)
+    rng = np.random.default_rng(11 * I + bool(pool))
     flat = np.concatenate([np.full(c, e) for e, c in enumerate(TILE_EDGES)] +
                           [rng.choice(np.arange(len(TILE_EDGES), E), size=T * K - sum(TILE_EDGES))])
     ids = rng.permutation(flat).reshape(T, K).astype(np.int32)
     w = rng.random((T, K)).astype(np.float32)
-    src, kw = np.arange(E), {}
+    check_tile_edges(rng, E, K, T, dt, I, ids, w, pool)
+
+
+@pytest.mark.parametrize("T", [1, 5], ids=["t1", "t5"])
+@pytest.mark.parametrize("dt,I", [(_lib.TYPE_Q4K, 768), (_lib.TYPE_Q4K, 512), (_lib.TYPE_Q4K, 256), (_lib.TYPE_Q6K, 768),
+                                  (_lib.TYPE_Q6K, 512), (_lib.TYPE_Q6K, 256)],
+                         ids=["q4k_i768", "q4k_i512", "q4k_i256", "q6k_i768", "q6k_i512", "q6k_i256"])
+def test_grouped_pinned_few_pairs(dt, I, T):
+    """At most two pairs per expert on average from a pinned store: large chunks that hold a pair or
+    two, four row tiles a workgroup."""
+    E, K = 20, 8
+    rng = np.random.default_rng(13 * I + T)
+    ids = np.stack([rng.choice(E, size=K, replace=False) for _ in range(T)]).astype(np.int32)
+    ids[0, 0] = E - 1                           # in neither the slots nor the store
+    w = rng.random((T, K)).astype(np.float32)
+    check_tile_edges(rng, E, K, T, dt, I, ids, w, "pinned")
+
+
+def check_tile_edges(rng, E, K, T, dt, I, ids, w, pool):
+    store = Store(E, I, dt)
+    src, kw, pinned = np.arange(E), {}, None
     if pool:
         slot_bytes, n_slots = (store.eb + 255) // 256 * 256, 12
         table = np.full(E, n_slots, np.int32)
@@ -420,7 +440,15 @@ def test_grouped_tile_edges(dt, I, pool):
             slots[table[e] * slot_bytes:table[e] * slot_bytes + store.eb] = store.t[e * store.eb:(e + 1) * store.eb]
         kw = dict(table=t_(table), slot_pool=slots.data_ptr(), slot_bytes=slot_bytes, n_slots=n_slots, n_store=E - 1)
         src[E - 1] = E                          # expert E of the padded store: zeros
-    out, h_out, pair, perm, xh = run_grouped(store, T, K, E, ids, w, "f32", **kw)
+    if pool == "pinned":
+        pinned = Pinned(E * store.eb)
+        pinned.arr[:] = store.host
+        kw["store_ptr"] = pinned.dev
+    try:
+        out, h_out, pair, perm, xh = run_grouped(store, T, K, E, ids, w, "f32", **kw)
+    finally:
+        if pinned:
+            pinned.free()
     host = np.concatenate([store.host, np.zeros(store.eb, np.uint8)])
     want, want_h = O.moe_tokens(H, I, dt, host, store.eb, E, src[ids], w, xh, n_threads=16, want_h=True)
     assert np.array_equal(h_out, want_h.reshape(T * K, I)[perm])
