@@ -440,16 +440,16 @@ __device__ inline void q6_lane_b(const Q6Lane &w, int i, int h, half8_t &bh, hal
     bl = __builtin_elementwise_fma(q, splat8(sl), splat8((_Float16)(float)(-1056 * (sc & 15))));
 }
 
-// The grouped down product for a Q6_K matrix at I = 512 and few pairs (see
-// launch_q6): 64 rows of one expert a workgroup, the lane's weights streamed
+// The grouped down product for a Q6_K matrix of few workgroups or, at I = 512, few
+// pairs (see plan_q6): 64 rows of one expert a workgroup, the lane's weights streamed
 // from HBM into registers (block s + 1 in flight while block s is multiplied),
-// the pairs in passes of 16 on MFMA 16x16x32.  A block's two integer sums stay
+// the pairs in passes of MT tiles of 16 on MFMA 16x16x32.  A block's two integer sums stay
 // below 2^24 (256 * 32 * 8 * 127 and 256 * 32 * 15 * 127), so each is exact and
 // 16*acc_h + acc_l rounds once, as ggml's (float)sumi.  y = the pair's gate
 // weight times the row value, to the pair's (t*K + k) row.
-template <int NB>
+template <int NB, int MT>
 __global__ __launch_bounds__(256, 4) void grouped_q6_kernel(GroupedArgs a) {
-    constexpr int GK = 16;
+    constexpr int GK = 16 * MT;
     int e, tile;
     tile_expert(blockIdx.x, a.H / 64, a.E, tile, e);
     const int n0 = a.offsets[e], ne = a.offsets[e + 1] - n0;
@@ -489,7 +489,11 @@ __global__ __launch_bounds__(256, 4) void grouped_q6_kernel(GroupedArgs a) {
         q6_lane_load(cw, rw, wo, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float y[MT][4];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[t][i] = 0.0f;
 #pragma unroll 1
         for (int s = 0; s < NB; ++s) {
             if (s + 1 < NB) {
@@ -498,36 +502,52 @@ __global__ __launch_bounds__(256, 4) void grouped_q6_kernel(GroupedArgs a) {
             }
             const float d = h2f_dev((uint16_t)cw.d);
             const AStageR<GK> &S = st[s & 1];
-            float4_t acc = {0, 0, 0, 0}, accl = {0, 0, 0, 0};
-            half8_t fa[2];
-            fa[0] = stage_frag(S, n, q6_a_offset(h, 0));
+            float4_t acc[MT], accl[MT];
+            half8_t fa[2][MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                acc[t] = accl[t] = float4_t{0, 0, 0, 0};
+                fa[0][t] = stage_frag(S, 16 * t + n, q6_a_offset(h, 0));
+            }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (i + 1 < 8) fa[(i + 1) & 1] = stage_frag(S, n, q6_a_offset(h, i + 1 < 8 ? i + 1 : 0));
                 half8_t bh, bl;
-                q6_lane_b(cw, i, h, bh, bl);
-                acc = mfma32(fa[i & 1], bh, acc);
-                accl = mfma32(fa[i & 1], bl, accl);
-            }
-            const float4 dxv = *(const float4 *)&s_dx[s][4 * h];
+                if (i + 1 < 8) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
-                const float sumi = 16.0f * acc[i] + accl[i];
-                y[i] = y[i] + (d * dx) * sumi;   // ggml's order: acc += (d*dx)*sumi
+                    for (int t = 0; t < MT; ++t)
+                        fa[(i + 1) & 1][t] = stage_frag(S, 16 * t + n, q6_a_offset(h, i + 1 < 8 ? i + 1 : 0));
+                }
+                q6_lane_b(cw, i, h, bh, bl);
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    acc[t] = mfma32(fa[i & 1][t], bh, acc[t]);
+                    accl[t] = mfma32(fa[i & 1][t], bl, accl[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const float4 dxv = *(const float4 *)&s_dx[s][16 * t + 4 * h];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
+                    const float sumi = 16.0f * acc[t][i] + accl[t][i];
+                    y[t][i] = y[t][i] + (d * dx) * sumi;   // ggml's order: acc += (d*dx)*sumi
+                }
             }
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             cw = nw;
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 4 * h + i;
-            if (r < np) {
-                const int q = a.perm[n0 + cb + r];
-                a.ypair[(size_t)q * a.H + row] = a.w[q] * y[i];
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 16 * t + 4 * h + i;
+                if (r < np) {
+                    const int q = a.perm[n0 + cb + r];
+                    a.ypair[(size_t)q * a.H + row] = a.w[q] * y[t][i];
+                }
             }
-        }
         __syncthreads();
     }
 }
@@ -635,13 +655,13 @@ hipError_t launch_swiglu_quant(const float *y2, int P, int I, float *h_out, int 
 }
 
 // ---------------------------------------------------------------------------
-// The Q4_K grouped product of few workgroups (see launch_q4): 64 rows of one
-// expert a workgroup, its pairs in passes of 16 on MFMA 16x16x32.  For each
+// The Q4_K grouped product of few workgroups (see plan_q4): 64 rows of one
+// expert a workgroup, its pairs in passes of MT tiles of 16 on MFMA 16x16x32.  For each
 // super-block s the lane's weights are loaded once (block s + 1 in flight
 // meanwhile); four waves per SIMD.
-template <int NB, bool DOWN>
+template <int NB, bool DOWN, int MT>
 __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
-    constexpr int GK = 16;                // pairs per pass
+    constexpr int GK = 16 * MT;           // pairs per pass
     int e, tile;
     tile_expert(blockIdx.x, (DOWN ? a.H : 2 * a.I) / 64, a.E, tile, e);
     const int n0 = a.offsets[e], ne = a.offsets[e + 1] - n0;
@@ -695,7 +715,11 @@ __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
         cw[2] = buf_load16(rw, wo2, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float y[MT][4];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[t][i] = 0.0f;
 #pragma unroll 1
         for (int s = 0; s < NB; ++s) {
             if (s + 1 < NB) {
@@ -711,32 +735,46 @@ __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
             // a half's products sum to at most 128 * 63 * 15 * 127 < 2^24, so
             // it is exact in fp32, and one add gives ggml's (float)sumi (a
             // whole block's sum can pass 2^24, where a running fp32 sum rounds)
-            float4_t acc = {0, 0, 0, 0}, acc0;
+            float4_t acc[MT], acc0[MT];
             // the fragments of K chunk i+1 are read before chunk i's products
-            half8_t fa[2];
-            fa[0] = stage_frag(S, n, q4_a_offset(h, 0));
+            half8_t fa[2][MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                acc[t] = float4_t{0, 0, 0, 0};
+                fa[0][t] = stage_frag(S, 16 * t + n, q4_a_offset(h, 0));
+            }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (i + 1 < 8) fa[(i + 1) & 1] = stage_frag(S, n, q4_a_offset(h, i + 1 < 8 ? i + 1 : 0));
+                if (i + 1 < 8) {
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        fa[(i + 1) & 1][t] = stage_frag(S, 16 * t + n, q4_a_offset(h, i + 1 < 8 ? i + 1 : 0));
+                }
                 const int L = i >> 2, nib = (i >> 1) & 1;
                 const half8_t bi = q4_b(L ? cw[2] : cw[1], i, sc.sc[L][nib]);
-                if (i == 4) {
-                    acc0 = acc;
-                    acc = float4_t{0, 0, 0, 0};
-                }
-                acc = mfma32(fa[i & 1], bi, acc);
-            }
-            acc = acc0 + acc;
-            const float4 dxv = *(const float4 *)&s_dx[s][4 * h];
-            const half4_t am = *(const half4_t *)&S.bs[n][4 * gm];
-            float4_t z = {0, 0, 0, 0};
-            z = __builtin_amdgcn_mfma_f32_16x16x16f16(am, sc.bm, z, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // ggml's order: acc += (d*dx)*sumi; acc -= (dmin*dx)*summ
-                const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
-                y[i] = y[i] + (sc.d * dx) * acc[i];
-                y[i] = y[i] - (sc.dmin * dx) * z[i];
+                for (int t = 0; t < MT; ++t) {
+                    if (i == 4) {
+                        acc0[t] = acc[t];
+                        acc[t] = float4_t{0, 0, 0, 0};
+                    }
+                    acc[t] = mfma32(fa[i & 1][t], bi, acc[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                acc[t] = acc0[t] + acc[t];
+                const float4 dxv = *(const float4 *)&s_dx[s][16 * t + 4 * h];
+                const half4_t am = *(const half4_t *)&S.bs[16 * t + n][4 * gm];
+                float4_t z = {0, 0, 0, 0};
+                z = __builtin_amdgcn_mfma_f32_16x16x16f16(am, sc.bm, z, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    // ggml's order: acc += (d*dx)*sumi; acc -= (dmin*dx)*summ
+                    const float dx = i == 0 ? dxv.x : i == 1 ? dxv.y : i == 2 ? dxv.z : dxv.w;
+                    y[t][i] = y[t][i] + (sc.d * dx) * acc[t][i];
+                    y[t][i] = y[t][i] - (sc.dmin * dx) * z[i];
+                }
             }
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
@@ -745,18 +783,20 @@ __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
             cw[2] = nw[2];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 4 * h + i;
-            if (r < np) {
-                const int pos = n0 + cb + r;
-                if (DOWN) {
-                    const int pp = a.perm[pos];
-                    a.ypair[(size_t)pp * a.H + row] = a.w[pp] * y[i];
-                } else {
-                    a.y2[(size_t)pos * out_n + row] = y[i];
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 16 * t + 4 * h + i;
+                if (r < np) {
+                    const int pos = n0 + cb + r;
+                    if (DOWN) {
+                        const int pp = a.perm[pos];
+                        a.ypair[(size_t)pp * a.H + row] = a.w[pp] * y[t][i];
+                    } else {
+                        a.y2[(size_t)pos * out_n + row] = y[t][i];
+                    }
                 }
             }
-        }
         __syncthreads();
     }
 }
@@ -1378,9 +1418,11 @@ static int host_row_tiles(const GroupedArgs &a) { return a.I == QK || (a.P > 16 
 
 // How a Q4_K product runs.  `full` estimates the chunks of one tile that the batch
 // fills.
-//   few  fewer than 512 workgroups of 128 rows: the 64-row kernel has twice as many,
-//        while a pass of 16 pairs serves an expert, or the one expert of 16 tokens (us: 64 experts, I = 256, up/gate of
-//        64 tokens 14.4 there, 17.6 on tiles; 128 tokens 19.9 / 17.7)
+//   few  no more than 512 workgroups of 128 rows: the 64-row kernel has twice as many. A
+//        pass of one tile while 16 pairs serve an expert, or the one expert of 16 tokens; of two
+//        tiles to twice that (us of up/gate, there / on tiles: 64 experts, I = 256, 64 tokens 14.3 / 17.2, 128 tokens 16.0 /
+//        17.4; 128, I = 256, 16-96 tokens 19.0-20.4 / 21.2-22.4, 128 tokens 23.4 / 22.4; 8 experts, I = 768, 48 pairs 10.0 / 16.0,
+//        128 pairs 12.0 / 16.2, 192 pairs 18.2 / 16.6; one expert, 16 tokens 9.7 / 15.8, 32 12.1 / 15.9, 33 21.3 / 15.6)
 //   wide chunks of three tiles, where they fill the chip and are mostly full themselves:
 //        up/gate from 40 pairs per expert and 510 workgroups on (us, one tile / three: 128 experts, I =
 //        768, 32 pairs 77.7 / 82.5, 40 90.9 / 85.8, 64 115.3 / 107.5, 250 354 / 319; 256, I = 512, 40 117.5 /
@@ -1402,21 +1444,29 @@ static GroupedPlan plan_q4(const GroupedArgs &a, bool down) {
     if (wide) return {TL_ROWS, 3, down ? 4 : 1};
     if (a.host) return {TL_ROWS, 3, down ? host_row_tiles(a) : 1};
     if (down && a.P >= 36 * a.E && a.P <= 64 * a.E && a.E * (rt / 4) >= 512) return {TL_ROWS, 3, 4};
-    if (full * rt < 512 && a.P <= 8 * a.E + 8 && !a.shared) return {64, 1, 1};
+    if (!a.shared) {
+        if ((full * rt < 512 || (a.E * rt <= 512 && a.P < 1024)) && a.P <= 8 * a.E + 8) return {64, 1, 1};
+        if (a.E * rt < 512 && a.P <= 16 * a.E + 16) return {64, 2, 1};
+    }
     return {TL_ROWS, 1, down && full * rt >= 2048 ? 2 : 1};
+}
+
+template <bool DOWN, int MT>
+static hipError_t launch_rows64(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
+    const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
+    if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false, MT>, grid, blk, st, e0, e1, a);
+    else if (nb == 3) return launch_b(grouped_q4_kernel<3, true, MT>, grid, blk, st, e0, e1, a);
+    else if (nb == 2) return launch_b(grouped_q4_kernel<2, true, MT>, grid, blk, st, e0, e1, a);
+    else return launch_b(grouped_q4_kernel<1, true, MT>, grid, blk, st, e0, e1, a);
 }
 
 template <bool DOWN>
 static hipError_t launch_q4(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    const int rows = DOWN ? a.H : 2 * a.I, nb = (DOWN ? a.I : a.H) / QK;
     const GroupedPlan p = plan_q4(a, DOWN);
     if (p.rows == TL_ROWS)
         return p.tiles == 3 ? launch_tile<DOWN, 3>(a, p.row_tiles, st, e0, e1) : launch_tile<DOWN, 1>(a, p.row_tiles, st, e0, e1);
-    const dim3 grid((unsigned)(rows / 64 * a.E)), blk(256);     // (row tile, expert) from the linear id
-    if constexpr (!DOWN) return launch_b(grouped_q4_kernel<8, false>, grid, blk, st, e0, e1, a);
-    else if (nb == 3) return launch_b(grouped_q4_kernel<3, true>, grid, blk, st, e0, e1, a);
-    else if (nb == 2) return launch_b(grouped_q4_kernel<2, true>, grid, blk, st, e0, e1, a);
-    else return launch_b(grouped_q4_kernel<1, true>, grid, blk, st, e0, e1, a);
+    return p.tiles == 2 ? launch_rows64<DOWN, 2>(a, st, e0, e1) : launch_rows64<DOWN, 1>(a, st, e0, e1);
 }
 
 template <int MT>
@@ -1433,25 +1483,49 @@ static hipError_t launch_tile6(const GroupedArgs &a, int rtw, hipStream_t st, hi
 //   host with weights in host memory, chunks of two tiles, as for Q4_K (all pinned, 128
 //        experts, I = 768, ms, one tile / two: 64 tokens 4.07 / 3.57, 200 4.23 / 3.67, 700 3.94 / 3.81;
 //        the 64-row kernel of 32-pair passes before 3.75, 3.79, 3.71)
-//   I = 512, half a pair to 4 pairs per expert: the 64-row kernel (us, there / on tiles:
-//        256 experts, 16 tokens 33.3 / 36.7, 128 tokens 75.0 / 77.8; below and above that range
-//        8 tokens 28.7 / 25.0, 512 tokens 89.9 / 81.5; I = 768, 128 experts, 64 tokens 62.4 / 50.5)
+//   few  no more than 512 workgroups of 128 rows (32 experts): the 64-row kernel, in passes of one
+//        tile while 16 pairs serve an expert, of two to twice that for 8 experts (us, there /
+//        on tiles: one expert, I = 768, 16 tokens 8.6 / 11.2, 32 10.2 / 11.1, 33 17.8 / 11.0; 8 experts, 32 pairs
+//        8.8 / 11.3, 128 pairs 10.0 / 11.4; 16 experts, 128 pairs 12.2 / 12.8, 256 pairs 14.7 / 13.2)
+//   I = 512  half a pair to 4 pairs per expert (8 of 64): the 64-row kernel, which is slower
+//        at I = 256 and 768; why rows of two super-blocks differ was not found, so this line is the
+//        measurement's (us, there / on tiles: 64 experts, 16 pairs 11.1 / 11.2, 128 pairs
+//        20.3 / 24.4, 512 22.9 / 24.6, 768 26.4 / 24.8; 128, 128 pairs 25.8 / 31.6, 512 37.3 / 40.3, 1,024 40.8 / 41.0;
+//        256, 32 pairs 16.7 / 17.6 (the whole call 44.9 / 43.1), 96 35.8 / 31.8, 128 31.8 / 35.6, 1,024 74.3 / 76.3,
+//        2,048 80.9 / 79.3; I = 768, 128 experts, 512 pairs 61.4 / 50.2; I = 256 24.4 / 21.2); passes of two tiles for few
+//        workgroups (16 experts, 256 pairs 11.2 / 11.9)
+//   one row tile a workgroup while all run in one round, 768 workgroups: two of them leave the
+//        chip idle (one expert, 512 tokens 12.9 / 18.6, and 24.7 of two tiles a chunk)
 //   two tiles a chunk from 40 pairs per expert on (us, one / two: 128 experts, I = 768, 32 pairs
 //        66.7 / 68.0, 48 85.8 / 75.4, 128 177 / 158; 64, I = 512, 40 pairs 37.7 / 31.2)
-// Two row tiles a workgroup, but one below two pairs per expert (us, one / two: 128
+// Else two row tiles a workgroup, but one below two pairs per expert (us, one / two: 128
 // experts, 24 tokens 43 / 48, 1,000 tokens 111 / 104).
 static GroupedPlan plan_q6(const GroupedArgs &a) {
     if (a.host) return {TL_ROWS, 2, host_row_tiles(a)};
+    const int full = max(a.P / 32, min(a.E, a.P)), rt = a.H / TL_ROWS;
+    if (!a.shared) {
+        if (a.E * rt <= 512 && a.P <= 8 * a.E + 8) return {64, 1, 1};
+        if (a.E * rt <= (a.I == 512 ? 512 : 128) && a.P <= 16 * a.E + 16) return {64, 2, 1};
+        if (a.I == 512 && a.E * rt > 512 && 2 * a.P >= a.E && a.P <= 4 * max(a.E, 128)) return {64, 1, 1};
+    }
+    if (full * rt <= 768) return {TL_ROWS, 1, 1};
     if (a.P >= 40 * a.E) return {TL_ROWS, 2, 2};
-    if (a.I == 512 && 2 * a.P > a.E && a.P <= 4 * a.E && !a.shared) return {64, 1, 1};
     return {TL_ROWS, 1, a.P < 2 * a.E ? 1 : 2};
+}
+
+template <int MT>
+static hipError_t launch_rows64_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const dim3 grid((unsigned)(a.H / 64 * a.E)), blk(256);
+    if (a.I == 3 * QK) return launch_b(grouped_q6_kernel<3, MT>, grid, blk, st, e0, e1, a);
+    if (a.I == 2 * QK) return launch_b(grouped_q6_kernel<2, MT>, grid, blk, st, e0, e1, a);
+    return launch_b(grouped_q6_kernel<1, MT>, grid, blk, st, e0, e1, a);
 }
 
 static hipError_t launch_q6(const GroupedArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const GroupedPlan p = plan_q6(a);
     if (p.rows == TL_ROWS)
         return p.tiles == 2 ? launch_tile6<2>(a, p.row_tiles, st, e0, e1) : launch_tile6<1>(a, p.row_tiles, st, e0, e1);
-    return launch_b(grouped_q6_kernel<2>, dim3((unsigned)(a.H / 64 * a.E)), dim3(256), st, e0, e1, a);
+    return p.tiles == 2 ? launch_rows64_q6<2>(a, st, e0, e1) : launch_rows64_q6<1>(a, st, e0, e1);
 }
 
 GroupedPlan plan_gateup_grouped(const GroupedArgs &a) { return plan_q4(a, false); }

@@ -428,11 +428,26 @@ def test_grouped_pinned_few_pairs(dt, I, T):
     check_tile_edges(rng, E, K, T, dt, I, ids, w, "pinned")
 
 
+# passes of one tile of 16 pairs and of two (64-row kernels): none, one, the tile's edges and the pass's
+@pytest.mark.parametrize("pool", [False, True], ids=["store", "pool"])
+@pytest.mark.parametrize("counts", [[0, 1, 2, 15, 16, 17, 9, 12], [0, 1, 15, 16, 17, 30, 32, 33]], ids=["one_tile", "two_tiles"])
+@pytest.mark.parametrize("dt,I", [(_lib.TYPE_Q4K, 768), (_lib.TYPE_Q4K, 512), (_lib.TYPE_Q4K, 256), (_lib.TYPE_Q6K, 768),
+                                  (_lib.TYPE_Q6K, 512), (_lib.TYPE_Q6K, 256)],
+                         ids=["q4k_i768", "q4k_i512", "q4k_i256", "q6k_i768", "q6k_i512", "q6k_i256"])
+def test_grouped_few_experts(dt, I, counts, pool):
+    E, K = 8, 2
+    T = sum(counts) // K
+    rng = np.random.default_rng(17 * I + T)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).reshape(T, K).astype(np.int32)
+    w = rng.random((T, K)).astype(np.float32)
+    check_tile_edges(rng, E, K, T, dt, I, ids, w, pool)
+
+
 def check_tile_edges(rng, E, K, T, dt, I, ids, w, pool):
     store = Store(E, I, dt)
     src, kw, pinned = np.arange(E), {}, None
     if pool:
-        slot_bytes, n_slots = (store.eb + 255) // 256 * 256, 12
+        slot_bytes, n_slots = (store.eb + 255) // 256 * 256, min(12, E // 2)
         table = np.full(E, n_slots, np.int32)
         table[:n_slots] = rng.permutation(n_slots)
         slots = torch.zeros(n_slots * slot_bytes, dtype=torch.uint8, device=DEV)

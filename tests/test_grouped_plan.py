@@ -36,6 +36,41 @@ def test_hbm_weights_take_large_chunks_from_40_pairs(T, tiles):
     assert plan(0, Q4, T, 8, 128, 768)[:2] == (128, tiles)
 
 
+# (down, type, tokens, K, experts, I) -> (rows, tiles, row tiles); the comment: what the other side costs
+FEW_WORKGROUPS = [
+    ((0, Q4, 16, 1, 1, 768), (64, 1, 1)),           # 15.8 us for 9.7 on tiles: a shared expert in launches of its own
+    ((0, Q4, 32, 1, 1, 768), (64, 2, 1)),           # 15.9 for 12.1
+    ((0, Q4, 33, 1, 1, 768), (128, 1, 1)),          # 21.3 for 15.6 in passes of 16
+    ((0, Q4, 64, 2, 8, 768), (64, 2, 1)),           # 16.2 for 12.0
+    ((0, Q4, 64, 8, 64, 512), (64, 1, 1)),          # 22.4 for 20.4: exactly 512 workgroups
+    ((0, Q4, 96, 8, 128, 256), (64, 1, 1)),         # 22.4 for 20.4
+    ((0, Q4, 128, 8, 128, 256), (128, 1, 1)),       # 23.4 for 22.4: with so many experts some have over 16 pairs
+    ((1, Q4, 16, 8, 32, 768), (64, 1, 1)),          # 11.8 for 9.6
+    ((1, Q6, 8, 1, 1, 768), (64, 1, 1)),            # 17.3 for 8.4 (two row tiles a workgroup: 8 workgroups)
+    ((1, Q6, 24, 1, 1, 768), (64, 2, 1)),           # 17.4 for 10.0
+    ((1, Q6, 64, 1, 1, 768), (128, 1, 1)),          # 23.4 for 11.2 in chunks of two tiles
+    ((1, Q6, 512, 1, 1, 768), (128, 1, 1)),         # 25.1 for 12.9
+    ((1, Q6, 32, 2, 8, 512), (64, 1, 1)),           # 15.2 for 7.2
+    ((1, Q6, 128, 2, 16, 512), (64, 2, 1)),         # 16.1 for 11.2
+    ((1, Q6, 192, 2, 8, 768), (128, 1, 1)),         # 24.4 for 12.5
+    ((1, Q6, 16, 8, 256, 512), (64, 1, 1)),         # 35.6 for 31.8
+    ((1, Q6, 64, 8, 64, 512), (64, 1, 1)),          # 24.7 for 22.9
+]
+
+
+@pytest.mark.parametrize("shape,want", FEW_WORKGROUPS)
+def test_few_workgroups(shape, want):
+    """Shapes that leave most of the chip idle on tiles of 128 rows take the 64-row kernels, and one
+    row tile a workgroup."""
+    assert plan(*shape) == want
+
+
+@pytest.mark.parametrize("shape", [s for s, w in FEW_WORKGROUPS if w[0] == 64])
+def test_shared_expert_beside_runs_on_tiles(shape):
+    """The 64-row kernels know no shared expert beside the routed ones."""
+    assert plan(*shape, 0, 1)[0] == 128
+
+
 def test_plan_refuses_bad_shapes():
     p = (ctypes.c_int32 * 3)()
     for bad in ((0, Q4, 0, 8, 128, 768), (0, Q4, 9000, 8, 128, 768), (0, Q4, 1, 8, 257, 768), (0, Q4, 1, 8, 128, 300),
