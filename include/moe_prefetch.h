@@ -466,10 +466,11 @@ typedef struct {
     double layer_ms;                       /* split 0: the fused layer launch */
     uint64_t layer_hbm_bytes;              /* its router rows + resident (and shared) experts' bytes */
     uint64_t layer_host_bytes;             /* its absent experts' bytes read from the pinned store */
-    /* moe_decode_batch: the grouped up/gate and down launches of the routed
-     * experts (each layer's launches waited for: timing mode serialises the
-     * host's share behind them); weights by source, one read per expert with
-     * pairs on the GPU; pairs the GPU computed */
+    /* moe_decode_batch: the grouped up/gate and down launches, of the routed
+     * experts and the shared one (each layer's launches waited for: timing mode
+     * serialises the host's share behind them); weights by source, one read per
+     * expert with pairs on the GPU; pairs the GPU computed, a token and the
+     * shared expert counting as one */
     double grouped_gateup_ms, grouped_down_ms;
     uint64_t grouped_launches, grouped_pairs;
     uint64_t grouped_gateup_hbm_bytes, grouped_down_hbm_bytes, grouped_gateup_host_bytes, grouped_down_host_bytes;

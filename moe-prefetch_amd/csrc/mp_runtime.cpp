@@ -3977,6 +3977,11 @@ int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out
                 (res ? c->kt.grouped_down_hbm_bytes : c->kt.grouped_down_host_bytes) += dn_b;
             }
             for (int i = 0; i < TK; ++i) c->kt.grouped_pairs += ids[i] >= 0 && ids[i] < ls.E && !host[(size_t)ids[i]];
+            if (ls.shared) {            // in the same launches, for every token; moe_cache_set_shared put it in HBM
+                c->kt.grouped_gateup_hbm_bytes += gu_b;
+                c->kt.grouped_down_hbm_bytes += dn_b;
+                c->kt.grouped_pairs += (uint64_t)n_tok;
+            }
         }
     for (int l = 0; l < NL; ++l) {
         if ((r = cache_observe(c, l, c->bh_ids + (size_t)l * TK, c->K, n_tok)) != MOE_OK) return r;

@@ -290,6 +290,38 @@ def test_token_outputs_in_inputs_run_in_order():
             hd.free()
 
 
+def test_batch_timing_counts_the_shared_expert():
+    """The timed launches hold the shared expert's rows beside the routed ones: its bytes are among the
+    HBM bytes and a pair a token among the pairs, in the layers that have one."""
+    E, I, K, B, n_slots = 64, 256, 8, 5, 60
+    c, held, keep, _ = _token_cache(3, E, I, n_slots, shared_layers=(0, 1))
+    try:
+        g = torch.Generator(device=keep[0].device)
+        g.manual_seed(1)
+        x = torch.randn((3, B, 2048), device=keep[0].device, generator=g)
+        out = torch.empty_like(x)
+        c.set_timing(True)
+        ids = c.decode_batch(x, out, stream=torch.cuda.current_stream().cuda_stream)
+        kt = c.kernel_times()
+        gu = 2 * I * (2048 // 256) * 144
+        hbm = [0, 0]
+        host = [0, 0]
+        for l in range(3):
+            dn = L().moe_expert_bytes(2048, I, Q6 if l % 2 else Q4) - gu
+            used = np.unique(ids[l])
+            n_res = int((used < n_slots).sum()) + (l < 2)
+            for part, b in ((0, gu), (1, dn)):
+                hbm[part] += n_res * b
+                host[part] += int((used >= n_slots).sum()) * b
+        assert [kt["grouped_gateup_hbm_bytes"], kt["grouped_down_hbm_bytes"]] == hbm
+        assert [kt["grouped_gateup_host_bytes"], kt["grouped_down_host_bytes"]] == host
+        assert kt["grouped_pairs"] == 3 * B * K + 2 * B and kt["grouped_launches"] == 3
+    finally:
+        c.close()
+        for h in held.values():
+            h.free()
+
+
 # the shared expert's rows beside the routed pairs: one to five tiles of 32 tokens, ragged, in chunks of
 # one tile and (E = 64, over 16 pairs per expert) of up to three; Q4_K and Q6_K down
 @pytest.mark.parametrize("E,I,B", [(256, 512, 1), (256, 512, 33), (128, 768, 97), (64, 256, 65), (64, 256, 150)])
