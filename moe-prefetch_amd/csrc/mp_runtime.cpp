@@ -295,6 +295,7 @@ struct moe_cache {
     int g_mode[2] = {-1, -1};          // (timing, split) the graph was captured with
     // batched decode (moe_decode_batch): buffers for up to b_cap tokens, grown on demand
     int b_cap = 0;
+    bool b_shared = false;              // with room for a shared expert's rows
     int32_t *b_ids = nullptr, *b_slots = nullptr, *b_counts = nullptr, *b_offs = nullptr, *b_perm = nullptr;
     int32_t *bh_ids = nullptr;         // pinned host [L][b_cap][K]
     float *b_w = nullptr;
@@ -1320,7 +1321,8 @@ struct GroupedWs {
 };
 
 // shared: with room for a shared expert's rows beside the pairs' (moe_decode_batch's own
-// workspace); without, a shared expert reuses the pairs' after them
+// workspace, of a cache that has one); without, a shared expert reuses the pairs' after them.
+// x's codes come first in either
 GroupedWs grouped_ws(int n_tok, int K, int H, int I, bool shared = false) {
     const size_t T = (size_t)n_tok, P0 = (size_t)n_tok * K, P = P0 + (shared ? T : 0);
     GroupedWs w{};
@@ -3615,10 +3617,10 @@ constexpr int GR_EXPERTS = 1, GR_COMBINE = 2, GR_X = 4;
 // launches and the combine adds its row (batch 16, 256 experts, I = 512: ~27 us a layer in
 // launches of its own, which leave the GPU nearly idle).
 static int grouped_run(const moe_grouped_desc *d, const GroupedHost &host, uint8_t *ws, hipStream_t st,
-                       int parts = GR_X | GR_EXPERTS | GR_COMBINE, const uint8_t *host_mask = nullptr, const float *hrows = nullptr, const uint8_t *hflag = nullptr,
-                       bool beside = false) {
-    const GroupedWs w = grouped_ws(d->n_tok, d->K, d->H, d->I, beside);
+                       int parts = GR_X | GR_EXPERTS | GR_COMBINE, const uint8_t *host_mask = nullptr,
+                       const float *hrows = nullptr, const uint8_t *hflag = nullptr, bool beside = false) {
     beside = beside && d->shared;
+    const GroupedWs w = grouped_ws(d->n_tok, d->K, d->H, d->I, beside);
     mp::GroupedArgs a{};
     a.offsets = d->offsets; a.perm = d->perm; a.w = d->w;
     a.table = d->table; a.slot_pool = d->slot_pool; a.slot_bytes = d->slot_bytes; a.n_slots = d->n_slots;
@@ -3731,26 +3733,28 @@ int moe_grouped_plan(int down, int down_type, int n_tok, int K, int E, int I, in
 
 // ---- batched decode through the cache ------------------------------------------
 static int batch_buffers(moe_cache *c, int n_tok) {
-    if (n_tok <= c->b_cap) return MOE_OK;
+    bool shared = false;                // of any layer: room for its rows
+    for (const Layer &ls : c->L) shared |= ls.shared != nullptr;
+    if (n_tok <= c->b_cap && (!shared || c->b_shared)) return MOE_OK;
+    n_tok = std::max(n_tok, c->b_cap);
     for (void *p : {(void *)c->b_ids, (void *)c->b_slots, (void *)c->b_counts, (void *)c->b_offs, (void *)c->b_perm,
-                    (void *)c->b_w, (void *)c->b_q8x, c->b_route_ws, c->b_ws})
+                    (void *)c->b_w, c->b_route_ws, c->b_ws})
         hipFree(p);
     if (c->bh_ids) hipHostFree(c->bh_ids);
     c->b_ids = c->b_slots = c->b_counts = c->b_offs = c->b_perm = c->bh_ids = nullptr;
     c->b_w = nullptr;
-    c->b_q8x = nullptr;
     c->b_route_ws = c->b_ws = nullptr;
     c->b_cap = 0;
     const size_t NL = c->L.size(), TK = (size_t)n_tok * c->K;
-    const size_t rws = route_ws_bytes(c->E, n_tok), gws = grouped_ws(n_tok, c->K, c->H, c->I, true).total;
+    const size_t rws = route_ws_bytes(c->E, n_tok), gws = grouped_ws(n_tok, c->K, c->H, c->I, shared).total;
     bool ok = hipMalloc(&c->b_ids, NL * TK * 4) == hipSuccess && hipMalloc(&c->b_slots, TK * 4) == hipSuccess &&
               hipMalloc(&c->b_w, TK * 4) == hipSuccess && hipMalloc(&c->b_counts, (size_t)c->E * 4) == hipSuccess &&
               hipMalloc(&c->b_offs, ((size_t)c->E + 1) * 4) == hipSuccess && hipMalloc(&c->b_perm, TK * 4) == hipSuccess &&
-              hipMalloc(&c->b_q8x, (size_t)n_tok * (c->H / 256) * mp::Q8K_BYTES) == hipSuccess &&
               hipMalloc(&c->b_route_ws, rws) == hipSuccess && hipMalloc(&c->b_ws, gws) == hipSuccess &&
               hipHostMalloc((void **)&c->bh_ids, NL * TK * 4, hipHostMallocDefault) == hipSuccess;
     if (!ok || hipMemset(c->b_route_ws, 0, rws) != hipSuccess) return fail(MOE_ERR_NOMEM, "batch buffers for %d tokens", n_tok);
     c->b_cap = n_tok;
+    c->b_shared = shared;
     return MOE_OK;
 }
 
@@ -3759,13 +3763,16 @@ static int batch_sidecar_buffers(moe_cache *c, int n_tok) {
     if (n_tok <= c->bs_cap) return MOE_OK;
     for (void *p : {(void *)c->bs_w, (void *)c->bs_q8, (void *)c->bs_mask, (void *)c->bs_flag, (void *)c->bs_rows})
         if (p) hipHostFree(p);
+    hipFree(c->b_q8x);
+    c->b_q8x = nullptr;
     c->bs_w = nullptr;
     c->bs_q8 = c->bs_mask = c->bs_flag = nullptr;
     c->bs_rows = nullptr;
     c->bs_cap = 0;
     const size_t TK = (size_t)n_tok * c->K;
     const unsigned fl = hipHostMallocMapped | hipHostMallocCoherent;
-    bool ok = hipHostMalloc((void **)&c->bs_w, TK * 4, hipHostMallocDefault) == hipSuccess &&
+    bool ok = hipMalloc(&c->b_q8x, (size_t)n_tok * (c->H / 256) * mp::Q8K_BYTES) == hipSuccess &&
+              hipHostMalloc((void **)&c->bs_w, TK * 4, hipHostMallocDefault) == hipSuccess &&
               hipHostMalloc((void **)&c->bs_q8, (size_t)n_tok * (c->H / 256) * mp::Q8K_BYTES, hipHostMallocDefault) ==
                   hipSuccess &&
               hipHostMalloc((void **)&c->bs_mask, 2 * (size_t)c->E, fl) == hipSuccess &&
@@ -3901,14 +3908,15 @@ int moe_decode_batch(moe_cache *c, const float *x, const float *bias, float *out
         rd.dummy = ls.S;
         rd.prior_on_logits = c->cfg.prior_on_logits;
         rd.E = c->E; rd.H = c->H; rd.K = c->K; rd.n_tok = n_tok;
-        rd.ids = c->b_ids + (size_t)l * TK; rd.w = c->b_w; rd.slots = c->b_slots; rd.q8x = c->b_q8x;
+        rd.ids = c->b_ids + (size_t)l * TK; rd.w = c->b_w; rd.slots = c->b_slots;
         rd.workspace = c->b_route_ws;
         // the router's launch also writes x's Q8_K: for the host's share, or as the grouped products read it
         mp::RouteLaunch xq{};
-        if (!sc) {
-            rd.q8x = nullptr;
+        if (sc) {
+            rd.q8x = c->b_q8x;
+        } else {
             uint8_t *ws = (uint8_t *)c->b_ws;
-            const GroupedWs w = grouped_ws(n_tok, c->K, c->H, c->I, true);
+            const GroupedWs w = grouped_ws(n_tok, c->K, c->H, c->I);
             xq.xa = (uint16_t *)(ws + w.xa);
             xq.xdx = (float *)(ws + w.xdx);
             xq.xbs = (uint16_t *)(ws + w.xbs);

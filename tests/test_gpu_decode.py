@@ -290,6 +290,61 @@ def test_token_outputs_in_inputs_run_in_order():
             hd.free()
 
 
+def test_batch_workspace_without_a_shared_expert():
+    """A cache without a shared expert holds no room for one: what the first batch of 4,096 tokens
+    allocates is the grouped and router workspaces and the routing (2 MiB pages a buffer)."""
+    E, I, K, B = 64, 768, 8, 4096
+    c, held, keep, _ = _token_cache(1, E, I, E)
+    try:
+        st = torch.cuda.current_stream().cuda_stream
+        x = torch.randn((1, B, 2048), device=keep[0].device)
+        out = torch.empty_like(x)
+        c.decode_batch(x[:, :2].contiguous(), out[:, :2].contiguous(), stream=st)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        c.decode_batch(x, out, stream=st)
+        took = free - torch.cuda.mem_get_info()[0]
+        need = L().moe_grouped_workspace_bytes(B, K, 2048, I) + L().moe_route_workspace_bytes(E, B) + 4 * 4 * B * K
+        assert took <= need + 9 * (2 << 20), (took, need)
+    finally:
+        c.close()
+        for h in held.values():
+            h.free()
+
+
+def test_batch_shared_expert_set_after_a_batch():
+    """A shared expert set once batches have run: the next one, of fewer tokens, has room for its rows."""
+    NL, E, I, K = 2, 64, 256, 8
+    c, held, keep, _ = _token_cache(NL, E, I, 60)
+    try:
+        st = torch.cuda.current_stream().cuda_stream
+        dev = keep[0].device
+        g = torch.Generator(device=dev)
+        g.manual_seed(3)
+        x = torch.randn((NL, 40, 2048), device=dev, generator=g)
+        c.decode_batch(x, torch.empty_like(x), stream=st)
+        eb = L().moe_expert_bytes(2048, I, Q6)
+        sh = torch.empty(eb, dtype=torch.uint8, device=dev)
+        synth_experts_dev(9, 1, 0, 1, I, Q6, sh.data_ptr(), eb)
+        c.set_shared(1, sh)
+        x = x[:, :33].contiguous()
+        out = torch.full_like(x, float("nan"))
+        c.decode_batch(x, out, stream=st)
+        torch.cuda.synchronize()
+        for t in range(33):
+            for l in range(NL):
+                want = torch.empty(2048, device=dev)
+                ids = torch.empty(K, dtype=torch.int32, device=dev)
+                c.decode_layer(l, x[l, t], want, ids=ids, stream=st)
+                c.observe(l, ids.cpu().numpy())
+                assert torch.equal(out[l, t], want), (l, t)
+            c.step()
+    finally:
+        c.close()
+        for h in held.values():
+            h.free()
+
+
 def test_batch_timing_counts_the_shared_expert():
     """The timed launches hold the shared expert's rows beside the routed ones: its bytes are among the
     HBM bytes and a pair a token among the pairs, in the layers that have one."""
