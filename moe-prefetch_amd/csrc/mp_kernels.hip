@@ -1475,15 +1475,14 @@ __device__ void fused_publish(const FusedArgs &a, uint32_t seq, const uint64_t *
     // a workgroup of this token gave up: nothing is published, so the host, which wants every
     // layer's words, copies back and synchronises and sees it (a layer beside this one may
     // already have published the late word)
-    if (__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == seq) return;
+    const uint32_t late = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (late == seq) return;
     for (int k = 0; k < K; ++k)
         __hip_atomic_store(a.pub + (size_t)a.pub_layer * K + k, s_rec[k], __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
-    if (a.pub_done) {
-        const uint32_t late = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a.pub_done)
         __hip_atomic_store(a.pub + (size_t)a.pub_L * K, ((uint64_t)seq << 32) | late, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
-    }
 }
 
 // 256 output rows of the combine, then (publishing) the count of finished
