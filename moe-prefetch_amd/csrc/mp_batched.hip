@@ -830,16 +830,43 @@ constexpr int TL_WB = 32 * Q4K_BYTES;   // one wave's raw weights of a super-blo
 // A direct load into LDS, 16 bytes a lane, lane-contiguous at lds (it writes no
 // register).  Not by the builtin: the compiler waits for every such load in flight
 // before an LDS read it cannot tell apart.  These are waited for by hand (vmcnt,
-// then a barrier).  m0 holds nothing across statements here: no builtin that takes
-// it is used beside this one.
+// then a barrier).
 __device__ inline void dma16(uint32_t lds, int voff, i32x4_t rsrc, int soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+                 :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
+}
+// A store of one word a lane, one instruction whatever the compiler makes of its
+// neighbours: waits after it count the stores in flight.  (No memory clobber: it is
+// in order with the loads and waits here, and nothing reads what it writes.)
+__device__ inline void store_f32(float v, i32x4_t rsrc, int voff) {
+    asm volatile("buffer_store_dword %0, %1, %2, 0 offen" :: "v"(v), "v"(voff), "s"(rsrc));
+}
+__device__ void buffer_store_f32(float v, i32x4_t rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
+// the finished rows of one tile of 32 pairs: the pairs' gate weights gw and output rows pp in
+// LDS (four of them read ahead of the stores), y to column col; rows past the chunk's pairs
+// lie past the buffer's end.  16 stores
+__device__ inline void store_down(const float y[16], const float *gw, const uint32_t *pp, i32x4_t ro, int h, int col) {
+    float4 g[2];
+    uint4 p[2];
+    g[0] = *(const float4 *)&gw[4 * h];
+    p[0] = *(const uint4 *)&pp[4 * h];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i + 1 < 4) {
+            g[(i + 1) & 1] = *(const float4 *)&gw[8 * (i + 1) + 4 * h];
+            p[(i + 1) & 1] = *(const uint4 *)&pp[8 * (i + 1) + 4 * h];
+        }
+        const float4 w = g[i & 1];
+        const uint4 r = p[i & 1];
+        store_f32(w.x * y[4 * i], ro, (int)(r.x + (uint32_t)col));
+        store_f32(w.y * y[4 * i + 1], ro, (int)(r.y + (uint32_t)col));
+        store_f32(w.z * y[4 * i + 2], ro, (int)(r.z + (uint32_t)col));
+        store_f32(w.w * y[4 * i + 3], ro, (int)(r.w + (uint32_t)col));
+    }
 }
 __device__ inline uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(lptr_t *)p; }
 constexpr uint32_t TL_NONE = 0xe0000000u;      // an offset past every buffer: reads zeros, is not stored
 constexpr int TL_QUAD = 1024 + 16;      // half a super-block of four rows of activation codes in LDS
-__device__ void buffer_store_f32(float v, i32x4_t rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
 
 __device__ inline void vm_lds_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -908,7 +935,8 @@ __device__ inline half8_t q4_tile_b(uint32_t w0, uint32_t w1, uint32_t M, uint32
 }
 
 template <int NB, bool DOWN, int MT>
-__global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(GroupedArgs a, int rtw) {
+__global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(GroupedArgs a, int row_tiles) {
+    const int rtw = DOWN ? row_tiles : 1;
     constexpr int GK = 32 * MT;
     constexpr int K = NB * QK;
     constexpr int ROWB = NB * Q4K_BYTES;
@@ -1042,19 +1070,21 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void grouped_q4_tile_kernel(G
         if (DOWN) pairs();
         vm_lds_barrier();
         load_a(ntc, 0, 1);
-        // the finished rows of a tile (rows past the chunk's pairs lie past the buffer's
-        // end: not stored), 16 NT stores
+        // the finished rows of a row tile (up/gate has one, stored after the last wait)
         auto store = [&](int rt) {
             const int col = 4 * (r0 + TL_ROWS * rt + 32 * wave + n) + (DOWN ? 0 : 16 * h * out_n);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < NT; ++t) {
+                if constexpr (DOWN) {
+                    store_down(y[t], s_gw + 32 * t, s_pp + 32 * t, ro, h, col);
+                } else {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int ru = 32 * t + 8 * (i >> 2) + (i & 3), r = ru + 4 * h;
-                    if (DOWN) buffer_store_f32(s_gw[r] * y[t][i], ro, (int)(s_pp[r] + (uint32_t)col), 0, 0);
-                    else buffer_store_f32(y[t][i], ro, ru * 4 * out_n + col, 0, 0);
-                    y[t][i] = 0.0f;
+                    for (int i = 0; i < 16; ++i)
+                        buffer_store_f32(y[t][i], ro, (32 * t + 8 * (i >> 2) + (i & 3)) * 4 * out_n + col, 0, 0);
                 }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) y[t][i] = 0.0f;
+            }
         };
         int rt = 0, s = 0;
 #pragma unroll 1
@@ -1275,13 +1305,11 @@ __global__ __launch_bounds__(256, MT == 1 ? 3 : 2) void grouped_q6_tile_kernel(G
         auto store = [&](int rt) {                  // 16 NT stores
             const int col = 4 * (r0 + TL_ROWS * rt + 32 * wave + n);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < NT; ++t) {
+                store_down(y[t], s_gw + 32 * t, s_pp + 32 * t, ro, h, col);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int r = 32 * t + 8 * (i >> 2) + (i & 3) + 4 * h;
-                    buffer_store_f32(s_gw[r] * y[t][i], ro, (int)(s_pp[r] + (uint32_t)col), 0, 0);
-                    y[t][i] = 0.0f;
-                }
+                for (int i = 0; i < 16; ++i) y[t][i] = 0.0f;
+            }
         };
         int rt = 0, s = 0;
 #pragma unroll 1
