@@ -283,12 +283,11 @@ __device__ inline void q4_scales(const uint4 &hdr, int h, Q4Scales &o) {
 // 16-byte chunk c of row r sits at position c ^ (r & 15), so the 16 rows one
 // fragment read touches fall in distinct banks.
 
-// R activation rows (32 for two M tiles of 16 pairs, 16 for one) and the group
-// sums of up to 32
+// R activation rows (32 for two M tiles of 16 pairs, 16 for one) and their group sums
 template <int R>
 struct __attribute__((aligned(16))) AStageR {
     _Float16 a[R][QK];
-    _Float16 bs[32][16];
+    _Float16 bs[R][16];
 };
 
 template <int R>
@@ -300,7 +299,7 @@ __device__ inline half8_t stage_frag(const AStageR<R> &st, int r, int off) {
 // Staging by direct buffer -> LDS loads: lane l of an instruction writes
 // base + 16*l.  rows[r]: activation row of pair r of the pass (r < np); rows
 // are K values long.  Wave w stages rows (R/4)w .. (R/4)w + R/4 - 1 (two per
-// instruction), wave 0 also the group sums; rows past np are not loaded.  The
+// instruction), wave 0 also the group sums (two lanes a row); rows past np are not loaded.  The
 // activation codes and the group sums are raw buffers, the lane's byte offsets
 // are computed once per pass of a chunk and block s's offset s*QK*2 is a
 // scalar: a step's staging costs no per-lane address arithmetic (up/gate at
@@ -346,14 +345,14 @@ __device__ inline void stage_offsets(StageOff<R> &o, const int *rows, int np, in
 }
 template <int R, bool SUMS = true>
 __device__ inline void stage_a_buf(AStageR<R> &st, const StageOff<R> &o, int np, i32x4_t ra, i32x4_t rbs, int s,
-                                   int wave) {
+                                   int wave, int lane) {
 #pragma unroll
     for (int j = 0; j < R / 8; ++j) {
         const int r0 = (R / 4) * wave + 2 * j;
         if (r0 >= np) break;
         buffer_load_lds(ra, (lptr_t *)&st.a[r0][0], 16, o.a[j], s * QK * 2, 0, 0);
     }
-    if (SUMS && wave == 0) buffer_load_lds(rbs, (lptr_t *)&st.bs[0][0], 16, o.bs, s * 32, 0, 0);
+    if (SUMS && wave == 0 && lane < 2 * R) buffer_load_lds(rbs, (lptr_t *)&st.bs[0][0], 16, o.bs, s * 32, 0, 0);
 }
 __device__ inline uint4 buf_load16(i32x4_t r, int voff, int soff) {
     const i32x4_t v = buffer_load_v4(r, voff, soff, 0);
@@ -484,7 +483,7 @@ __global__ __launch_bounds__(256, 4) void grouped_q6_kernel(GroupedArgs a) {
         for (int i = tid; i < GK * NB; i += 256) s_dx[i % NB][i / NB] = a.hdx[(size_t)s_rows[i / NB] * NB + (i % NB)];
         StageOff<GK> so;
         stage_offsets(so, s_rows, np, K, wave, lane);
-        stage_a_buf<GK, false>(st[0], so, np, ra, ra, 0, wave);
+        stage_a_buf<GK, false>(st[0], so, np, ra, ra, 0, wave, lane);
         Q6Lane cw, nw;
         q6_lane_load(cw, rw, wo, 0);
         __builtin_amdgcn_s_waitcnt(0);
@@ -498,7 +497,7 @@ __global__ __launch_bounds__(256, 4) void grouped_q6_kernel(GroupedArgs a) {
         for (int s = 0; s < NB; ++s) {
             if (s + 1 < NB) {
                 q6_lane_load(nw, rw, wo, (s + 1) * Q6K_BYTES);
-                stage_a_buf<GK, false>(st[(s + 1) & 1], so, np, ra, ra, s + 1, wave);
+                stage_a_buf<GK, false>(st[(s + 1) & 1], so, np, ra, ra, s + 1, wave, lane);
             }
             const float d = h2f_dev((uint16_t)cw.d);
             const AStageR<GK> &S = st[s & 1];
@@ -708,7 +707,7 @@ __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
         for (int i = tid; i < GK * NB; i += 256) s_dx[i % NB][i / NB] = adx[(size_t)s_rows[i / NB] * NB + (i % NB)];
         StageOff<GK> so;
         stage_offsets(so, s_rows, np, K, wave, lane);
-        stage_a_buf(st[0], so, np, ra, rbs, 0, wave);
+        stage_a_buf(st[0], so, np, ra, rbs, 0, wave, lane);
         uint4 cw[3], nw[3];
         cw[0] = buf_load16(rw, wo0, 0);
         cw[1] = buf_load16(rw, wo1, 0);
@@ -730,7 +729,7 @@ __global__ __launch_bounds__(256, 4) void grouped_q4_kernel(GroupedArgs a) {
             Q4Scales sc;
             q4_scales(cw[0], h, sc);
             const AStageR<GK> &S = st[s & 1];
-            if (s + 1 < NB) stage_a_buf(st[(s + 1) & 1], so, np, ra, rbs, s + 1, wave);
+            if (s + 1 < NB) stage_a_buf(st[(s + 1) & 1], so, np, ra, rbs, s + 1, wave, lane);
             // each 128-value half of the super-block in its own accumulator:
             // a half's products sum to at most 128 * 63 * 15 * 127 < 2^24, so
             // it is exact in fp32, and one add gives ggml's (float)sumi (a
