@@ -3,8 +3,8 @@ the C ABI against the oracle on the same seeded inputs.
 
   moe_dispatch         counts, offsets and the (token, k)-stable permutation
                        bit-exact (uniform, skewed, all-one-expert, ragged,
-                       several 4096-pair passes, E = 64/128/256, ids outside
-                       [0, E) dropped)
+                       many segments of 1,024 pairs, E = 64/128/256, ids
+                       outside [0, E) dropped)
   moe_quant_rows       Q8_K values, scales and group sums bit-exact (f32, bf16,
                        zero rows, ties of the largest magnitude)
   moe_route (logits)   ids / weights / probabilities from given logits
@@ -12,11 +12,13 @@ the C ABI against the oracle on the same seeded inputs.
   moe_grouped_experts  every token's output and every pair's SwiGLU
                        activations within 1e-3 relative L2 of the ggml-style
                        oracle, and in fact bit-exact (Q4_K and Q6_K down,
-                       intermediate 768/512/256, batch 1..512, tokens crowding
-                       a few experts into several passes, experts in HBM slots
+                       intermediate 768/512/256, batch 1..640, tokens crowding
+                       a few experts into several chunks, experts in HBM slots
                        / a pinned host store / nowhere, super-block sums past
-                       2**24)
+                       2**24); which kernel each shape runs on is
+                       test_grouped_plan.py's
 """
+import ctypes
 import zlib
 
 import numpy as np
@@ -187,15 +189,14 @@ def routing(rng, T, K, E, kind):
     elif kind == "dups":    # ids drawn with replacement from 5 experts: repeats inside a token, uneven
         hot = rng.choice(E, size=5, replace=False)
         ids = np.stack([rng.choice(hot, size=K, replace=True) for _ in range(T)])
-    elif kind == "edges":   # exact counts at the edges of the two-pass chunks' M tiles: 48 pairs (a
-        # second pass of 16, its second tile empty), 49 (17), 33, 64, 65 (a second chunk of 1), 32, 17
-        # and 16; the other experts share the rest (ids repeat inside tokens)
+    elif kind == "edges":   # exact counts at the edges of tiles of 16 and 32 pairs; the other experts
+        # share the rest (ids repeat inside tokens)
         fixed = [48, 49, 33, 64, 65, 32, 17, 16]
         flat = np.concatenate([np.full(c, e) for e, c in enumerate(fixed)] +
                               [rng.choice(np.arange(len(fixed), E), size=T * K - sum(fixed))])
         ids = rng.permutation(flat).reshape(T, K)
         assert [int((ids == e).sum()) for e in range(len(fixed))] == fixed
-    else:   # crowd: most tokens share a handful of experts (several passes of 64 pairs)
+    else:   # crowd: most tokens share a handful of experts (several chunks each)
         hot = rng.choice(E, size=K + 2, replace=False)
         ids = np.stack([rng.choice(hot, size=K, replace=False) if rng.random() < 0.8 else
                         rng.choice(E, size=K, replace=False) for _ in range(T)])
@@ -239,10 +240,10 @@ GROUPED_CASES = {
     "q4k_i256_t150_e64_crowded": (_lib.TYPE_Q4K, 256, 150, 64, "crowd", "f32"),
     "q4k_i768_t24_repeated_ids": (_lib.TYPE_Q4K, 768, 24, 128, "repeat", "bf16"),
     "q6k_i512_t40_ids_with_replacement": (_lib.TYPE_Q6K, 512, 40, 128, "dups", "f32"),
-    # at most 8 pairs per expert on average: one 16-row M tile a pass
+    # few pairs per expert: up/gate on 64 rows in the first, several chunks of the crowded experts in the second
     "q4k_i256_t20_one_tile": (_lib.TYPE_Q4K, 256, 20, 128, "uniform", "bf16"),
     "q4k_i512_t100_crowded_one_tile": (_lib.TYPE_Q4K, 512, 100, 128, "crowd", "f32"),
-    # more than 16 pairs per expert on average: chunks of two 32-pair passes
+    # 17 to 50 pairs per expert: chunks of one tile of 32 pairs, and of two for Q6_K down from 40 on
     "q6k_i768_t512": (_lib.TYPE_Q6K, 768, 512, 128, "uniform", "bf16"),
     "q6k_i512_t300_crowded": (_lib.TYPE_Q6K, 512, 300, 128, "crowd", "f32"),
     "q6k_i256_t300_e64": (_lib.TYPE_Q6K, 256, 300, 64, "uniform", "bf16"),
@@ -252,13 +253,33 @@ GROUPED_CASES = {
     "q6k_i512_t300_tile_edges": (_lib.TYPE_Q6K, 512, 300, 128, "edges", "f32"),
     "q6k_i512_t200_e32": (_lib.TYPE_Q6K, 512, 200, 32, "uniform", "f32"),
     "q6k_i256_t400_e32_crowded": (_lib.TYPE_Q6K, 256, 400, 32, "crowd", "bf16"),
+    # both sides of the lines that give weights in HBM larger chunks: up/gate of 504 and 516 workgroups of
+    # three tiles, a down matrix in chunks of three with four row tiles, a Q6_K one of two
+    "q4k_i768_t512_e32_one_tile": (_lib.TYPE_Q4K, 768, 512, 32, "uniform", "f32"),
+    "q4k_i768_t516_e32_three_tiles": (_lib.TYPE_Q4K, 768, 516, 32, "uniform", "f32"),
+    "q4k_i256_t640_three_tiles": (_lib.TYPE_Q4K, 256, 640, 128, "uniform", "bf16"),
+    "q6k_i512_t319_e64_one_tile": (_lib.TYPE_Q6K, 512, 319, 64, "uniform", "f32"),
+    "q6k_i512_t320_e64_two_tiles": (_lib.TYPE_Q6K, 512, 320, 64, "uniform", "f32"),
 }
+# the tiles of a chunk (up/gate, down) that the cases above are there for
+GROUPED_TILES = {"q4k_i768_t512_e32_one_tile": (1, 1), "q4k_i768_t516_e32_three_tiles": (3, 1),
+                 "q4k_i256_t640_three_tiles": (1, 3), "q6k_i512_t319_e64_one_tile": (1, 1),
+                 "q6k_i512_t320_e64_two_tiles": (1, 2)}
+
+
+def plan(down, dt, T, K, E, I, host=0):
+    """(rows of a workgroup, tiles a chunk or pass holds, row tiles)"""
+    p = (ctypes.c_int32 * 3)()
+    _lib.check(L().moe_grouped_plan(down, dt, T, K, E, I, host, 0, p), "plan")
+    return tuple(p)
 
 
 @pytest.mark.parametrize("case", list(GROUPED_CASES))
 def test_grouped_experts_vs_oracle(case):
     dt, I, T, E, kind, xt = GROUPED_CASES[case]
     K = 8
+    if case in GROUPED_TILES:
+        assert tuple(plan(down, dt, T, K, E, I)[:2] for down in (0, 1)) == tuple((128, n) for n in GROUPED_TILES[case])
     rng = np.random.default_rng(zlib.crc32(case.encode()))
     store = Store(E, I, dt)
     ids, w = routing(rng, T, K, E, kind)
@@ -320,15 +341,32 @@ class LargeSumStore:
         self.t = t_(self.host)
 
 
-@pytest.mark.parametrize("dt,T", [(_lib.TYPE_Q4K, 8), (_lib.TYPE_Q4K, 24), (_lib.TYPE_Q4K, 48),
-                                  (_lib.TYPE_Q4K, 96), (_lib.TYPE_Q6K, 48), (_lib.TYPE_Q6K, 96)],
-                         ids=["q4k_t8", "q4k_t24", "q4k_t48", "q4k_t96", "q6k_t48", "q6k_t96"])
-def test_grouped_experts_sums_past_2_24(dt, T):
+# (type, tokens, pinned): (rows, tiles) of up/gate and of down
+LARGE_SUMS = {
+    (_lib.TYPE_Q4K, 8, False): ((64, 1), (64, 1)),
+    (_lib.TYPE_Q4K, 24, False): ((64, 2), (64, 2)),
+    (_lib.TYPE_Q4K, 48, False): ((128, 1), (128, 1)),
+    (_lib.TYPE_Q4K, 96, False): ((128, 1), (128, 1)),
+    (_lib.TYPE_Q4K, 96, True): ((128, 3), (128, 3)),
+    (_lib.TYPE_Q4K, 160, True): ((128, 3), (128, 3)),
+    (_lib.TYPE_Q6K, 8, False): ((64, 1), (64, 1)),
+    (_lib.TYPE_Q6K, 48, False): ((128, 1), (128, 1)),
+    (_lib.TYPE_Q6K, 96, False): ((128, 1), (128, 1)),
+    (_lib.TYPE_Q6K, 96, True): ((128, 3), (128, 2)),
+}
+
+
+@pytest.mark.parametrize("dt,T,pinned", list(LARGE_SUMS),
+                         ids=["%s_t%d%s" % ("q6k" if d == _lib.TYPE_Q6K else "q4k", t, "_pinned" if p else "")
+                              for d, t, p in LARGE_SUMS])
+def test_grouped_experts_sums_past_2_24(dt, T, pinned):
     """Super-block integer sums beyond fp32's exact integers (2**24): the
     grouped kernels still equal ggml's (float)sumi bit for bit.  16 experts,
-    top-8: 4, 12, 24 and 48 pairs per expert (one-tile passes, one-pass and
-    two-pass chunks)."""
+    top-8: 4, 12, 24, 48 and 80 pairs per expert, in passes of one and two tiles
+    of 16 pairs, chunks of one tile of 32 and, from a pinned store, of two
+    (48 pairs, and any Q6_K down) and three (80)."""
     E, K, I = 16, 8, 768
+    assert tuple(plan(down, dt, T, K, E, I, pinned)[:2] for down in (0, 1)) == LARGE_SUMS[dt, T, pinned]
     rng = np.random.default_rng(77 + T)
     store = LargeSumStore(E, I, dt)
     x = (1.0 - 0.06 * rng.random((T, H))).astype(np.float32)      # Q8_K codes -127 .. -119
@@ -341,7 +379,15 @@ def test_grouped_experts_sums_past_2_24(dt, T):
                         for j in range(4)], 1).astype(np.int64)        # element order of ggml's Q4_K
     sums = (63 * q * q8).sum(1)
     assert np.abs(sums).max() > 2 ** 24, np.abs(sums).max()
-    out, h_out, pair, perm, xh = run_grouped(store, T, K, E, ids, w, "f32", x_host=x)
+    host = Pinned(store.host.size) if pinned else None
+    try:
+        if pinned:
+            host.arr[:] = store.host
+        out, h_out, pair, perm, xh = run_grouped(store, T, K, E, ids, w, "f32", x_host=x,
+                                                 store_ptr=host.dev if pinned else None)
+    finally:
+        if pinned:
+            host.free()
     want, want_h = O.moe_tokens(H, I, dt, store.host, store.eb, E, ids, w, xh, n_threads=16, want_h=True)
     hw = want_h.reshape(T * K, I)[perm]
     assert np.isfinite(want).all() and np.abs(hw).min() > 0
@@ -402,8 +448,8 @@ TILE_EDGES = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 161, 193]
                          ids=["q4k_i768", "q4k_i512", "q4k_i256", "q6k_i768", "q6k_i512", "q6k_i256"])
 def test_grouped_tile_edges(dt, I, pool):
     """From a store in HBM, alone or behind a slot pool (some experts in slots, some in the store,
-    the last in neither): chunks of one tile (Q6_K: two).  Behind a slot pool from a pinned store:
-    chunks of up to three tiles (two)."""
+    the last in neither): chunks of one tile.  Behind a slot pool from a pinned store: chunks of up
+    to three tiles (Q6_K down: two)."""
     E, K, T = 20, 8, 150
     rng = np.random.default_rng(11 * I + bool(pool))
     flat = np.concatenate([np.full(c, e) for e, c in enumerate(TILE_EDGES)] +

@@ -312,10 +312,12 @@ def test_batch_workspace_without_a_shared_expert():
             h.free()
 
 
-def test_batch_shared_expert_set_after_a_batch():
-    """A shared expert set once batches have run: the next one, of fewer tokens, has room for its rows."""
+@pytest.mark.parametrize("n_slots", [60, 64], ids=["absent", "resident"])
+def test_batch_shared_expert_set_after_a_batch(n_slots):
+    """A shared expert set once batches have run: the next one, of fewer tokens, has room for its rows
+    (with every expert resident, in chunks of one tile)."""
     NL, E, I, K = 2, 64, 256, 8
-    c, held, keep, _ = _token_cache(NL, E, I, 60)
+    c, held, keep, _ = _token_cache(NL, E, I, n_slots)
     try:
         st = torch.cuda.current_stream().cuda_stream
         dev = keep[0].device
@@ -377,8 +379,8 @@ def test_batch_timing_counts_the_shared_expert():
             h.free()
 
 
-# the shared expert's rows beside the routed pairs: one to five tiles of 32 tokens, ragged, in chunks of
-# one tile and (E = 64, over 16 pairs per expert) of up to three; Q4_K and Q6_K down
+# the shared expert's rows beside the routed pairs: one to five tiles of 32 tokens, ragged, in chunks of up
+# to three (Q6_K down: two), since some experts are absent; Q4_K and Q6_K down
 @pytest.mark.parametrize("E,I,B", [(256, 512, 1), (256, 512, 33), (128, 768, 97), (64, 256, 65), (64, 256, 150)])
 def test_decode_batch_shared_expert_tiles(E, I, B):
     rig = Rig([E - 8, E // 2], [Q4, Q6], T=B, I=I, E=E, shared=True, zipf_s=1.0, admit="window", batch_tables=True)
