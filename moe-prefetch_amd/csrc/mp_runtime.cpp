@@ -3363,7 +3363,7 @@ int moe_decode_token(moe_cache *c, const float *x, const float *bias, float *out
     // it; the graph copies the inputs first).
     const size_t xb = (size_t)NL * c->H, bb = (size_t)NL * c->E;
     const bool apart = (out + xb <= x || x + xb <= out) && (!bias || out + xb <= bias || bias + bb <= out);
-    const bool together = fused && !sc && !c->timing;
+    const bool together = fused && !sc && !c->timing && NL > 1;
     // A captured graph's launch costs ~30 us of latency here (ROCm 7 on
     // MI355X) against ~11 us for a kernel launch.  The graph frees the host sooner,
     // which CPU-assisted serving and streaming need (the host serves a layer
@@ -3424,7 +3424,8 @@ int moe_decode_token(moe_cache *c, const float *x, const float *bias, float *out
     c->pub_on = publish;
     // per-kernel HIP-event timing needs eager launches: hipEventElapsedTime
     // does not accept events recorded as nodes of a graph
-    mp::FusedMulti many{};
+    mp::FusedMulti many;            // (4 KiB: what the layers do not fill is not read)
+    many.n = many.kt = 0;
     mp::FusedMulti *multi = together && (use_graph || apart) ? &many : nullptr;
     if (!use_graph) {
         for (int l = 0; l < NL; ++l) {
