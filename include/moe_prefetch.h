@@ -574,8 +574,9 @@ int moe_decode_layer(moe_cache *c, int layer, const float *x, const float *bias,
  * out dev [L][H]; then the routed ids come back (one copy), are observed in
  * layer order and the cache steps.  ids_host [L][K] receives them when not NULL.
  * The call returns with out complete in device memory.  When the layers are
- * launched directly without CPU-assisted serving or streaming (at most 8
- * layers, graph mode 0 or 1, no timing), the fused launches publish the ids
+ * launched directly (moe_cache_set_decode_path: those that share launches, or
+ * at most 8; graph mode 0 for any) without CPU-assisted serving, streaming or
+ * timing, the fused launches publish the ids
  * into mapped memory as tagged words and the call returns once all of them
  * carry the token's number, without synchronising the stream: the last launch
  * may still be retiring, and work enqueued later on the stream orders after it

@@ -1457,12 +1457,12 @@ static int host_row_tiles(const GroupedArgs &a) { return a.I == QK || (a.P > 16 
 //        600 workgroups on, or where a chunk holds an expert and these fill the 512 places of one
 //        round (128 experts, I = 768, 40 pairs 55.5 / 52.4, 64 68.5 / 66.6, 96 91.3 / 107.5, 128 116.9 /
 //        113.7; 64 experts, 64 pairs 40.0 / 43.6)
-//   host with weights in host memory, chunks of three tiles at any number of pairs: an expert
-//        is read once per chunk over PCIe, and two workgroups a CU instead of four fetch
-//        fewer of the lines that two super-blocks share twice (all weights pinned, 128
-//        experts, I = 768, ms of up/gate + down, one tile / three: 64 tokens 5.86 + 3.28 / 5.20 + 2.42, 200
-//        5.94 + 3.36 / 5.25 + 2.47, 700 6.00 + 2.98 / 5.34 + 2.57; the 64-row kernels of 32-pair
-//        passes that were here before read them in 5.35 + 2.64)
+//   host with weights in host memory, chunks of three tiles at any number of pairs: an expert is
+//        read once per chunk over PCIe, and two workgroups a CU instead of four read faster,
+//        probably as fewer of the lines that two super-blocks share are fetched twice (all weights
+//        pinned, 128 experts, I = 768, ms of up/gate + down, one tile / three: 64 tokens 5.86 + 3.28 /
+//        5.20 + 2.42, 200 5.94 + 3.36 / 5.25 + 2.47, 700 6.00 + 2.98 / 5.34 + 2.57; 64-row kernels
+//        in passes of 32 pairs, each chunk of two read once, 5.35 + 2.64)
 // Down rows (short K) take several row tiles a workgroup, which share its start (us: 512
 // tokens 48.7 with one, 46.8 with two; 4,096 255 with one, 215 with four of three tiles).
 static GroupedPlan plan_q4(const GroupedArgs &a, bool down) {
@@ -1509,7 +1509,7 @@ static hipError_t launch_tile6(const GroupedArgs &a, int rtw, hipStream_t st, hi
 // How a Q6_K down product runs.
 //   host with weights in host memory, chunks of two tiles, as for Q4_K (all pinned, 128
 //        experts, I = 768, ms, one tile / two: 64 tokens 4.07 / 3.57, 200 4.23 / 3.67, 700 3.94 / 3.81;
-//        the 64-row kernel of 32-pair passes before 3.75, 3.79, 3.71)
+//        64-row kernel in passes of 32 pairs 3.75, 3.79, 3.71)
 //   few  no more than 512 workgroups of 128 rows (32 experts): the 64-row kernel, in passes of one
 //        tile while 16 pairs serve an expert, of two to twice that for 8 experts (us, there /
 //        on tiles: one expert, I = 768, 16 tokens 8.6 / 11.2, 32 10.2 / 11.1, 33 17.8 / 11.0; 8 experts, 32 pairs
